@@ -173,6 +173,16 @@ int mo_int_qdq(const void* x, void* y, int64_t outer, int64_t axis, int64_t inne
                const void* amax, int amax_dtype, int num_bits, int is_unsigned,
                int narrow_range, void* stream);
 
+/* Backward of the fake quantisers (straight-through estimator with clipping): dx = dy where
+ * |x| <= amax, 0 elsewhere, NaN on either side of the comparison giving 0.  Replaces
+ * _fake_tensor_quant_backward of TQ/tensor_quant.py (abs, compare, where: three passes and a boolean
+ * tensor) behind FakeTensorQuantFunction / ScaledE4M3Function /
+ * DynamicBlockQuantizationFunction.backward.  x, dy and dx have type dtype and are viewed as
+ * [outer, axis, inner]; amax has `axis` elements of type amax_dtype; narrow_amax rounds it to dtype
+ * first (what type promotion does to a 0-dim amax of another type).  dx may alias dy. */
+int mo_ste_mask(const void* x, const void* dy, void* dx, int64_t outer, int64_t axis, int64_t inner,
+                int dtype, const void* amax, int amax_dtype, int narrow_amax, void* stream);
+
 /* FP8 / integer fake quantisation with one amax per two-dimensional block: x viewed as
  * [rows, cols], amax[(row / block_rows) * (cols / block_cols) + col / block_cols] -- the layout a
  * quantizer with block_sizes on the last two dims gives its amax (FP8_2D_BLOCKWISE_WEIGHT_ONLY_CFG,

@@ -39,6 +39,7 @@ SIGNATURES = {
     "mo_nvfp4_quantize_multi": [_P, _INT, _P, _I64, _INT, _INT, _INT, _INT, _P],
     "mo_fp8_qdq": [_P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _P],
     "mo_int_qdq": [_P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _P],
+    "mo_ste_mask": [_P, _P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _P],
     "mo_nvfp4_qdq": [_P, _P, _I64, _I64, _INT, _P, _INT, _INT, _INT, _P],
     "mo_qdq_sq_err": [_P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _INT, _INT, _P, _P],
     "mo_mxfp4_quantize": [_P, _I64, _INT, _INT, _P, _P, _P],
@@ -335,6 +336,18 @@ def int_qdq(x, amax, outer, axis, inner, num_bits, unsigned, narrow_range, out=N
          dtype_code(amax.dtype), int(num_bits), int(bool(unsigned)), int(bool(narrow_range)),
          _stream(x))
     return y
+
+
+def ste_mask(x, grad, amax, outer, axis, inner, narrow_amax=False):
+    """``grad`` where ``|x| <= amax``, zero elsewhere (``x`` and ``grad`` of one dtype, contiguous, viewed
+    as [outer, axis, inner]); ``narrow_amax`` rounds the amax to that dtype first."""
+    _require_device(x, grad, amax)
+    assert x.is_contiguous() and grad.is_contiguous() and amax.is_contiguous() and x.dtype == grad.dtype
+    assert outer * axis * inner == x.numel() == grad.numel() and amax.numel() == axis
+    out = torch.empty_like(grad)
+    call("mo_ste_mask", x, _ptr(x), _ptr(grad), _ptr(out), outer, axis, inner, dtype_code(x.dtype),
+         _ptr(amax), dtype_code(amax.dtype), int(narrow_amax), _stream(x))
+    return out
 
 
 def blocks2d_covered(x, rows, cols, block_rows, block_cols) -> bool:

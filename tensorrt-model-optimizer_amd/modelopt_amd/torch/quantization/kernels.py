@@ -12,7 +12,7 @@ from ... import _hip
 
 __all__ = [
     "amax_layout", "kept_dims_first", "dense_flat_view", "absmax_accumulate", "reduce_amax_gpu", "fake_quant_int", "fake_quant_fp8",
-    "fake_quant_nvfp4", "fake_quant_block_fp", "mul_last_dim",
+    "ste_mask", "fake_quant_nvfp4", "fake_quant_block_fp", "mul_last_dim",
 ]
 
 
@@ -186,6 +186,23 @@ def fake_quant_fp8(x, amax=None, saturate=False):
     return _qdq(x, amax, lambda x2, a, outer, axis, inner: _hip.fp8_qdq(
         x2, a, outer, axis, inner, saturate),
         lambda x2, a, rows, cols, br, bc: _hip.fp8_qdq_blocks2d(x2, a, rows, cols, br, bc, saturate))
+
+
+def ste_mask(x, amax, grad):
+    """``torch.where(x.abs() <= amax, grad, 0)`` in one pass, or None where the kernel does not apply:
+    mixed types, a gradient in another memory order, an amax on two separated runs of dims."""
+    if (not (x.is_cuda and grad.is_cuda and amax.is_cuda) or x.dtype != grad.dtype or x.dim() == 0
+            or x.shape != grad.shape or x.dtype not in _hip._DTYPES or amax.dtype not in _hip._DTYPES
+            or not x.is_contiguous() or not grad.is_contiguous()):
+        return None
+    layout = (1, 1, x.numel()) if amax.numel() == 1 and amax.dim() <= x.dim() else None
+    if layout is None and amax.dim() == x.dim():
+        layout = _qdq_layout(x, amax)
+    if layout is None:
+        return None
+    # a 0-dim amax takes the type of x in the comparison, one with dims promotes x to the wider type
+    return _hip.ste_mask(x, grad, amax.reshape(-1).contiguous(), *layout,
+                         narrow_amax=amax.dim() == 0 and amax.dtype != x.dtype)
 
 
 def fake_quant_nvfp4(x, global_amax, block_size=16, mode=0):

@@ -179,6 +179,9 @@ QUANT_DESC_8BIT_CONVTRANSPOSE3D_WEIGHT_PER_CHANNEL = QuantizerAttributeConfig(nu
 def _fake_tensor_quant_backward(inputs, amax, grad_outputs):
     if amax is None:
         return grad_outputs
+    masked = kernels.ste_mask(inputs, amax, grad_outputs)
+    if masked is not None:
+        return masked
     zero = grad_outputs.new_zeros(1)
     return torch.where(inputs.abs() <= amax, grad_outputs, zero)
 
