@@ -7,33 +7,40 @@
 //   cur[t]  = T( sum_j T(x[t, j] * wq_r[j]) )              wq_r = T(qdq(w; T(f32(amax) * r)))
 //   loss[r] += ( sum_t f32(T(cur[t] - org[t]))^2 ) / tokens
 //
-// Work decomposition: a lane owns one (output row, block).  The block of the quantised weight
-// stays in the lane's registers as fp32; the activations of a token are the same for every
-// lane, so they are read through uniform (scalar) loads and cost the vector ALU nothing.  The
-// org[] values of a lane live in LDS ([token][lane], conflict-free).  VALU-bound: each product
-// is one multiply, one rounding to T and one add (bf16: two products share the rounding and the
-// add, see token_dots).
-//
-// A weight with few (row, block) pairs does not fill the chip with one wavefront per 64 pairs
-// (1024 x 4096 in blocks of 128 is 512 wavefronts for 1024 SIMDs, and a lone wavefront on a
-// SIMD runs at two thirds of the rate three of them reach together), so a workgroup may hold
-// 2 or 4 wavefronts that own the same 64 pairs and share the tokens of a pass between them;
-// their partial sums meet in LDS and wavefront 0 adds them in wavefront order, so the result
-// does not depend on timing.
+// Every product is rounded to T before it is summed, so the products themselves cannot be one
+// contraction; what the matrix cores can do is make the products (an outer product per column j,
+// whose fp32 result is exact for 16-bit operands) and add them up once they are rounded (a
+// contraction with a 0 / 1 matrix).  Issue costs, measured per wavefront instruction: 4.5 cycles for
+// v_mul_f32, v_cvt_pk_bf16_f32, v_pk_mul_f16 and v_dot2c, 16 cycles for a 16x16x32 and 32 for a
+// 32x32x16 matrix instruction, which run beside the vector instructions of other wavefronts and take
+// about 8 cycles of the issue port themselves.
+//   bf16: products on the matrix cores, one conversion per two products on the vector ALU, sums on the
+//         matrix cores (clip_losses_bf16): 0.5 vector instructions per product where multiply,
+//         convert and v_dot2c took 2.
+//   fp16: v_pk_mul_f16 rounds two products at once, sums on the matrix cores (clip_losses_f16): 0.5
+//         vector instructions per product where multiply, round and add took about 4.
+//   fp32: no rounding to do, one multiply and one add per product (clip_losses_f32).
+// Measured figures stand at the launch below.
 #include "common.h"
 #include "qdq_ops.h"
 
 namespace mo {
 
 constexpr int kClipMaxRatios = 32;
-constexpr int kClipTokens = 64;   // tokens per wavefront and pass over the ratios (org[] in LDS)
+constexpr int kClipTokens = 64;   // tokens of a pass over the ratios (fp32: per wavefront)
 constexpr int kClipLanes = 64;
-constexpr int kClipMaxSplit = 4;  // wavefronts that may share the tokens of one (row, block) set
+constexpr int kClipWaves = 4;     // wavefronts of a workgroup (fp32: at most)
 
 struct ClipRatios {
     float r[kClipMaxRatios];
     int count;
 };
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x32_t __attribute__((ext_vector_type(32)));
 
 template <int DT>
 __device__ __forceinline__ float clip_round(float v) {
@@ -42,29 +49,376 @@ __device__ __forceinline__ float clip_round(float v) {
     else return v;
 }
 
-// For each of `tc` tokens, T( sum_j T(x[t, j] * w[j]) ) -- products rounded to T one by one,
-// summed in fp32 in index order -- handed to fn(t, value).
+// The quantiser of one block at one ratio: `w_amax * ratio` on a tensor is an fp32 product rounded
+// to the dtype of the amax.
+__device__ __forceinline__ IntOp::Scale clip_scale(const IntOp& op, float amax, int amax_dtype, float ratio) {
+    float clipped = amax * ratio;
+    if (amax_dtype == MO_BF16) clipped = clip_round<MO_BF16>(clipped);
+    else if (amax_dtype == MO_F16) clipped = clip_round<MO_F16>(clipped);
+    return op.make(clipped);
+}
+
+// op.apply where clip_fast says so, less the sign of a zero (the value is only summed)
+__device__ __forceinline__ bool clip_fast(const IntOp& op, const IntOp::Scale& s) {
+    return s.fast && op.bound <= 2047.0f;   // codes of at most 11 bits: the short quotient
+}
+__device__ __forceinline__ float clip_qdq_fast(const IntOp& op, float v, const IntOp::Scale& s) {
+    const float q = __builtin_amdgcn_fmed3f(__builtin_rintf(v * s.mul), op.lo, op.bound);
+    return exact_quotient_short(q, s.div, s.rdiv);
+}
+
+// ------------------------------------------------------------------------------------- bf16
+// A wavefront owns 32 rows of one weight block and all tokens of a pass, in two tiles of 32.  For two
+// columns (j, j + 8) of the block, v_mfma_f32_32x32x4_2b_bf16 with the tokens as A, reduced to one of
+// its four k by zeroing the others, and the weights as B gives the exact products of 32 tokens x 32
+// rows in 32 registers: register i of the first half and of the second half are the same token and
+// row under j and j + 8.  One conversion rounds the two into a word.  Four such words of a lane (four
+// tokens) are an A operand of v_mfma_f32_16x16x32_bf16 in which every word is a k pair of its own; the
+// B operand, constant through the kernel, sends pair p to output column p, so the instruction adds
+// lo + hi of each of the 64 x 4 words to a sum of its own: lane l, register i of group a holds
+//   row 4 (l >> 4) + i + 16 ((l >> 2) & 1), token 8 a + 4 ((l >> 3) & 1) + (l & 3)
+// of the tile.  The partial outputs of the unclipped block stay in registers in the same places.
+// The weights are quantised as they are used, 16 columns at a time, by the lane that supplies them to
+// the matrix instruction; no LDS and no barrier anywhere.
+template <int BS>
+__device__ __forceinline__ void clip_losses_bf16(const uint16_t* __restrict__ x, int tokens,
+                                                 const uint16_t* __restrict__ w, int n, int k,
+                                                 const void* __restrict__ w_amax, int amax_dtype,
+                                                 const ClipRatios& ratios, int r0, int r1,
+                                                 const IntOp& op, float* __restrict__ loss) {
+    constexpr int NC = BS / 16;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int fr = lane & 31, kg = lane >> 5;
+    const int nblk = k / BS, b = blockIdx.y;
+    const int row0 = (blockIdx.x * kClipWaves + wave) * 32;
+    if (row0 >= n) return;
+    int row = row0 + fr < n ? row0 + fr : n - 1;
+    const float amax = load_scalar(w_amax, amax_dtype, (int64_t)row * nblk + b);
+    bf16x8_t pair_sum;
+    {
+        uint32_t m[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[i] = (lane & 15) == 4 * (lane >> 4) + i ? 0x3F803F80u : 0u;
+        __builtin_memcpy(&pair_sum, m, 16);
+    }
+    f32x32_t zero;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) zero[i] = 0.0f;
+    for (int t0 = 0; t0 < tokens; t0 += kClipTokens) {
+        int xrow[2];
+        bool live[2];   // a token past the end counts as a row of zeros
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            const int t = t0 + 32 * m + fr;
+            live[m] = t < tokens;
+            xrow[m] = live[m] ? t : tokens - 1;
+        }
+        // The addresses are made anew for every chunk from a row number: three 64-bit addresses kept
+        // across the chunk loop would cost the third wavefront of a SIMD.
+        u32x4 wraw, xraw[2];
+        auto fetch = [&](int c) {
+            asm volatile("" : "+v"(row), "+v"(xrow[0]), "+v"(xrow[1]));
+            const int col = b * BS + c * 16 + kg * 8;
+            wraw = *(const u32x4*)(w + ((int64_t)row * k + col));
+#pragma unroll
+            for (int m = 0; m < 2; ++m) xraw[m] = *(const u32x4*)(x + ((int64_t)xrow[m] * k + col));
+        };
+        fetch(0);
+        uint32_t org[2][8];   // rounded partial outputs of the unclipped block, two a word
+        for (int v = r0 - 1; v < r1; ++v) {   // r0 - 1: the unclipped block
+            IntOp::Scale s = {};
+            if (v >= r0) s = clip_scale(op, amax, amax_dtype, ratios.r[v]);
+            f32x4 acc[2][4];
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int a = 0; a < 4; ++a) acc[m][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+            for (int c = 0; c < NC; ++c) {
+                uint32_t wb[4] = {wraw.x, wraw.y, wraw.z, wraw.w};
+                if (v >= r0) {
+                    float q[8];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        q[2 * j] = u2f(wb[j] << 16);
+                        q[2 * j + 1] = u2f(wb[j] & 0xFFFF0000u);
+                    }
+                    // the choice between the exact-reciprocal quotient and a division is per block
+                    if (clip_fast(op, s)) {
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) q[j] = clip_qdq_fast(op, q[j], s);
+                    } else {
+                        keep_branch();
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) q[j] = op.apply<false>(q[j], s);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) wb[j] = f32x2_to_bf16x2(q[2 * j], q[2 * j + 1]);
+                }
+                uint32_t xb[2][4];
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    xb[m][0] = live[m] ? xraw[m].x : 0u;
+                    xb[m][1] = live[m] ? xraw[m].y : 0u;
+                    xb[m][2] = live[m] ? xraw[m].z : 0u;
+                    xb[m][3] = live[m] ? xraw[m].w : 0u;
+                }
+                fetch(c + 1 < NC ? c + 1 : 0);   // the first one again for the next ratio
+                auto products = [&](int q) {   // column q & 7 of either half of the chunk, tile q >> 3
+                    const int m = q >> 3, e = q & 7;
+                    const uint32_t one = xb[m][e >> 1] & ((e & 1) ? 0xFFFF0000u : 0x0000FFFFu);
+                    const uint32_t aw[2] = {(e & 2) ? 0u : one, (e & 2) ? one : 0u};
+                    const uint32_t bw[2] = {wb[(e >> 2) * 2], wb[(e >> 2) * 2 + 1]};
+                    s16x4_t av, bv;
+                    __builtin_memcpy(&av, aw, 8);
+                    __builtin_memcpy(&bv, bw, 8);
+                    return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(av, bv, zero, 0, 0, 0);
+                };
+                f32x32_t d = products(0);
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    f32x32_t ahead;   // the next products run under this step's conversions
+                    if (q + 1 < 16) ahead = products(q + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) {
+                        uint32_t pw[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) pw[i] = f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]);
+                        bf16x8_t pv;
+                        __builtin_memcpy(&pv, pw, 16);
+                        acc[q >> 3][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pv, pair_sum, acc[q >> 3][a], 0, 0, 0);
+                    }
+                    if (q + 1 < 16) d = ahead;
+                    // Steps stay apart: left alone, the scheduler converts the first of the products
+                    // ahead within this step and waits out the matrix instruction that makes them.
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (v < r0) {
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) {
+                        org[m][2 * a] = f32x2_to_bf16x2(acc[m][a][0], acc[m][a][1]);
+                        org[m][2 * a + 1] = f32x2_to_bf16x2(acc[m][a][2], acc[m][a][3]);
+                    }
+                continue;
+            }
+            float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int a = 0; a < 4; ++a)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const uint32_t o = org[m][2 * a + h];
+                        const uint32_t cur = f32x2_to_bf16x2(acc[m][a][2 * h], acc[m][a][2 * h + 1]);
+                        const uint32_t dd = f32x2_to_bf16x2(u2f(cur << 16) - u2f(o << 16),
+                                                            u2f(cur & 0xFFFF0000u) - u2f(o & 0xFFFF0000u));
+                        const float lo = u2f(dd << 16), hi = u2f(dd & 0xFFFF0000u);
+                        sum[2 * h] += lo * lo;
+                        sum[2 * h + 1] += hi * hi;
+                    }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {   // the other tokens of the rows: lane bits 0, 1 and 3
+                sum[i] += __shfl_xor(sum[i], 1, kWave);
+                sum[i] += __shfl_xor(sum[i], 2, kWave);
+                sum[i] += __shfl_xor(sum[i], 8, kWave);
+            }
+            if ((lane & 11) == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int r = row0 + 4 * (lane >> 4) + i + 16 * ((lane >> 2) & 1);
+                    if (r < n) loss[((int64_t)v * n + r) * nblk + b] += sum[i] / (float)tokens;
+                }
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------- fp16
+// A lane owns one row of one weight block, its quantised weights in registers, two a word; the
+// activations are uniform over the wavefront (scalar loads, two columns a word).  One v_pk_mul_f16 gives
+// two rounded products; the words of four tokens are an A operand of v_mfma_f32_16x16x32_f16 and are
+// summed as in the bf16 form: lane l, register i holds row 4 (l >> 4) + i + 16 ((l >> 2) & 3), token
+// l & 3 of the four.  The partial outputs of the unclipped block stay in LDS.
+template <int BS>
+__device__ __forceinline__ void clip_losses_f16(const uint16_t* __restrict__ x, int tokens,
+                                                const uint16_t* __restrict__ w, int n, int k,
+                                                const void* __restrict__ w_amax, int amax_dtype,
+                                                const ClipRatios& ratios, int r0, int r1, const IntOp& op,
+                                                float* __restrict__ loss, u32x2* __restrict__ org) {
+    constexpr int GW = 4;            // words of a token read ahead together (8 columns)
+    constexpr int NG = BS / 2 / GW;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nblk = k / BS, b = blockIdx.y;
+    const int row0 = (blockIdx.x * kClipWaves + wave) * kClipLanes;
+    if (row0 >= n) return;
+    org += (size_t)wave * (kClipTokens / 4) * kClipLanes + lane;
+    const int row = row0 + lane < n ? row0 + lane : n - 1;
+    const uint16_t* wp = w + (int64_t)row * k + b * BS;
+    const float amax = load_scalar(w_amax, amax_dtype, (int64_t)row * nblk + b);
+    f16x8_t pair_sum;
+    {
+        uint32_t m[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[i] = (lane & 15) == 4 * (lane >> 4) + i ? 0x3C003C00u : 0u;
+        __builtin_memcpy(&pair_sum, m, 16);
+    }
+    const uint32_t* xw = (const uint32_t*)(x + b * BS);
+    const int xstride = k / 2;
+    uint32_t wq[BS / 2];
+    for (int t0 = 0; t0 < tokens; t0 += kClipTokens) {
+        const int tc = tokens - t0 < kClipTokens ? tokens - t0 : kClipTokens;
+        for (int v = r0 - 1; v < r1; ++v) {   // r0 - 1: the unclipped block
+            IntOp::Scale s = {};
+            if (v >= r0) s = clip_scale(op, amax, amax_dtype, ratios.r[v]);
+            // opaque to the optimiser, which would otherwise keep the block live beside its
+            // quantised form instead of reading it again (L2) for every ratio
+            const uint16_t* src = wp;
+            asm volatile("" : "+v"(src));
+#pragma unroll
+            for (int c0 = 0; c0 < BS / 8; c0 += 2) {
+                u32x4 raw[2] = {*(const u32x4*)(src + 8 * c0), *(const u32x4*)(src + 8 * c0 + 8)};
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const uint32_t rw[4] = {raw[c].x, raw[c].y, raw[c].z, raw[c].w};
+                    float q[8];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        q[2 * j] = f16_bits_to_f32(rw[j] & 0xFFFFu);
+                        q[2 * j + 1] = f16_bits_to_f32(rw[j] >> 16);
+                    }
+                    if (v >= r0) {
+                        if (clip_fast(op, s)) {
+#pragma unroll
+                            for (int j = 0; j < 8; ++j) q[j] = clip_qdq_fast(op, q[j], s);
+                        } else {
+                            keep_branch();
+#pragma unroll
+                            for (int j = 0; j < 8; ++j) q[j] = op.apply<false>(q[j], s);
+                        }
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            wq[4 * (c0 + c) + j] = f32_to_f16_bits(q[2 * j]) | (f32_to_f16_bits(q[2 * j + 1]) << 16);
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) wq[4 * (c0 + c) + j] = rw[j];
+                    }
+                }
+            }
+            float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int g4 = 0; g4 * 4 < tc; ++g4) {
+                const uint32_t* xr[4];   // past the end: the last token again, left out below
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int t = 4 * g4 + i < tc ? 4 * g4 + i : tc - 1;
+                    xr[i] = xw + (int64_t)(t0 + t) * xstride;
+                }
+                f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+                uint32_t cur[4][GW];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < GW; ++j) cur[i][j] = xr[i][j];
+#pragma unroll
+                for (int g = 0; g < NG; ++g) {
+                    uint32_t next[4][GW];
+                    if (g + 1 < NG) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+#pragma unroll
+                            for (int j = 0; j < GW; ++j) next[i][j] = xr[i][GW * (g + 1) + j];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int j = 0; j < GW; ++j) {
+                        uint32_t pw[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            f16x2_t a, c;
+                            __builtin_memcpy(&a, &cur[i][j], 4);
+                            __builtin_memcpy(&c, &wq[GW * g + j], 4);
+                            const f16x2_t p = a * c;
+                            __builtin_memcpy(&pw[i], &p, 4);
+                        }
+                        f16x8_t pv;
+                        __builtin_memcpy(&pv, pw, 16);
+                        acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pv, pair_sum, acc[j & 1], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (g + 1 < NG) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+#pragma unroll
+                            for (int j = 0; j < GW; ++j) cur[i][j] = next[i][j];
+                    }
+                }
+                float out[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) out[i] = clip_round<MO_F16>(acc[0][i] + acc[1][i]);
+                if (v < r0) {
+                    u32x2 o;
+                    o.x = f32_to_f16_bits(out[0]) | (f32_to_f16_bits(out[1]) << 16);
+                    o.y = f32_to_f16_bits(out[2]) | (f32_to_f16_bits(out[3]) << 16);
+                    org[g4 * kClipLanes] = o;
+                } else {
+                    const u32x2 o = org[g4 * kClipLanes];
+                    const float og[4] = {f16_bits_to_f32(o.x & 0xFFFFu), f16_bits_to_f32(o.x >> 16),
+                                         f16_bits_to_f32(o.y & 0xFFFFu), f16_bits_to_f32(o.y >> 16)};
+                    const bool counts = 4 * g4 + (lane & 3) < tc;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float d = clip_round<MO_F16>(out[i] - og[i]);
+                        sum[i] += counts ? d * d : 0.0f;
+                    }
+                }
+            }
+            if (v < r0) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {   // the other tokens of the rows: lane bits 0 and 1
+                sum[i] += __shfl_xor(sum[i], 1, kWave);
+                sum[i] += __shfl_xor(sum[i], 2, kWave);
+            }
+            if ((lane & 3) == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int r = row0 + 4 * (lane >> 4) + i + 16 * ((lane >> 2) & 3);
+                    if (r < n) loss[((int64_t)v * n + r) * nblk + b] += sum[i] / (float)tokens;
+                }
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------- fp32
+// A lane owns one (output row, block), its quantised weights in registers; the activations of a token
+// are uniform over the wavefront and are read through scalar loads; org[] of a lane lives in LDS
+// ([token][lane], conflict-free).  A weight with few (row, block) pairs does not fill the chip with
+// one wavefront per 64 pairs, so a workgroup may hold 2 wavefronts that own the same 64 pairs and
+// share the tokens of a pass between them; their partial sums meet in LDS and wavefront 0 adds them in
+// wavefront order, so the result does not depend on timing.
 //
-// x is uniform over the wavefront: it is read through scalar loads, 16 elements a group, and
-// unpacking 16-bit pairs is scalar-ALU work.  The loads are software-pipelined one group ahead
-// (across token boundaries too); scalar loads return out of order, so a wait covers every load
-// in flight, hence the order "use the group that has arrived, then issue the next load, then
-// do the vector work", which the scheduling barriers pin down.
-template <int DT, int BS, typename Fn>
-__device__ __forceinline__ void token_dots(const void* __restrict__ x, int64_t x0, int64_t stride,
+// For each of `tc` tokens, sum_j x[t, j] * w[j] in index order, handed to fn(t, value).  The scalar
+// loads are software-pipelined one group of 16 elements ahead (across token boundaries too); they return
+// out of order, so a wait covers every load in flight, hence the order "use the group that has
+// arrived, then issue the next load, then do the vector work", which the scheduling barriers pin down.
+template <int BS, typename Fn>
+__device__ __forceinline__ void token_dots(const float* __restrict__ x, int64_t x0, int64_t stride,
                                            int tc, const float (&w)[BS], Fn fn) {
     constexpr int NG = BS / 16;
-    constexpr int WORDS = DT == MO_F32 ? 16 : 8;   // dwords per group of 16 elements
-    const uint32_t* xp = (const uint32_t*)((const char*)x + x0 * Elem<DT>::bytes);
-    const int64_t stride_words = stride * Elem<DT>::bytes / 4;
-    uint32_t cur[WORDS];
+    const float* xp = x + x0;
+    float cur[16];
 #pragma unroll
-    for (int j = 0; j < WORDS; ++j) cur[j] = xp[j];
+    for (int j = 0; j < 16; ++j) cur[j] = xp[j];
     for (int t = 0; t < tc; ++t) {
-        const uint32_t* row = xp + (int64_t)t * stride_words;
+        const float* row = xp + (int64_t)t * stride;
         // the group after the last one of this token: the first of the next token (of this
         // token again after the last, a valid address whose data is not used)
-        const uint32_t* next_row = t + 1 < tc ? row + stride_words : row;
+        const float* next_row = t + 1 < tc ? row + stride : row;
         // four partial sums: the order of the fp32 accumulation is free, a single chain of
         // dependent adds is not
         float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -72,81 +426,33 @@ __device__ __forceinline__ void token_dots(const void* __restrict__ x, int64_t x
         for (int g = 0; g < NG; ++g) {
             float xs[16];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                if constexpr (DT == MO_F32) xs[j] = u2f(cur[j]);
-                else if constexpr (DT == MO_BF16)
-                    xs[j] = (j & 1) ? u2f(cur[j / 2] & 0xFFFF0000u) : u2f(cur[j / 2] << 16);
-                else
-                    xs[j] = f16_bits_to_f32((j & 1) ? cur[j / 2] >> 16 : cur[j / 2] & 0xFFFFu);
-            }
+            for (int j = 0; j < 16; ++j) xs[j] = cur[j];
             __builtin_amdgcn_sched_barrier(0);
-            const uint32_t* nxt = g + 1 < NG ? row + (g + 1) * WORDS : next_row;
+            const float* nxt = g + 1 < NG ? row + (g + 1) * 16 : next_row;
 #pragma unroll
-            for (int j = 0; j < WORDS; ++j) cur[j] = nxt[j];
+            for (int j = 0; j < 16; ++j) cur[j] = nxt[j];
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < 16; j += 2) {
-                if constexpr (DT == MO_BF16) {
-                    // both rounded products in one word (one conversion for the pair), added to
-                    // a running sum by one instruction: v_dot2c_f32_bf16(pair, (1, 1), acc) =
-                    // acc + pair.lo + pair.hi.  Four vector instructions per two products where
-                    // multiply, round and add one by one take six.  The instruction's add is
-                    // not a correctly rounded fp32 add (about 2e-6 relative at worst) and it
-                    // flushes bf16 denormals; the sum is rounded to bf16 below, and measured
-                    // against the CPU's arithmetic the losses come out bit-equal as often as
-                    // with exact adds (the difference that shows is the order of the adds).
-                    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-                    const uint32_t pk = f32x2_to_bf16x2(xs[j] * w[16 * g + j], xs[j + 1] * w[16 * g + j + 1]);
-                    const uint32_t one2 = 0x3F803F80u;   // (1.0, 1.0)
-                    bf16x2_t pv, ov;
-                    __builtin_memcpy(&pv, &pk, 4);
-                    __builtin_memcpy(&ov, &one2, 4);
-                    acc[(j / 2) & 3] = __builtin_amdgcn_fdot2_f32_bf16(pv, ov, acc[(j / 2) & 3], false);
-                } else {
-                    acc[j & 3] += clip_round<DT>(xs[j] * w[16 * g + j]);
-                    acc[(j + 1) & 3] += clip_round<DT>(xs[j + 1] * w[16 * g + j + 1]);
-                }
-            }
+            for (int j = 0; j < 16; ++j) acc[j & 3] += xs[j] * w[16 * g + j];
             __builtin_amdgcn_sched_barrier(0);
         }
-        fn(t, clip_round<DT>((acc[0] + acc[1]) + (acc[2] + acc[3])));
+        fn(t, (acc[0] + acc[1]) + (acc[2] + acc[3]));
     }
 }
 
-// org[] of a lane in LDS, [token][lane] (conflict-free), stored in the tensor dtype (the values
-// are rounded to it anyway).
-template <int DT> struct OrgStore { typedef uint16_t type; };
-template <> struct OrgStore<MO_F32> { typedef float type; };
-
-template <int DT>
-__device__ __forceinline__ typename OrgStore<DT>::type org_pack(float v) {
-    if constexpr (DT == MO_F32) return v;
-    else if constexpr (DT == MO_BF16) return (uint16_t)(f2u(v) >> 16);
-    else return (uint16_t)f32_to_f16_bits(v);
-}
-
-template <int DT>
-__device__ __forceinline__ float org_unpack(typename OrgStore<DT>::type v) {
-    if constexpr (DT == MO_F32) return v;
-    else if constexpr (DT == MO_BF16) return u2f((uint32_t)v << 16);
-    else return f16_bits_to_f32(v);
-}
-
-template <int DT, int BS>
-__global__ __launch_bounds__(kClipLanes * kClipMaxSplit) void awq_clip_loss_kernel(
-    const void* __restrict__ x, int tokens, const void* __restrict__ w, int n, int k,
-    const void* __restrict__ w_amax, int amax_dtype, ClipRatios ratios, IntOp op,
-    float* __restrict__ loss) {
+template <int BS>
+__device__ __forceinline__ void clip_losses_f32(const float* __restrict__ x, int tokens,
+                                                const float* __restrict__ w, int n, int k,
+                                                const void* __restrict__ w_amax, int amax_dtype,
+                                                const ClipRatios& ratios, int r0, int r1, const IntOp& op,
+                                                float* __restrict__ loss, float* smem) {
     constexpr int NC = BS / 8;
     constexpr int GC = NC < 4 ? NC : 4;   // chunks loaded together
-    typedef typename OrgStore<DT>::type org_t;
-    // dynamic LDS: org[pass_tokens][64] in the tensor dtype, then part[2][split][64] fp32
-    extern __shared__ __align__(16) unsigned char clip_smem[];
+    // dynamic LDS: org[pass_tokens][64], then part[2][split][64]
     const int split = blockDim.x / kClipLanes;
     const int pass_tokens = split * kClipTokens;
-    org_t (*org)[kClipLanes] = (org_t (*)[kClipLanes])clip_smem;
-    float (*part)[kClipLanes] =
-        (float (*)[kClipLanes])(clip_smem + (size_t)pass_tokens * kClipLanes * sizeof(org_t));
+    float (*org)[kClipLanes] = (float (*)[kClipLanes])smem;
+    float (*part)[kClipLanes] = org + pass_tokens;
     const int lane = threadIdx.x % kClipLanes;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kClipLanes);
     const int nblk = k / BS;
@@ -167,13 +473,13 @@ __global__ __launch_bounds__(kClipLanes * kClipMaxSplit) void awq_clip_loss_kern
         asm volatile("" : "+v"(base));
 #pragma unroll
         for (int c0 = 0; c0 < NC; c0 += GC) {
-            RawChunk<DT> raw[GC];
+            RawChunk<MO_F32> raw[GC];
 #pragma unroll
-            for (int c = 0; c < GC; ++c) load_raw<DT>(w, base + 8 * (c0 + c), raw[c]);
+            for (int c = 0; c < GC; ++c) load_raw<MO_F32>(w, base + 8 * (c0 + c), raw[c]);
 #pragma unroll
             for (int c = 0; c < GC; ++c) {
                 float v[8];
-                unpack_raw<DT>(raw[c], v);
+                unpack_raw<MO_F32>(raw[c], v);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) wv[8 * (c0 + c) + j] = f(v[j]);
             }
@@ -188,26 +494,16 @@ __global__ __launch_bounds__(kClipLanes * kClipMaxSplit) void awq_clip_loss_kern
         const int mine = (int)((int64_t)tc * (wave + 1) / split) - lo;
         const int64_t x0 = (int64_t)(t0 + lo) * k + xb;
         refill([](float v) { return v; });
-        token_dots<DT, BS>(x, x0, k, mine, wv,
-                           [&](int t, float v) { org[lo + t][lane] = org_pack<DT>(v); });
-        for (int r = 0; r < ratios.count; ++r) {
-            // `w_amax * ratio` on a tensor: fp32 product rounded to the dtype of the amax
-            float clipped = amax * ratios.r[r];
-            if (amax_dtype == MO_BF16) clipped = clip_round<MO_BF16>(clipped);
-            else if (amax_dtype == MO_F16) clipped = clip_round<MO_F16>(clipped);
-            IntOp::Scale s = op.make(clipped);
+        token_dots<BS>(x, x0, k, mine, wv, [&](int t, float v) { org[lo + t][lane] = v; });
+        for (int r = r0; r < r1; ++r) {
+            const IntOp::Scale s = clip_scale(op, amax, amax_dtype, ratios.r[r]);
             // the choice between the exact-reciprocal quotient and a division is per block, not
             // per element: one branch around the whole loop
-            if (s.fast) {
-                s.fast = true;
-                refill([&](float v) { return clip_round<DT>(op.apply<false>(v, s)); });
-            } else {
-                s.fast = false;
-                refill([&](float v) { return clip_round<DT>(op.apply<false>(v, s)); });
-            }
+            if (clip_fast(op, s)) refill([&](float v) { return clip_qdq_fast(op, v, s); });
+            else refill([&](float v) { return op.apply<false>(v, s); });
             float sum = 0.0f;
-            token_dots<DT, BS>(x, x0, k, mine, wv, [&](int t, float cur) {
-                const float d = clip_round<DT>(cur - org_unpack<DT>(org[lo + t][lane]));
+            token_dots<BS>(x, x0, k, mine, wv, [&](int t, float cur) {
+                const float d = cur - org[lo + t][lane];
                 sum += d * d;
             });
             if (split > 1) {
@@ -225,6 +521,26 @@ __global__ __launch_bounds__(kClipLanes * kClipMaxSplit) void awq_clip_loss_kern
             }
         }
     }
+}
+
+// blockIdx.z takes the ratios [z R / Z, (z + 1) R / Z): each share scores the unclipped block for itself
+template <int DT, int BS>
+__global__ __launch_bounds__(kClipLanes * kClipWaves, DT == MO_BF16 ? 3 : 2) void awq_clip_loss_kernel(
+    const void* __restrict__ x, int tokens, const void* __restrict__ w, int n, int k,
+    const void* __restrict__ w_amax, int amax_dtype, ClipRatios ratios, IntOp op,
+    float* __restrict__ loss) {
+    extern __shared__ __align__(16) unsigned char clip_smem[];
+    const int r0 = (int)(blockIdx.z * (unsigned)ratios.count / gridDim.z);
+    const int r1 = (int)((blockIdx.z + 1) * (unsigned)ratios.count / gridDim.z);
+    if constexpr (DT == MO_BF16)
+        clip_losses_bf16<BS>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype, ratios,
+                             r0, r1, op, loss);
+    else if constexpr (DT == MO_F16)
+        clip_losses_f16<BS>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype, ratios,
+                            r0, r1, op, loss, (u32x2*)clip_smem);
+    else
+        clip_losses_f32<BS>((const float*)x, tokens, (const float*)w, n, k, w_amax, amax_dtype, ratios, r0, r1,
+                            op, loss, (float*)clip_smem);
 }
 
 }  // namespace mo
@@ -253,25 +569,40 @@ extern "C" int mo_awq_clip_losses(const void* x, int64_t tokens, const void* w, 
     mo::IntOp op;
     op.bound = (float)((1 << (num_bits - 1 + (is_unsigned ? 1 : 0))) - 1);
     op.lo = is_unsigned ? 0.0f : (narrow_range ? -op.bound : -op.bound - 1.0f);
-    const dim3 grid((unsigned)((n + mo::kClipLanes - 1) / mo::kClipLanes),
-                    (unsigned)(k / block_size));
-    // Wavefronts per 64 (row, block) pairs.  Measured on 4096-wide rows, 64 tokens, bf16: up to
-    // about 2048 such sets (two wavefronts per SIMD) a workgroup of four -- one wavefront on
-    // each SIMD of a compute unit -- is faster (1024 rows: 848 -> 406 us, 2048 rows: 870 ->
-    // 729 us, 3072 rows: 1349 -> 1043 us); from 2048 sets on the single wavefront is (4096 rows:
-    // 1359 us either way, 14336 rows: 4017 against 4642 us).  Eight are slower than four
-    // everywhere.  Each wavefront should still get 8 tokens or more.
-    const int64_t sets = (int64_t)grid.x * grid.y;
-    int split = sets < mo::tuned("clip_split_below_sets", 2048) ? mo::kClipMaxSplit : 1;
-    while (split > 1 && tokens < 8 * split) split /= 2;
-    const size_t elem = dtype == MO_F32 ? 4 : 2;
-    if (dtype == MO_F32 && split > 2) split = 2;   // org[] of a pass stays within 64 KB of LDS
-    split = (int)mo::tuned("clip_split", split);
-    const size_t smem = (size_t)split * mo::kClipTokens * mo::kClipLanes * elem +
-                        (split > 1 ? (size_t)2 * split * mo::kClipLanes * sizeof(float) : 0);
+    const int rows_per_group = dtype == MO_BF16 ? 32 * mo::kClipWaves
+                               : dtype == MO_F16 ? mo::kClipLanes * mo::kClipWaves : mo::kClipLanes;
+    dim3 grid((unsigned)((n + rows_per_group - 1) / rows_per_group), (unsigned)(k / block_size));
+    int waves = mo::kClipWaves;
+    size_t smem = 0;
+    if (dtype == MO_F32) {
+        // Up to about 2048 sets of 64 pairs (two wavefronts per SIMD) two wavefronts to a set are
+        // faster, from there on one is; each should still get 8 tokens or more, and org[] of a pass
+        // stays within 64 KB of LDS.
+        const int64_t sets = (int64_t)grid.x * grid.y;
+        waves = sets < 2048 && tokens >= 16 ? 2 : 1;
+        smem = (size_t)waves * mo::kClipTokens * mo::kClipLanes * 4 +
+               (waves > 1 ? (size_t)2 * waves * mo::kClipLanes * sizeof(float) : 0);
+    } else {
+        if (dtype == MO_F16) smem = (size_t)mo::kClipWaves * mo::kClipTokens * mo::kClipLanes * 2;
+        // A wavefront goes through all ratios unless there are too few of them to fill the chip; then
+        // 2 to 11 of them share the ratios, each scoring the unclipped block once more.  11 ratios, 64
+        // tokens, blocks of 128 (before: one vector-ALU kernel for both types, 1070 / 2160 us on the
+        // first line):
+        //   bf16  4096 x 4096, 4096 wavefronts: 464 us (2 shares: 488); 1024 x 4096, 1024: 147, 137 with 2,
+        //         138 with 3; 1024 x 1024, 256: 143, 86 with 2, 50 with 4, 55 with 8
+        //   fp16  4096 x 4096, 2048 wavefronts: 496 us, 430 with 2 shares, 450 with 4; 1024 x 4096, 512:
+        //         307, 143 with 4, 156 with 8; 1024 x 1024, 128: 272, 95 with 4, 71 with 8, 69 with 11
+        // What bounds the bf16 form: a step of 2048 products is 128 cycles of matrix instructions and
+        // about 110 of vector instructions plus 40 of the port that issues both; measured 180.
+        const int64_t sets = (int64_t)grid.x * grid.y * mo::kClipWaves;
+        int64_t share = ((dtype == MO_BF16 ? 2048 : 3072) + sets - 1) / sets;
+        if (dtype == MO_BF16 && share > 4) share = 4;
+        if (share > n_ratios) share = n_ratios;
+        grid.z = (unsigned)mo::tuned("clip_shares", share);
+    }
     hipStream_t s = (hipStream_t)stream;
 #define CALL(DT, BS)                                                                       \
-    mo::awq_clip_loss_kernel<DT, BS><<<grid, mo::kClipLanes * split, smem, s>>>(           \
+    mo::awq_clip_loss_kernel<DT, BS><<<grid, mo::kClipLanes * waves, smem, s>>>(           \
         x, (int)tokens, w, (int)n, (int)k, w_amax, amax_dtype, rr, op, loss)
 #define BY_BS(DT)                                                         \
     switch (block_size) {                                                 \

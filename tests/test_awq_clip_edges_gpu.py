@@ -1,0 +1,70 @@
+"""The 16-bit clip search at the edges of its tiles: 32 rows (bf16) or 64 rows (fp16) per wavefront, tiles
+of 32 tokens or groups of 4, passes of 64, shares of the ratios, codes too wide for the short
+quotient, blocks whose scale leaves the range of the reciprocal."""
+
+import pytest
+import torch
+
+from modelopt_amd import _hip
+from oracle import awq as oawq
+from oracle import reduce
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+RATIOS = [round(0.5 + 0.05 * i, 2) for i in range(10)] + [1.0]
+
+
+def _case(n, k, tokens, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    w = (0.05 * torch.randn(n, k, generator=g)).to(dtype)
+    x = (torch.randn(tokens, k, generator=g) * torch.exp(0.5 * torch.randn(1, k, generator=g))).to(dtype)
+    return w, x
+
+
+def _losses(w, x, block, num_bits=4, ratios=RATIOS):
+    w_amax = reduce.reduce_amax(w.reshape(-1, block), axis=[1], keepdims=True)
+    loss = torch.zeros(len(ratios), w.shape[0], w.shape[1] // block, device=DEV)
+    assert _hip.awq_clip_losses_into(x.to(DEV), w.to(DEV), w_amax.to(DEV), ratios, block, num_bits, False, False, loss)
+    return loss.cpu()
+
+
+def _check(got, want):
+    """Sums in another order flip the rounding of a partial output now and then (one step of the dtype
+    of one token's error); the losses of a ratio agree on aggregate as in the tests of the kernel."""
+    for i, r in enumerate(RATIOS):
+        assert float((got[i] - want[r]).abs().sum() / want[r].abs().sum()) < 2e-4, r
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,k,tokens,block", [
+    (1, 16, 1, 16), (31, 64, 31, 16), (33, 128, 32, 128), (65, 256, 33, 64), (129, 128, 63, 32), (257, 128, 66, 128),
+    (130, 64, 5, 64), (64, 32, 127, 32)])
+def test_tile_edges(dtype, n, k, tokens, block):
+    w, x = _case(n, k, tokens, dtype, n + tokens)
+    want, _ = oawq.awq_clip_search(w, [x], block, 4, max_tokens_per_batch=1 << 20)
+    _check(_losses(w, x, block), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wide_codes_and_extreme_scales(dtype):
+    w, x = _case(40, 128, 20, dtype, 3)
+    want, _ = oawq.awq_clip_search(w, [x], 64, 13, max_tokens_per_batch=1 << 20)
+    got = _losses(w, x, 64, num_bits=13)
+    for i, r in enumerate(RATIOS[:-1]):    # 13 bits: only clipping costs anything worth comparing
+        assert float((got[i] - want[r]).abs().sum() / want[r].abs().sum()) < 2e-4, r
+    if dtype == torch.bfloat16:            # a block below 2^-64: the divided form, exact zeros apart
+        w[:, :64] *= 2.0 ** -90
+        want, _ = oawq.awq_clip_search(w, [x], 64, 4, max_tokens_per_batch=1 << 20)
+        _check(_losses(w, x, 64), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_shares_of_the_ratios_give_the_same_bits(dtype):
+    """few rows share the ratios between wavefronts, many do not; a row's losses do not depend on it"""
+    w, x = _case(4096, 1024, 40, dtype, 9)
+    whole = _losses(w, x, 16)
+    for r0 in (0, 1024, 4032):
+        rows = slice(r0, r0 + 64)
+        assert torch.equal(_losses(w[rows].contiguous(), x, 16), whole[:, rows])
+        one = _losses(w[rows].contiguous(), x, 16, ratios=RATIOS[3:4])
+        assert torch.equal(one[0], whole[3, rows])
