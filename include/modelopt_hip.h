@@ -215,6 +215,21 @@ int mo_absmax_blocks2d(const void* x, int64_t rows, int64_t cols, int64_t block_
 int mo_nvfp4_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* amax,
                  int amax_dtype, int block_size, int mode, void* stream);
 
+/* Fake quantisation of x[rows, k] with one abs-max for the tensor or block scales along k, for rows of
+ * any length and alignment, optionally of T(x * pre_scale[column]) instead of x:
+ *   MO_ROW_INT    p0 = num_bits, p1 = is_unsigned, p2 = narrow_range   (mo_int_qdq)
+ *   MO_ROW_FP8    p0 = saturate                                        (mo_fp8_qdq)
+ *   MO_ROW_NVFP4  p0 = block size 8 / 16 / 32, p1 = mode               (mo_nvfp4_qdq)
+ *   MO_ROW_MX     p0 = block size 8 / 16 / 32, p1 = element format, power-of-two block scales, no amax
+ *                                                                      (mo_block_fp_qdq)
+ * with the arithmetic of the entry point in brackets.  pre_scale (optional): k elements of type dtype, the
+ * pre_quant_scale of TensorQuantizer.forward (TQ/nn/modules/tensor_quantizer.py:881-882), multiplied and
+ * rounded to dtype before anything else: the reference passes over the tensor once for the product and
+ * again for the quantizer.  x, y and pre_scale aligned to their elements.  y may alias x. */
+enum mo_row_kind { MO_ROW_INT = 0, MO_ROW_FP8 = 1, MO_ROW_NVFP4 = 2, MO_ROW_MX = 3 };
+int mo_row_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* pre_scale,
+               int kind, int p0, int p1, int p2, const void* amax, int amax_dtype, void* stream);
+
 /* ------------------------------------------------------------------ real quantize + pack */
 
 /* Squared fake-quantisation error for n_cand candidate amax values in one pass over x viewed

@@ -246,6 +246,83 @@ __device__ __forceinline__ void store_chunk_guarded(void* p, int64_t base, int64
         if (col + j < limit) store_elem<DT>(p, base + col + j, v[j]);
 }
 
+// ---------------------------------------------------------------- chunks of rows of any length
+// Division of a chunk number below 2^31 by the chunks of a row: one multiply and a shift.
+struct RowDiv { uint32_t d, m, s; };
+inline RowDiv row_div(uint32_t d) {   // 1 <= d < 2^31
+    RowDiv r = {d, 0, 0};
+    uint32_t l = 0;
+    while ((1ull << l) < d) ++l;
+    // m = ceil(2^(31 + l) / d) exceeds the exact quotient by less than d <= 2^l parts in 2^(31 + l), which
+    // moves n * m by less than 2^(31 + l) for n < 2^31: the floor stays that of n / d
+    r.m = (uint32_t)(((1ull << (31 + l)) + d - 1) / d);
+    r.s = l;
+    return r;
+}
+__device__ __forceinline__ uint32_t row_of(uint32_t chunk, const RowDiv& r) {
+    return r.s == 0 ? chunk : __umulhi(chunk, r.m) >> (r.s - 1);
+}
+
+// Elements [col, col + 8) of the row that starts at element `base`, of which only columns below k
+// exist (the rest read as zero): one 16-byte access at whatever alignment the row has -- global memory
+// accesses of gfx950 need none -- and element accesses only where the row ends inside the chunk.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+template <int DT>
+__device__ __forceinline__ void load_raw_row(const void* p, int64_t base, int64_t col, int64_t k,
+                                             RawChunk<DT>& r) {
+    zero_raw<DT>(r);
+    if (col + 8 <= k) {
+        if constexpr (DT == MO_F32) {
+            const u32x4_any* q = (const u32x4_any*)((const float*)p + base + col);
+            r.a = __builtin_nontemporal_load(q);
+            r.b = __builtin_nontemporal_load(q + 1);
+        } else {
+            r.a = __builtin_nontemporal_load((const u32x4_any*)((const uint16_t*)p + base + col));
+        }
+    } else if (col < k) {
+        if constexpr (DT == MO_F32) {
+            const uint32_t* q = (const uint32_t*)p + base;
+            uint32_t w[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) w[j] = col + j < k ? q[col + j] : 0u;
+            r.a = u32x4{w[0], w[1], w[2], w[3]};
+            r.b = u32x4{w[4], w[5], w[6], w[7]};
+        } else {
+            const uint16_t* q = (const uint16_t*)p + base;
+            uint32_t w[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                w[j] = (col + 2 * j < k ? (uint32_t)q[col + 2 * j] : 0u) |
+                       (col + 2 * j + 1 < k ? (uint32_t)q[col + 2 * j + 1] << 16 : 0u);
+            r.a = u32x4{w[0], w[1], w[2], w[3]};
+        }
+    }
+}
+
+template <int DT>
+__device__ __forceinline__ void store_row(void* p, int64_t base, int64_t col, int64_t k, const float (&v)[8]) {
+    if (col + 8 <= k) {
+        if constexpr (DT == MO_F32) {
+            u32x4_any* q = (u32x4_any*)((float*)p + base + col);
+            u32x4_any a = {f2u(v[0]), f2u(v[1]), f2u(v[2]), f2u(v[3])}, b = {f2u(v[4]), f2u(v[5]), f2u(v[6]), f2u(v[7])};
+            __builtin_nontemporal_store(a, q);
+            __builtin_nontemporal_store(b, q + 1);
+        } else {
+            uint32_t w[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (DT == MO_BF16) w[j] = f32x2_to_bf16x2(v[2 * j], v[2 * j + 1]);
+                else w[j] = f32_to_f16_bits(v[2 * j]) | (f32_to_f16_bits(v[2 * j + 1]) << 16);
+            }
+            u32x4_any a = {w[0], w[1], w[2], w[3]};
+            __builtin_nontemporal_store(a, (u32x4_any*)((uint16_t*)p + base + col));
+        }
+    } else {
+        store_chunk_guarded<DT>(p, base, col, k, v);
+    }
+}
+
 // Scalar read of an amax / scale operand given in any of the three float dtypes.
 __device__ __forceinline__ float load_scalar(const void* p, int dtype, int64_t i) {
     if (dtype == MO_F32) return ((const float*)p)[i];

@@ -40,6 +40,7 @@ SIGNATURES = {
     "mo_fp8_qdq": [_P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _P],
     "mo_int_qdq": [_P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _P],
     "mo_ste_mask": [_P, _P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _P],
+    "mo_row_qdq": [_P, _P, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _P, _INT, _P],
     "mo_nvfp4_qdq": [_P, _P, _I64, _I64, _INT, _P, _INT, _INT, _INT, _P],
     "mo_qdq_sq_err": [_P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _INT, _INT, _P, _P],
     "mo_mxfp4_quantize": [_P, _I64, _INT, _INT, _P, _P, _P],
@@ -415,6 +416,23 @@ def qdq_sq_err_into(x, cand, loss, outer, axis, inner, kind, num_bits=8, unsigne
     if rc != 0:
         raise RuntimeError(f"mo_qdq_sq_err failed: {load().mo_error_string(rc).decode()}")
     return True
+
+
+MO_ROW_INT, MO_ROW_FP8, MO_ROW_NVFP4, MO_ROW_MX = 0, 1, 2, 3   # enum mo_row_kind
+
+
+def row_qdq(x, pre_scale, kind, p0=0, p1=0, p2=0, amax=None):
+    """Fake quantisation of ``T(x * pre_scale)`` (``x`` itself when ``pre_scale`` is None) along the last dim
+    in one pass; ``kind`` and ``p0`` .. ``p2`` as in ``mo_row_qdq``, ``amax`` one device element (None for
+    ``MO_ROW_MX``)."""
+    _require_device(x, pre_scale, amax)
+    assert x.is_contiguous() and (pre_scale is None or (pre_scale.is_contiguous() and pre_scale.dtype == x.dtype
+                                                        and pre_scale.numel() == x.shape[-1]))
+    k = x.shape[-1]
+    y = torch.empty_like(x)
+    call("mo_row_qdq", x, _ptr(x), _ptr(y), x.numel() // k if k else 0, k, dtype_code(x.dtype), _ptr(pre_scale),
+         kind, int(p0), int(p1), int(p2), _ptr(amax), MO_F32 if amax is None else dtype_code(amax.dtype), _stream(x))
+    return y
 
 
 ELEM_FORMATS = ["E4M3", "E5M2", "INT8", "E0M3", "E1M2", "E3M0", "E2M1", "E3M2", "E2M3", "E8M0"]

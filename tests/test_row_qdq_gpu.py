@@ -1,0 +1,84 @@
+"""Row-wise fake quantisation (pre-scaled, ragged or unaligned rows) against the kernels for whole tensors,
+which the oracle tests pin, on zero-padded copies; bit for bit."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from modelopt_amd import _hip
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+DTYPES = [torch.bfloat16, torch.float16, torch.float32]
+MX = {name: i for i, name in enumerate(_hip.ELEM_FORMATS[:-1])}
+
+
+def _bits(t):
+    return t.contiguous().view(torch.int32 if t.element_size() == 4 else torch.int16)
+
+
+def _whole(x, kind, p0, p1, p2, amax):
+    if kind == _hip.MO_ROW_INT:
+        return _hip.int_qdq(x, amax, 1, 1, x.numel(), p0, p1, p2)
+    if kind == _hip.MO_ROW_FP8:
+        return _hip.fp8_qdq(x, amax, 1, 1, x.numel(), bool(p0))
+    k, block = x.shape[-1], p0
+    padded = F.pad(x, (0, -k % block)).contiguous()
+    y = _hip.nvfp4_qdq(padded, amax, block, p1) if kind == _hip.MO_ROW_NVFP4 else _hip.block_fp_qdq(padded, block, p1)
+    return y[..., :k]
+
+
+KINDS = ([(_hip.MO_ROW_INT, 8, 0, 0), (_hip.MO_ROW_INT, 4, 1, 0), (_hip.MO_ROW_INT, 16, 0, 1),
+          (_hip.MO_ROW_FP8, 1, 0, 0), (_hip.MO_ROW_FP8, 0, 0, 0)]
+         + [(_hip.MO_ROW_NVFP4, b, m, 0) for b in (8, 16, 32) for m in (0, 1)]
+         + [(_hip.MO_ROW_MX, b, f, 0) for b, f in zip((8, 16, 32, 8, 16, 32, 8, 16, 32), MX.values())])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("kind,p0,p1,p2", KINDS)
+# one element, less than a chunk, one past a chunk or a block, whole blocks, tiles with a remainder
+@pytest.mark.parametrize("rows,k", [(1, 1), (3, 7), (5, 17), (2, 33), (7, 64), (130, 65), (33, 1030)])
+@pytest.mark.parametrize("pre", [False, True])
+def test_equals_the_whole_tensor_kernels(dtype, kind, p0, p1, p2, rows, k, pre):
+    g = torch.Generator().manual_seed(rows * 1000 + k)
+    x = (torch.randn(rows, k, generator=g) * torch.exp(torch.randn(rows, k, generator=g))).to(dtype)
+    x.view(-1)[::37] = 0.0
+    x.view(-1)[1::53] = -0.0
+    x = x.to(DEV)
+    s = torch.exp(0.5 * torch.randn(k, generator=g)).to(dtype).to(DEV) if pre else None
+    seen = x * s if pre else x
+    amax = None if kind == _hip.MO_ROW_MX else (0.8 * seen.abs().amax()).float().reshape(1)
+    got = _hip.row_qdq(x, s, kind, p0, p1, p2, amax)
+    assert torch.equal(_bits(got), _bits(_whole(seen, kind, p0, p1, p2, amax)))
+
+
+@pytest.mark.parametrize("kind,p0,p1,p2", [(_hip.MO_ROW_FP8, 1, 0, 0), (_hip.MO_ROW_NVFP4, 16, 0, 0), (_hip.MO_ROW_MX, 32, 0, 0)])
+def test_unaligned_base_and_non_finite_blocks(kind, p0, p1, p2):
+    g = torch.Generator().manual_seed(1)
+    flat = torch.randn(40 * 96 + 1, generator=g).bfloat16()
+    flat[5], flat[700], flat[1500] = float("nan"), float("inf"), float("-inf")
+    x = flat.to(DEV)[1:].view(40, 96)                 # two bytes off a 16-byte boundary
+    amax = torch.full((1,), 3.0, device=DEV)
+    got = _hip.row_qdq(x, None, kind, p0, p1, p2, None if kind == _hip.MO_ROW_MX else amax)
+    want = _whole(x.clone(), kind, p0, p1, p2, amax)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    keep = ~torch.isnan(want)
+    assert torch.equal(_bits(got[keep]), _bits(want[keep]))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("block", [8, 16, 32])
+@pytest.mark.parametrize("rows,k", [(1, 3), (9, 40), (130, 72), (17, 1000)])
+def test_nvfp4_quantize_of_ragged_rows_equals_padded_rows(dtype, block, rows, k):
+    g = torch.Generator().manual_seed(k)
+    x = torch.randn(rows, k, generator=g).to(dtype).to(DEV)
+    padded = F.pad(x, (0, -k % block)).contiguous()
+    amax = x.abs().amax().float()
+    got, want = (_hip.nvfp4_quantize(t, amax, block) for t in (x, padded))
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.uint8) if a.dtype != torch.float32 else a,
+                           b.view(torch.uint8) if b.dtype != torch.float32 else b)
+    # the literal division of every element, and the scales handed in, give the same codes
+    exact = _hip.nvfp4_quantize(x, amax, block, flags=_hip.MO_FLAG_FORCE_EXACT)
+    given = _hip.nvfp4_quantize(x, got[2], block, True, got[1])
+    assert torch.equal(exact[0], got[0]) and torch.equal(given[0], got[0])
