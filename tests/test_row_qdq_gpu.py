@@ -82,3 +82,42 @@ def test_nvfp4_quantize_of_ragged_rows_equals_padded_rows(dtype, block, rows, k)
     exact = _hip.nvfp4_quantize(x, amax, block, flags=_hip.MO_FLAG_FORCE_EXACT)
     given = _hip.nvfp4_quantize(x, got[2], block, True, got[1])
     assert torch.equal(exact[0], got[0]) and torch.equal(given[0], got[0])
+
+
+FORMATS = {
+    "int8": {"num_bits": 8}, "uint4": {"num_bits": 4, "unsigned": True}, "fp8": {"num_bits": (4, 3)},
+    "nvfp4": {"num_bits": (2, 1), "block_sizes": {-1: 16, "type": "dynamic", "scale_bits": (4, 3)}},
+    "mxfp6": {"num_bits": (3, 2), "block_sizes": {-1: 32, "type": "dynamic", "scale_bits": (8, 0)}},
+    "mxint8": {"num_bits": 8, "block_sizes": {-1: 8, "type": "dynamic", "scale_bits": (8, 0)}},
+    # two-level scales of another element format, and blocks of 64, have no one-pass form
+    "e1m2": {"num_bits": (1, 2), "block_sizes": {-1: 16, "type": "dynamic", "scale_bits": (4, 3)}},
+}
+
+
+@pytest.mark.parametrize("name", FORMATS)
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("form", ["plain", "transposed", "unaligned", "scale_fp32", "grad", "dynamic", "collects"])
+def test_a_pre_quant_scale_equals_the_scaled_input(name, dtype, form):
+    from modelopt_amd.torch.quantization.config import QuantizerAttributeConfig
+    from modelopt_amd.torch.quantization.nn import TensorQuantizer
+
+    g = torch.Generator().manual_seed(3)
+    flat = torch.randn(2 * 9 * 72 + 1, generator=g).mul_(3).to(dtype)
+    flat[77], flat[300], flat[900] = float("nan"), float("inf"), float("-inf")
+    flat = flat.to(DEV)
+    x = flat[1:] if form == "unaligned" else flat[:-1]
+    x = x.view(2, 72, 9).transpose(1, 2) if form == "transposed" else x.view(2, 9, 72)
+    scale = torch.exp(0.5 * torch.randn(72, generator=g)).to(torch.float32 if form == "scale_fp32" else dtype).to(DEV)
+    plain, scaled = (TensorQuantizer(QuantizerAttributeConfig(**FORMATS[name])) for _ in range(2))
+    scaled.pre_quant_scale = scale
+    if form != "dynamic" and not plain.is_mx_format:
+        plain.amax = scaled.amax = torch.tensor(2.5, dtype=dtype, device=DEV)
+    if form == "collects":
+        plain.enable_calib(), scaled.enable_calib()
+    if form == "grad":
+        x = x.clone().requires_grad_()
+    got, want = scaled(x), plain(x * scale)
+    assert got.dtype == want.dtype and got.shape == want.shape
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    keep = ~torch.isnan(want)
+    assert torch.equal(got[keep], want[keep])
