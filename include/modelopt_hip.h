@@ -436,6 +436,17 @@ int mo_nf4_quantize(const void* x, int64_t n, int64_t block_size, int dtype, voi
  * (TQ/src/tensor_quant_gpu.cu:146-197) / NF4QTensor.dequantize (TQ/qtensor/nf4_tensor.py:157-201). */
 int mo_nf4_dequantize(const uint8_t* packed, int64_t nbytes, int64_t block_size,
                       const void* scales, void* y, int dtype, void* stream);
+/* Double quantisation of the block scales (qtensor/nf4_tensor.py:101-128) behind their mean: scales
+ * [rows, width] of type dtype, mean one element of it; b = T(s - mean), factor[row] =
+ * T(T(1 / max|b|) * bound), q = clamp(round(T(b * factor))) as int8 (0 for NaN); 1 <= bound <= 127. */
+int mo_nf4_scales_quantize(const void* scales, int64_t rows, int64_t width, int dtype, const void* mean,
+                           int bound, int8_t* q, void* factor, void* stream);
+/* mo_nf4_dequantize with the scale of block b taken from its int8 form:
+ * T(T(scales[b] / factor[b / width]) + mean); MO_ERR_UNSUPPORTED (nothing launched) unless the block
+ * size is 8 times a power of two, nbytes a multiple of 4, y 16-byte and packed 4-byte aligned. */
+int mo_nf4_dequantize_double(const uint8_t* packed, int64_t nbytes, int64_t block_size, const int8_t* scales,
+                             int64_t width, const void* factor, const void* mean, void* y, int dtype,
+                             void* stream);
 
 /* codes[i] = (x[i] < 0) << 3 | ordinal of the E2M1 magnitude nearest to |x[i]| (0, .5, 1, 1.5, 2,
  * 3, 4, 6; ties to the even code, NaN and infinity give ordinal 7, -0.0 gives code 0): one byte

@@ -11,7 +11,7 @@
 // whether the upper one wins is monotone in v: for each pair of neighbours there is one
 // threshold t[j] with "upper wins <=> v > t[j]", and code = number of thresholds below v.
 // The thresholds depend on T (the differences are rounded to T) and are found on the host by
-// bisection on exactly the comparison above; the kernel does a four-step binary search.
+// bisection on exactly the comparison above; fp32 does a four-step binary search over them.
 #include "common.h"
 
 namespace mo {
@@ -154,92 +154,111 @@ __global__ __launch_bounds__(256) void nf4_quantize_tile_kernel(
     }
 }
 
-// Table form for the 16-bit dtypes and large inputs.  The scaled value v is itself a 16-bit value
-// with |v| <= 1, so its code can be read from a table indexed by its bit pattern: 0x3F81
-// magnitudes for bf16 (0 .. 1.0), 0x3C01 for fp16, times two signs -- under 32 KiB of one-byte
-// codes.  A small kernel fills the table in device memory from the same thresholds (so the two
-// forms agree by construction); a workgroup copies it to LDS once and then converts
-// kNf4LutTiles tiles, which replaces the 19-instruction search per element by one LDS read.
-// Chunks whose block abs-max is zero, tiny or not finite take the threshold search.
-constexpr int kNf4LutBytes = 32768;
-constexpr int kNf4LutTiles = 8;
-template <int DT> struct Nf4Lut;
-template <> struct Nf4Lut<MO_BF16> { static constexpr int half = 0x3F81, slot = 0; };
-template <> struct Nf4Lut<MO_F16> { static constexpr int half = 0x3C01, slot = 1; };
-
-__device__ __align__(16) uint8_t g_nf4_lut[2][kNf4LutBytes];
+// The 16-bit dtypes.  The code of x under block abs-max a is the number of boundaries m[j] below x / a
+// (at m[j] itself where the tie rounds to the upper side), m[j] the point between two neighbours of
+// type T where the comparison above tips: 9 significant bits (bf16) or 12 (fp16).  m[j] * a then fits
+// fp32 exactly, so the side of x is the sign of x - m[j] * a, one FMA without an error in its sign;
+// and x / a is either m[j] or at least 2^-23 of it away, so the rounding of the quotient to fp32 never
+// crosses a boundary.  Which boundary to ask follows from x / a to within 1/32: a bucket of 1/16 holds one
+// boundary at most (they are 0.08 apart), and an approximate quotient is enough since neighbouring buckets
+// both hold a boundary near their common edge.  Seven vector instructions and one conflict-free LDS
+// read of 8 bytes an element.  14336 x 4096 bf16: 25.7 us (5.7 TB/s); with the code
+// of every 16-bit quotient in a 32 KB LDS table, an exact quotient and its rounding an element, 40.7 us.
+constexpr int kNf4Buckets = 33;   // round(16 * x / a) + 16
+struct Nf4Bucket { float m; uint32_t edge; };
+struct Nf4Buckets { Nf4Bucket b[kNf4Buckets]; };
 
 template <int DT>
-__global__ __launch_bounds__(256) void nf4_build_lut_kernel(Nf4Thresholds thresholds) {
-    const Nf4Regs th = nf4_regs(thresholds);
-    constexpr int half = Nf4Lut<DT>::half;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= kNf4LutBytes) return;
-    uint32_t code = 0;
-    if (e < 2 * half) {
-        const uint32_t sign = e >= half ? 1u : 0u;
-        const uint32_t bits = (uint32_t)(e - (int)sign * half) | (sign << 15);
-        const float v = DT == MO_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
-        code = nf4_code(v, th);
-    }
-    g_nf4_lut[Nf4Lut<DT>::slot][e] = (uint8_t)code;
+__device__ __forceinline__ uint32_t chunk_max_bits(const RawChunk<DT>& r) {
+    uint32_t t = pk_max_u16(pk_max_u16(r.a.x & 0x7FFF7FFFu, r.a.y & 0x7FFF7FFFu),
+                            pk_max_u16(r.a.z & 0x7FFF7FFFu, r.a.w & 0x7FFF7FFFu));
+    t = (t & 0xFFFFu) > (t >> 16) ? (t & 0xFFFFu) : (t >> 16);
+    return DT == MO_BF16 ? t << 16 : f2u(f16_bits_to_f32(t));
 }
 
 template <int DT>
-__global__ __launch_bounds__(256) void nf4_quantize_lut_kernel(
-    const void* __restrict__ x, int64_t chunks, int lanes_per_block, int shift,
-    Nf4Thresholds thresholds, void* __restrict__ scales, uint32_t* __restrict__ packed) {
-    __shared__ __align__(16) uint8_t lut[kNf4LutBytes];
-    constexpr int half = Nf4Lut<DT>::half;
-    {
-        const u32x4* src = (const u32x4*)g_nf4_lut[Nf4Lut<DT>::slot];
-        u32x4* dst = (u32x4*)lut;
+__global__ __launch_bounds__(256) void nf4_quantize_buckets_kernel(
+    const void* __restrict__ x, int64_t chunks, int lanes_per_block, int shift, Nf4Thresholds thresholds,
+    Nf4Buckets buckets, void* __restrict__ scales, uint32_t* __restrict__ packed) {
+    __shared__ Nf4Bucket tab[kNf4Buckets];
+    const int64_t c0 = (int64_t)blockIdx.x * kNf4TileChunks + threadIdx.x;
+    RawChunk<DT> raw[4];
 #pragma unroll
-        for (int i = 0; i < kNf4LutBytes / 16 / 256; ++i) dst[threadIdx.x + i * 256] = src[threadIdx.x + i * 256];
+    for (int u = 0; u < 4; ++u) {
+        const int64_t c = c0 + u * 256;
+        zero_raw<DT>(raw[u]);
+        if (c < chunks) load_raw<DT>(x, c << 3, raw[u]);
     }
+    if (threadIdx.x < kNf4Buckets) tab[threadIdx.x] = buckets.b[threadIdx.x];
     __syncthreads();
-    const Nf4Regs th = nf4_regs(thresholds);
-    for (int t = 0; t < kNf4LutTiles; ++t) {
-        const int64_t c0 = ((int64_t)blockIdx.x * kNf4LutTiles + t) * kNf4TileChunks + threadIdx.x;
-        if (c0 - threadIdx.x >= chunks) break;  // uniform: the whole tile is past the end
-        RawChunk<DT> raw[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int64_t c = c0 + u * 256;
-            zero_raw<DT>(raw[u]);
-            if (c < chunks) load_raw<DT>(x, c << 3, raw[u]);
-        }
+    for (int u = 0; u < 4; ++u) {
+        const int64_t c = c0 + u * 256;
+        float v[8];
+        unpack_raw<DT>(raw[u], v);
+        // chunks is a multiple of lanes_per_block, so the lanes of a block are all in or all out
+        const float amax = u2f(group_max_u32(chunk_max_bits<DT>(raw[u]), shift));
+        if (c >= chunks) continue;
+        if ((threadIdx.x & (lanes_per_block - 1)) == 0) store_elem<DT>(scales, c >> shift, amax);
+        uint32_t w = 0;
+        if (mid_range(amax)) {
+            const float r16 = 16.0f / amax;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int64_t c = c0 + u * 256;
-            float v[8];
-            unpack_raw<DT>(raw[u], v);
-            uint32_t m = 0;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t a = f2u(v[j]) & 0x7FFFFFFFu;
-                m = a > m ? a : m;
+            for (int i = 0; i < 8; ++i) {
+                const int j = i ^ 1;   // even element of a pair in the high nibble of its byte
+                // the rounding of the sum leaves the bucket number in the low mantissa bits
+                const uint32_t k = f2u(__builtin_fmaf(v[j], r16, 12582912.0f + 16.0f)) - 0x4B400000u;
+                const Nf4Bucket e = tab[k];
+                const float d = __builtin_fmaf(-e.m, amax, v[j]);
+                // the sign of the tiny edge says which side d == 0 is on, its low bits are the code below
+                const uint32_t code = e.edge + (d > u2f(e.edge) ? 1u : 0u);
+                w = __builtin_amdgcn_alignbit(code, w, 4);
             }
-            m = group_max_u32(m, shift);
-            if (c >= chunks) continue;
-            const float amax = u2f(m);
-            if ((threadIdx.x & (lanes_per_block - 1)) == 0) store_elem<DT>(scales, c >> shift, amax);
-            uint32_t w = 0;
-            if (mid_range(amax)) {
-                const float r = 1.0f / amax;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float q = exact_quotient(v[j], amax, r);
-                    const uint32_t bits = DT == MO_BF16 ? f32_to_bf16_bits(q) : f32_to_f16_bits(q);
-                    const uint32_t entry = (bits & 0x7FFFu) + ((bits >> 15) & 1u) * (uint32_t)half;
-                    w |= (uint32_t)lut[entry] << (4 * (j ^ 1));
-                }
-            } else {
-                w = nf4_codes8<DT>(v, amax, th);
-            }
-            __builtin_nontemporal_store(w, packed + c);
+        } else {
+            keep_branch();
+            w = nf4_codes8<DT>(v, amax, nf4_regs(thresholds));   // zero, tiny or not finite
         }
+        __builtin_nontemporal_store(w, packed + c);
     }
+}
+
+// Double-quantised scales, one wavefront per scale block: everything behind the mean, with every
+// intermediate rounded to the type of the scales as the tensor expression rounds it
+// (T(s - mean), abs-max, T(T(1 / amax) * bound), T(product), round, clamp).  Nine launches of a
+// few microseconds each as tensor operations (37 us with their gaps for 3584 x 256 bf16), 5.2 us here.
+template <int DT>
+__global__ __launch_bounds__(256) void nf4_scales_quantize_kernel(const void* __restrict__ scales, int64_t rows,
+                                                                  int width, const void* __restrict__ mean,
+                                                                  float bound, int8_t* __restrict__ q,
+                                                                  void* __restrict__ factor) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int lane = threadIdx.x & 63;
+    const float z = load_elem<DT>(mean, 0);
+    const int64_t base = row * width;
+    uint32_t m = 0;
+    for (int i = lane; i < width; i += 64) {
+        const uint32_t t = f2u(nf4_round_via<DT>(load_elem<DT>(scales, base + i) - z)) & 0x7FFFFFFFu;
+        m = t > m ? t : m;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t t = __shfl_xor(m, o, 64);
+        m = t > m ? t : m;
+    }
+    const float f = nf4_round_via<DT>(nf4_round_via<DT>(1.0f / u2f(m)) * bound);
+    if (lane == 0) store_elem<DT>(factor, row, f);
+    for (int i = lane; i < width; i += 64) {
+        const float b = nf4_round_via<DT>(load_elem<DT>(scales, base + i) - z);
+        float v = __builtin_rintf(nf4_round_via<DT>(b * f));
+        v = v < -bound ? -bound : (v > bound ? bound : v);
+        q[base + i] = v == v ? (int8_t)(int)v : (int8_t)0;
+    }
+}
+
+// T(T(q / factor) + mean): the scale of a block from its int8 form
+template <int DT>
+__device__ __forceinline__ float nf4_scale_of(int8_t q, float factor, float mean) {
+    return nf4_round_via<DT>(nf4_round_via<DT>((float)q / factor) + mean);
 }
 
 // y[2i] = T(table[byte >> 4] * f32(scale[block])), y[2i + 1] = T(table[byte & 15] * ...)
@@ -257,25 +276,37 @@ __global__ __launch_bounds__(256) void nf4_dequantize_kernel(const uint8_t* __re
     }
 }
 
-template <int DT>
+// DOUBLE: int8 scales, decoded on the way (one division per 8 elements): `width` of them share a factor.
+// 14336 x 4096 bf16 in blocks of 64: 29.6 us, 28.2 with decoded scales; decoding them first was a division
+// and a sum as tensor operations, 12 us and two launches.
+template <int DT, bool DOUBLE>
 __global__ __launch_bounds__(256) void nf4_dequantize_tile_kernel(
     const uint32_t* __restrict__ packed, int64_t chunks, int shift,
-    const void* __restrict__ scales, void* __restrict__ y) {
+    const void* __restrict__ scales, uint32_t width, const void* __restrict__ factor,
+    const void* __restrict__ mean, void* __restrict__ y) {
     __shared__ float table[16];
     if (threadIdx.x < 16) table[threadIdx.x] = kNf4Table[threadIdx.x];
     __syncthreads();
     const int64_t c0 = (int64_t)blockIdx.x * kNf4TileChunks + threadIdx.x;
     uint32_t w[4];
+    float sc[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-        const int64_t c = c0 + u * 256;
-        w[u] = c < chunks ? __builtin_nontemporal_load(packed + c) : 0u;
+        int64_t c = c0 + u * 256;
+        c = c < chunks ? c : chunks - 1;
+        w[u] = __builtin_nontemporal_load(packed + c);
+        const int64_t b = c >> shift;
+        if constexpr (DOUBLE)
+            sc[u] = nf4_scale_of<DT>(((const int8_t*)scales)[b], load_elem<DT>(factor, (uint32_t)b / width),
+                                     load_elem<DT>(mean, 0));
+        else
+            sc[u] = load_elem<DT>(scales, b);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int64_t c = c0 + u * 256;
         if (c >= chunks) continue;
-        const float s = load_elem<DT>(scales, c >> shift);
+        const float s = sc[u];
         float v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = table[(w[u] >> (4 * (j ^ 1))) & 0xFu] * s;
@@ -342,6 +373,48 @@ static Nf4Thresholds nf4_thresholds(int dtype) {
     return th;
 }
 
+// The buckets of a 16-bit type from its thresholds.  t[j] is the largest fp32 value on the lower side: the
+// boundary itself when that side has the tie, the value just below it otherwise.
+static Nf4Buckets nf4_buckets(int dtype, const Nf4Thresholds& th) {
+    const uint32_t rest = dtype == MO_BF16 ? 0x7FFFu : 0xFFFu;   // mantissa bits below a boundary's last one
+    float m[15];
+    bool upper_has_tie[15];
+    for (int j = 0; j < 15; ++j) {
+        uint32_t u;
+        __builtin_memcpy(&u, &th.t[j], 4);
+        upper_has_tie[j] = (u & rest) != 0;
+        m[j] = upper_has_tie[j] ? from_key(ordered_key(th.t[j]) + 1) : th.t[j];
+    }
+    Nf4Buckets out;
+    for (int i = 0; i < kNf4Buckets; ++i) {
+        const double lo = (i - 16.5) / 16.0 - 1e-4, hi = (i - 15.5) / 16.0 + 1e-4;
+        uint32_t below = 0;
+        while (below < 15 && m[below] < lo) ++below;
+        const bool inside = below < 15 && m[below] <= hi;
+        out.b[i].m = inside ? m[below] : 2.0f;   // x - 2 * amax is negative: the code below it stands
+        // +-2^-120: far below any difference of two values of the type within the range of the buckets
+        out.b[i].edge = (inside && upper_has_tie[below] ? 0x83800000u : 0x03800000u) | below;
+    }
+    return out;
+}
+
+struct Nf4Tables {
+    Nf4Thresholds th;
+    Nf4Buckets buckets;
+};
+
+// built once per type: a function-local constant, initialised under the language's own lock
+static const Nf4Tables& nf4_tables(int dtype) {
+    static const auto make = [](int d) {
+        Nf4Tables t;
+        t.th = nf4_thresholds(d);
+        t.buckets = d == MO_F32 ? Nf4Buckets{} : nf4_buckets(d, t.th);
+        return t;
+    };
+    static const Nf4Tables tables[3] = {make(MO_F32), make(MO_F16), make(MO_BF16)};
+    return tables[dtype];
+}
+
 static inline unsigned nf4_blocks_for(int64_t items) {
     int64_t b = (items + 255) / 256;
     if (b < 1) b = 1;
@@ -367,30 +440,22 @@ extern "C" int mo_nf4_quantize(const void* x, int64_t n, int64_t block_size, int
     if (!x || !scales || !packed) return MO_ERR_ARG;
     const int64_t nblocks = (n + block_size - 1) / block_size;
     hipStream_t s = (hipStream_t)stream;
-    const mo::Nf4Thresholds th = mo::nf4_thresholds(dtype);
+    const mo::Nf4Tables& tables = mo::nf4_tables(dtype);
+    const mo::Nf4Thresholds& th = tables.th;
     int shift = -1;  // block_size == 8 << shift
     for (int k = 0; k <= 6; ++k)
         if (block_size == (8ll << k)) shift = k;
     const int64_t tiles = (n / 8 + mo::kNf4TileChunks - 1) / mo::kNf4TileChunks;
     if (shift >= 0 && n % block_size == 0 && (((uintptr_t)x & 15u) == 0) &&
         (((uintptr_t)packed & 3u) == 0) && tiles <= 0x7FFFFFFF) {
-        if (dtype != MO_F32 && tiles >= 64 * mo::kNf4LutTiles) {  // large 16-bit input: table form
-            const unsigned g = (unsigned)((tiles + mo::kNf4LutTiles - 1) / mo::kNf4LutTiles);
-            if (dtype == MO_BF16) {
-                mo::nf4_build_lut_kernel<MO_BF16><<<mo::kNf4LutBytes / 256, 256, 0, s>>>(th);
-                mo::nf4_quantize_lut_kernel<MO_BF16><<<g, 256, 0, s>>>(
-                    x, n / 8, 1 << shift, shift, th, scales, (uint32_t*)packed);
-            } else {
-                mo::nf4_build_lut_kernel<MO_F16><<<mo::kNf4LutBytes / 256, 256, 0, s>>>(th);
-                mo::nf4_quantize_lut_kernel<MO_F16><<<g, 256, 0, s>>>(
-                    x, n / 8, 1 << shift, shift, th, scales, (uint32_t*)packed);
-            }
-            return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
-        }
 #define CALL(DT)                                                                    \
-    mo::nf4_quantize_tile_kernel<DT><<<(unsigned)tiles, 256, 0, s>>>(               \
-        x, n / 8, 1 << shift, shift, th, scales, (uint32_t*)packed)
-        DISPATCH_DT(dtype, CALL)
+    mo::nf4_quantize_buckets_kernel<DT><<<(unsigned)tiles, 256, 0, s>>>(            \
+        x, n / 8, 1 << shift, shift, th, tables.buckets, scales, (uint32_t*)packed)
+        if (dtype == MO_BF16) CALL(MO_BF16);
+        else if (dtype == MO_F16) CALL(MO_F16);
+        else
+            mo::nf4_quantize_tile_kernel<MO_F32><<<(unsigned)tiles, 256, 0, s>>>(
+                x, n / 8, 1 << shift, shift, th, scales, (uint32_t*)packed);
 #undef CALL
         return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
     }
@@ -401,8 +466,24 @@ extern "C" int mo_nf4_quantize(const void* x, int64_t n, int64_t block_size, int
     return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
 }
 
-extern "C" int mo_nf4_dequantize(const uint8_t* packed, int64_t nbytes, int64_t block_size,
-                                 const void* scales, void* y, int dtype, void* stream) {
+extern "C" int mo_nf4_scales_quantize(const void* scales, int64_t rows, int64_t width, int dtype,
+                                      const void* mean, int bound, int8_t* q, void* factor, void* stream) {
+    if (rows < 0 || width < 0 || bound < 1 || bound > 127) return MO_ERR_ARG;
+    if (dtype != MO_F32 && dtype != MO_F16 && dtype != MO_BF16) return MO_ERR_DTYPE;
+    if (rows == 0 || width == 0) return MO_OK;
+    if (!scales || !mean || !q || !factor) return MO_ERR_ARG;
+    if (width > 0x3FFFFFFF || rows > 0x7FFFFFFFll * 4) return MO_ERR_UNSUPPORTED;
+    const unsigned g = (unsigned)((rows + 3) / 4);
+#define CALL(DT)                                                                    \
+    mo::nf4_scales_quantize_kernel<DT><<<g, 256, 0, (hipStream_t)stream>>>(         \
+        scales, rows, (int)width, mean, (float)bound, q, factor)
+    DISPATCH_DT(dtype, CALL)
+#undef CALL
+    return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
+}
+
+static int nf4_dequantize(const uint8_t* packed, int64_t nbytes, int64_t block_size, const void* scales,
+                          int64_t width, const void* factor, const void* mean, void* y, int dtype, void* stream) {
     if (nbytes < 0 || block_size <= 0 || (block_size & 1)) return MO_ERR_ARG;
     if (dtype != MO_F32 && dtype != MO_F16 && dtype != MO_BF16) return MO_ERR_DTYPE;
     if (nbytes == 0) return MO_OK;
@@ -414,16 +495,34 @@ extern "C" int mo_nf4_dequantize(const uint8_t* packed, int64_t nbytes, int64_t 
     const int64_t tiles = (nbytes / 4 + mo::kNf4TileChunks - 1) / mo::kNf4TileChunks;
     if (shift >= 0 && nbytes % 4 == 0 && (((uintptr_t)y & 15u) == 0) &&
         (((uintptr_t)packed & 3u) == 0) && tiles <= 0x7FFFFFFF) {
-#define CALL(DT)                                                                    \
-    mo::nf4_dequantize_tile_kernel<DT><<<(unsigned)tiles, 256, 0, s>>>(             \
-        (const uint32_t*)packed, nbytes / 4, shift, scales, y)
+        if (factor && ((nbytes / 4) >> shift) > 0xFFFFFFFFll) return MO_ERR_UNSUPPORTED;
+#define CALL(DT)                                                                           \
+    if (factor)                                                                            \
+        mo::nf4_dequantize_tile_kernel<DT, true><<<(unsigned)tiles, 256, 0, s>>>(          \
+            (const uint32_t*)packed, nbytes / 4, shift, scales, (uint32_t)width, factor, mean, y); \
+    else                                                                                   \
+        mo::nf4_dequantize_tile_kernel<DT, false><<<(unsigned)tiles, 256, 0, s>>>(         \
+            (const uint32_t*)packed, nbytes / 4, shift, scales, 1u, nullptr, nullptr, y)
         DISPATCH_DT(dtype, CALL)
 #undef CALL
         return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
     }
+    if (factor) return MO_ERR_UNSUPPORTED;
     const unsigned g = mo::nf4_blocks_for(nbytes);
 #define CALL(DT) mo::nf4_dequantize_kernel<DT><<<g, 256, 0, s>>>(packed, nbytes, block_size, scales, y)
     DISPATCH_DT(dtype, CALL)
 #undef CALL
     return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
+}
+
+extern "C" int mo_nf4_dequantize(const uint8_t* packed, int64_t nbytes, int64_t block_size,
+                                 const void* scales, void* y, int dtype, void* stream) {
+    return nf4_dequantize(packed, nbytes, block_size, scales, 1, nullptr, nullptr, y, dtype, stream);
+}
+
+extern "C" int mo_nf4_dequantize_double(const uint8_t* packed, int64_t nbytes, int64_t block_size,
+                                        const int8_t* scales, int64_t width, const void* factor,
+                                        const void* mean, void* y, int dtype, void* stream) {
+    if (width < 1 || width > 0x7FFFFFFF || (nbytes > 0 && (!factor || !mean))) return MO_ERR_ARG;
+    return nf4_dequantize(packed, nbytes, block_size, scales, width, factor, mean, y, dtype, stream);
 }

@@ -64,6 +64,8 @@ SIGNATURES = {
     "mo_int4_pack_rows": [_P, _I64, _I64, _I64, _I64, _INT, _P, _P, _P],
     "mo_int4_pack_rows_via": [_P, _I64, _I64, _I64, _I64, _INT, _P, _INT, _P, _P],
     "mo_nf4_quantize": [_P, _I64, _I64, _INT, _P, _P, _P],
+    "mo_nf4_scales_quantize": [_P, _I64, _I64, _INT, _P, _INT, _P, _P, _P],
+    "mo_nf4_dequantize_double": [_P, _I64, _I64, _P, _I64, _P, _P, _P, _INT, _P],
     "mo_nf4_dequantize": [_P, _I64, _I64, _P, _P, _INT, _P],
     "mo_mul_cols": [_P, _I64, _I64, _INT, _P, _INT, _P, _P],
     "mo_scale_block_int_qdq": [_P, _I64, _I64, _INT, _P, _INT, _I64, _INT, _INT, _INT, _P, _P],
@@ -732,6 +734,36 @@ def nf4_dequantize(packed, scales, block_size):
     y = torch.empty(packed.numel() * 2, dtype=scales.dtype, device=packed.device)
     call("mo_nf4_dequantize", packed, _ptr(packed), packed.numel(), block_size, _ptr(scales),
          _ptr(y), dtype_code(scales.dtype), _stream(packed))
+    return y
+
+
+def nf4_scales_quantize(scales, mean, bound):
+    """Block scales [rows, width] less their ``mean`` (one element of the same dtype) to int8 per row:
+    (int8 [rows, width], ``bound / abs-max`` [rows] in the dtype of ``scales``)."""
+    _require_device(scales, mean)
+    rows, width = scales.shape
+    assert scales.is_contiguous() and mean.numel() == 1 and mean.dtype == scales.dtype
+    q = torch.empty((rows, width), dtype=torch.int8, device=scales.device)
+    factor = torch.empty(rows, dtype=scales.dtype, device=scales.device)
+    call("mo_nf4_scales_quantize", scales, _ptr(scales), rows, width, dtype_code(scales.dtype), _ptr(mean),
+         int(bound), _ptr(q), _ptr(factor), _stream(scales))
+    return q, factor
+
+
+def nf4_dequantize_double(packed, scales, factor, mean, block_size):
+    """``nf4_dequantize`` with int8 ``scales`` decoded on the way, in the dtype of ``factor`` and ``mean``;
+    None, with nothing launched, where the kernel has no such form."""
+    _require_device(packed, scales, factor, mean)
+    n, rows = packed.numel() * 2, factor.numel()
+    if (scales.dtype != torch.int8 or factor.dtype not in _DTYPES or mean.dtype != factor.dtype or mean.numel() != 1
+            or rows == 0 or scales.numel() % rows or scales.numel() * block_size < n
+            or block_size < 8 or block_size & (block_size - 1) or packed.numel() % 4 or packed.data_ptr() % 4
+            or n // block_size >> 31):
+        return None
+    assert packed.is_contiguous() and scales.is_contiguous() and factor.is_contiguous()
+    y = torch.empty(n, dtype=factor.dtype, device=packed.device)
+    call("mo_nf4_dequantize_double", packed, _ptr(packed), packed.numel(), block_size, _ptr(scales),
+         scales.numel() // rows, _ptr(factor), _ptr(mean), _ptr(y), dtype_code(factor.dtype), _stream(packed))
     return y
 
 

@@ -46,6 +46,10 @@ class NF4QTensor(BaseQuantizedTensor):
         bound = 2 ** (num_scale_bits - 1) - 1
         block_scales = scales.view(-1, scale_block_size)
         zero_point = block_scales.mean()
+        if (scales.is_cuda and scales.dtype in _hip._DTYPES and 1 <= bound <= 127 and scales.numel()
+                and not (torch.is_grad_enabled() and scales.requires_grad)):
+            q, factor = _hip.nf4_scales_quantize(block_scales.contiguous(), zero_point, bound)
+            return q, factor, zero_point
         block_scales = block_scales - zero_point
         factor = bound / reduce_amax(block_scales, -1)
         q = block_scales * factor.expand(block_scales.shape[0], scale_block_size)
@@ -58,9 +62,13 @@ class NF4QTensor(BaseQuantizedTensor):
         block = kwarg["block_sizes"][-1]
         data = self._quantized_data.contiguous().view(-1)
         dev = data.device
-        n_blocks = data.numel() * 2 // block
-        scales = _dequantize_scalers(kwarg["scale"].to(dev), kwarg["double_scale"].to(dev),
-                                     kwarg["scale_zeros"].to(dev), dtype)[:n_blocks].contiguous()
-        flat = _hip.nf4_dequantize(data, scales, block)
+        scale, double_scale, zeros = (kwarg[k].to(dev) for k in ("scale", "double_scale", "scale_zeros"))
+        flat = None
+        if double_scale.dtype == zeros.dtype == dtype and dev.type == "cuda":
+            flat = _hip.nf4_dequantize_double(data, scale.contiguous(), double_scale.contiguous(), zeros, block)
+        if flat is None:
+            n_blocks = data.numel() * 2 // block
+            scales = _dequantize_scalers(scale, double_scale, zeros, dtype)[:n_blocks].contiguous()
+            flat = _hip.nf4_dequantize(data, scales, block)
         n = math.prod(self.metadata["shape"])
         return flat[:n].reshape(self.metadata["shape"]).to(dtype)

@@ -218,3 +218,46 @@ def test_full_size_weight_roundtrip_error():
     rows = slice(5000, 5064)
     want, _ = nf4.nf4_quantize(x[rows].cpu(), 64, 1)
     assert torch.equal(packed.view(14336, -1)[rows].cpu().view(-1), want)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,width", [(1, 1), (1, 256), (5, 3), (7, 64), (9, 300)])
+def test_double_quantised_scales_equal_the_tensor_expressions(dtype, rows, width):
+    """One launch for the int8 scales and one for decoding with them, bit for bit what the tensor
+    operations give; a row of equal scales (0 / 0) and a row with an infinity among them."""
+    g = torch.Generator().manual_seed(rows * width)
+    scales = (torch.rand(rows, width, generator=g) + 0.01).to(dtype)
+    if rows > 5:
+        scales[2] = 0.5
+        scales[4, width // 2] = float("inf")
+    mean = torch.tensor(0.5, dtype=dtype) if rows > 5 else scales.mean()
+    scales, mean = scales.to(DEV), mean.to(DEV)
+    q, factor = _hip.nf4_scales_quantize(scales, mean, 127)
+    centred = scales - mean
+    want_factor = 127 / centred.abs().amax(-1, keepdim=True)
+    want = (centred * want_factor).round().nan_to_num(nan=0.0).clamp(-127, 127).to(torch.int8)
+    assert_bits_equal(factor.cpu(), want_factor.flatten().cpu())
+    assert torch.equal(q, want)
+    packed = torch.randint(0, 256, (rows * width * 4,), generator=g, dtype=torch.uint8).to(DEV)
+    for block in (8, 16):
+        data = packed[:rows * width * block // 2] if block == 8 else packed.repeat(2)
+        decoded = ((q / want_factor).to(dtype) + mean).flatten()
+        got = _hip.nf4_dequantize_double(data, q, factor, mean, block)
+        assert_bits_equal(got.cpu(), _hip.nf4_dequantize(data, decoded, block).cpu())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_quantize_every_block_scale(dtype):
+    """Each significand of the block abs-max with values around all decision points."""
+    n = 128 if dtype == torch.bfloat16 else 1024
+    amax = (1 + torch.arange(n) / n).view(-1, 1)
+    t = nf4.NF4_TABLE.float()
+    mid = (t[:-1] + t[1:]) / 2
+    step = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    v = torch.cat([mid * (1 + i * step / 2) for i in range(-4, 5)])
+    x = torch.zeros(n, 192)
+    x[:, 0:1] = amax
+    x[:, 1:1 + v.numel()] = v * amax
+    _check_quantize(x.to(dtype).flatten(), 192)
+    x = torch.cat([amax, v.repeat(n, 1) * amax, torch.zeros(n, 256 - 1 - v.numel())], 1)
+    _check_quantize(x.to(dtype).flatten(), 256)
