@@ -74,6 +74,14 @@ enum { MO_ABSMAX_REREAD = 1u };
 int mo_absmax_hinted(const void* x, int64_t outer, int64_t axis, int64_t inner, int dtype,
                      float* acc, unsigned hints, void* stream);
 
+/* The abs-max of one tensor as a value of out_dtype at `out` (rounded to it), n > 0, x 16-byte aligned
+ * (MO_ERR_UNSUPPORTED otherwise): mo_absmax without an accumulator to clear first.  hints as above.
+ * parts: MO_AMAX_PARTS_BYTES of scratch that no other call in flight uses; nothing in it need be set. */
+#define MO_AMAX_PARTS 1024
+#define MO_AMAX_PARTS_BYTES (4 * MO_AMAX_PARTS + 16)
+int mo_absmax_tensor(const void* x, int64_t n, int dtype, unsigned hints, void* out, int out_dtype, void* parts,
+                     void* stream);
+
 /* Two per-tensor mo_absmax calls (x0 of n0 elements into acc0, x1 of n1 into acc1, one dtype) in
  * one launch: the key and the value states of an attention layer reach their quantizers
  * together (k_bmm_quantizer / v_bmm_quantizer, TQ/plugins/huggingface.py:52-69, each a
@@ -230,6 +238,13 @@ enum mo_row_kind { MO_ROW_INT = 0, MO_ROW_FP8 = 1, MO_ROW_NVFP4 = 2, MO_ROW_MX =
 int mo_row_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* pre_scale,
                int kind, int p0, int p1, int p2, const void* amax, int amax_dtype, void* stream);
 
+/* Fake quantisation with the abs-max of x itself (a quantizer without a calibrated amax,
+ * TensorQuantizer._get_amax then _fake_quantize, TQ/nn/modules/tensor_quantizer.py:505-514, 604-640):
+ * kind MO_ROW_INT, MO_ROW_FP8 or MO_ROW_NVFP4 with p0 .. p2 as above; x and y 16-byte aligned, y not x;
+ * parts as for mo_absmax_tensor. */
+int mo_dynamic_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, int kind, int p0, int p1, int p2,
+                   void* parts, void* stream);
+
 /* ------------------------------------------------------------------ real quantize + pack */
 
 /* Squared fake-quantisation error for n_cand candidate amax values in one pass over x viewed
@@ -359,6 +374,11 @@ int mo_nvfp4_quantize_fused(const void* x, int64_t rows, int64_t k, int dtype, i
 int mo_fused_amax_qdq(const void* x, void* y, int64_t n, int dtype, int kind, int num_bits,
                       int is_unsigned, int narrow_range, int saturate, float* amax_out,
                       void* workspace, int64_t spin_limit, void* stream);
+
+/* mo_nvfp4_quantize with the abs-max of x itself (x 16-byte aligned, MO_ERR_UNSUPPORTED otherwise);
+ * parts as for mo_absmax_tensor. */
+int mo_nvfp4_quantize_dynamic(const void* x, int64_t rows, int64_t k, int dtype, int block_size, void* parts,
+                              uint8_t* packed, uint8_t* wsf_out, float* wsf2_out, int flags, void* stream);
 
 /* NVFP4 unpack + rescale.  Replaces NVFP4QTensor.dequantize (TQ/qtensor/nvfp4_tensor.py
  * :234-297) and fp4_dequantize (TQ/triton/fp4_kernel.py:307):

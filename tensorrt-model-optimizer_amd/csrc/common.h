@@ -330,6 +330,25 @@ __device__ __forceinline__ float load_scalar(const void* p, int dtype, int64_t i
     return bf16_bits_to_f32(((const uint16_t*)p)[i]);
 }
 
+// The abs-max of a tensor as an earlier launch of the same call left it: the maxima of `n` parts (bit
+// patterns of non-negative floats), handed to a kernel as an amax of "type" kAmaxParts + n.  No
+// accumulator to clear first, no atomics that the workgroups of the first wave all meet at, and no
+// launch to fold the parts: every workgroup of the consumer folds them (at most 4 KB from L2).
+constexpr int kAmaxParts = 16;   // above the values of mo_dtype
+constexpr int kMaxAmaxParts = MO_AMAX_PARTS;
+
+// The amax of a workgroup of 256 lanes, all of which call this; smem: 4 words.
+__device__ __forceinline__ float tensor_amax(const void* amax, int dtype, uint32_t* smem);
+
+// launches: parts of x (16-byte aligned), their fold to one value of out_dtype
+int launch_absmax_parts(const void* x, int64_t n, int dtype, bool keep, uint32_t* parts, int* nparts, hipStream_t s);
+int launch_fold_parts(const uint32_t* parts, int nparts, void* out, int out_dtype, hipStream_t s);
+// mo_nvfp4_qdq and mo_row_qdq behind their checks, amax_dtype a type or parts
+int nvfp4_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* amax, int amax_dtype,
+              int block_size, int mode, hipStream_t s);
+int row_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* pre, int kind, int p0, int p1,
+            int p2, const void* amax, int amax_dtype, hipStream_t s);
+
 // ---------------------------------------------------------------- E4M3 (OCP e4m3fn)
 
 // gfx950's FP8 converts implement OCP E4M3: v_cvt_pk_fp8_f32 rounds to nearest even, keeps
@@ -505,6 +524,25 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t* smem) {
     return v;
 }
 
+
+__device__ __forceinline__ float tensor_amax(const void* amax, int dtype, uint32_t* smem) {
+    if (dtype < kAmaxParts) return load_scalar(amax, dtype, 0);
+    const uint32_t* parts = (const uint32_t*)amax;
+    const int n = dtype - kAmaxParts;
+    uint32_t m = 0;
+    for (int i = threadIdx.x; i < n; i += 1024) {
+        uint32_t t[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) t[u] = parts[i + u * 256 < n ? i + u * 256 : n - 1];   // the last one again past the end
+#pragma unroll
+        for (int u = 0; u < 4; ++u) m = t[u] > m ? t[u] : m;
+    }
+    m = wave_max_u32(m);
+    if ((threadIdx.x & (kWave - 1)) == 0) smem[threadIdx.x / kWave] = m;
+    __syncthreads();
+    const uint32_t a = smem[0] > smem[1] ? smem[0] : smem[1], b = smem[2] > smem[3] ? smem[2] : smem[3];
+    return u2f(a > b ? a : b);
+}
 
 // ---------------------------------------------------------------- one-launch amax -> quantize
 // The fused kernels read their share of the tensor into registers, agree on the global abs-max

@@ -96,7 +96,8 @@ __global__ __launch_bounds__(256) void row_qdq_kernel(const void* __restrict__ x
                                                       uint32_t chunks, int64_t k, RowDiv div,
                                                       const void* __restrict__ pre,
                                                       const void* __restrict__ amax, int amax_dtype, F f) {
-    f.start(amax ? load_scalar(amax, amax_dtype, 0) : 0.0f);
+    __shared__ uint32_t smem[4];
+    f.start(amax ? tensor_amax(amax, amax_dtype, smem) : 0.0f);
     const uint32_t c0 = blockIdx.x * kRowTileChunks + threadIdx.x;
     RawChunk<DT> raw[kRowU], sc[kRowU];
     uint32_t row[kRowU], col[kRowU];
@@ -180,6 +181,19 @@ static int dispatch_row(const void* x, void* y, int64_t rows, int64_t k, const v
     return MO_OK;
 }
 
+// amax_dtype: a type, or parts (kAmaxParts + their number)
+int row_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* pre, int kind, int p0, int p1,
+            int p2, const void* amax, int amax_dtype, hipStream_t s) {
+    int rc;
+    switch (dtype) {
+        case MO_F32: rc = dispatch_row<MO_F32>(x, y, rows, k, pre, kind, p0, p1, p2, amax, amax_dtype, s); break;
+        case MO_F16: rc = dispatch_row<MO_F16>(x, y, rows, k, pre, kind, p0, p1, p2, amax, amax_dtype, s); break;
+        default: rc = dispatch_row<MO_BF16>(x, y, rows, k, pre, kind, p0, p1, p2, amax, amax_dtype, s); break;
+    }
+    if (rc != MO_OK) return rc;
+    return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
+}
+
 }  // namespace mo
 
 extern "C" int mo_row_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* pre_scale,
@@ -202,13 +216,5 @@ extern "C" int mo_row_qdq(const void* x, void* y, int64_t rows, int64_t k, int d
     if (!x || !y || (kind != MO_ROW_MX && !amax)) return MO_ERR_ARG;
     const uintptr_t need = dtype == MO_F32 ? 3u : 1u;
     if (((uintptr_t)x | (uintptr_t)y | (uintptr_t)pre_scale) & need) return MO_ERR_ARG;
-    hipStream_t s = (hipStream_t)stream;
-    int rc;
-    switch (dtype) {
-        case MO_F32: rc = mo::dispatch_row<MO_F32>(x, y, rows, k, pre_scale, kind, p0, p1, p2, amax, amax_dtype, s); break;
-        case MO_F16: rc = mo::dispatch_row<MO_F16>(x, y, rows, k, pre_scale, kind, p0, p1, p2, amax, amax_dtype, s); break;
-        default: rc = mo::dispatch_row<MO_BF16>(x, y, rows, k, pre_scale, kind, p0, p1, p2, amax, amax_dtype, s); break;
-    }
-    if (rc != MO_OK) return rc;
-    return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
+    return mo::row_qdq(x, y, rows, k, dtype, pre_scale, kind, p0, p1, p2, amax, amax_dtype, (hipStream_t)stream);
 }

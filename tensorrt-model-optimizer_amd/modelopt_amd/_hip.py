@@ -28,6 +28,9 @@ SIGNATURES = {
     "mo_error_string": [_INT],
     "mo_absmax": [_P, _I64, _I64, _I64, _INT, _P, _P],
     "mo_absmax_hinted": [_P, _I64, _I64, _I64, _INT, _P, ctypes.c_uint, _P],
+    "mo_absmax_tensor": [_P, _I64, _INT, ctypes.c_uint, _P, _INT, _P, _P],
+    "mo_dynamic_qdq": [_P, _P, _I64, _I64, _INT, _INT, _INT, _INT, _INT, _P, _P],
+    "mo_nvfp4_quantize_dynamic": [_P, _I64, _I64, _INT, _INT, _P, _P, _P, _P, _INT, _P],
     "mo_absmax_pair": [_P, _I64, _P, _P, _I64, _P, _INT, _P],
     "mo_value_ranges": [_P, _P, _P, _INT, _P, _I64, _P],
     "mo_awq_pick_scale": [_P, _I64, _P, _I64, _P, _P, _P, _P, _P, _INT, _P],
@@ -236,6 +239,27 @@ def absmax_into(x: torch.Tensor, acc: torch.Tensor, outer: int, axis: int, inner
     return acc
 
 
+AMAX_PARTS_BYTES = 4 * 1024 + 16   # MO_AMAX_PARTS_BYTES
+
+
+def _amax_parts(x):
+    """Scratch of one call: two threads may launch on one stream, so calls do not share it."""
+    return torch.empty(AMAX_PARTS_BYTES // 4, dtype=torch.int32, device=x.device)
+
+
+def absmax_tensor(x: torch.Tensor, out_dtype: torch.dtype, reread: bool = False):
+    """The abs-max of a contiguous tensor as a one-element tensor of ``out_dtype``, nothing to clear first;
+    None, with nothing launched, for an empty or unaligned tensor.  ``reread`` as in ``absmax_into``."""
+    _require_device(x)
+    if x.numel() == 0 or x.data_ptr() % 16 or x.dtype not in _DTYPES or out_dtype not in _DTYPES:
+        return None
+    assert x.is_contiguous()
+    out = torch.empty(1, dtype=out_dtype, device=x.device)
+    call("mo_absmax_tensor", x, _ptr(x), x.numel(), _DTYPES[x.dtype], MO_ABSMAX_REREAD if reread else 0, _ptr(out),
+         _DTYPES[out_dtype], _ptr(_amax_parts(x)), _stream(x))
+    return out
+
+
 def absmax_pair_into(x0: torch.Tensor, acc0: torch.Tensor, x1: torch.Tensor, acc1: torch.Tensor):
     """Per-tensor ``absmax_into`` of two dense tensors of one dtype (each into its own one-element
     accumulator) in one launch.  False, with nothing launched, when the pair is not covered."""
@@ -437,6 +461,20 @@ def row_qdq(x, pre_scale, kind, p0=0, p1=0, p2=0, amax=None):
     return y
 
 
+def dynamic_qdq(x, kind, p0=0, p1=0, p2=0):
+    """Fake quantisation with the abs-max of ``x`` itself (``kind`` and ``p0`` .. ``p2`` as in ``row_qdq``, no
+    MX formats) in two launches; None, with nothing launched, for an empty or unaligned tensor."""
+    _require_device(x)
+    if x.numel() == 0 or x.data_ptr() % 16 or x.dtype not in _DTYPES:
+        return None
+    assert x.is_contiguous()
+    k = x.shape[-1] if x.dim() else 1
+    y = torch.empty_like(x)
+    call("mo_dynamic_qdq", x, _ptr(x), _ptr(y), x.numel() // k, k, _DTYPES[x.dtype], kind, int(p0), int(p1), int(p2),
+         _ptr(_amax_parts(x)), _stream(x))
+    return y
+
+
 ELEM_FORMATS = ["E4M3", "E5M2", "INT8", "E0M3", "E1M2", "E3M0", "E2M1", "E3M2", "E2M3", "E8M0"]
 
 
@@ -514,6 +552,24 @@ def nvfp4_quantize(x, amax_f32, block_size=16, amax_is_wsf2=False, wsf_in=None, 
     call("mo_nvfp4_quantize", x, _ptr(x), rows, k, dtype_code(x.dtype), block_size,
          _ptr(amax_f32), int(amax_is_wsf2), _ptr(wsf_arg), _ptr(packed),
          None if wsf_in is not None else _ptr(wsf), _ptr(wsf2), int(flags), _stream(x))
+    return packed, wsf.view(torch.float8_e4m3fn), wsf2
+
+
+def nvfp4_quantize_dynamic(x, block_size=16, flags=0):
+    """``nvfp4_quantize`` with the abs-max of ``x`` itself, nothing to clear first; None, with nothing
+    launched, for an empty or unaligned tensor."""
+    _require_device(x)
+    if x.numel() == 0 or x.dim() == 0 or x.data_ptr() % 16 or x.dtype not in _DTYPES:
+        return None
+    assert x.is_contiguous()
+    k = x.shape[-1]
+    kp = -(-k // block_size) * block_size
+    lead = tuple(x.shape[:-1])
+    packed = torch.empty(lead + (kp // 2,), dtype=torch.uint8, device=x.device)
+    wsf = torch.empty(lead + (kp // block_size,), dtype=torch.uint8, device=x.device)
+    wsf2 = torch.empty((), dtype=torch.float32, device=x.device)
+    call("mo_nvfp4_quantize_dynamic", x, _ptr(x), x.numel() // k, k, _DTYPES[x.dtype], block_size,
+         _ptr(_amax_parts(x)), _ptr(packed), _ptr(wsf), _ptr(wsf2), int(flags), _stream(x))
     return packed, wsf.view(torch.float8_e4m3fn), wsf2
 
 

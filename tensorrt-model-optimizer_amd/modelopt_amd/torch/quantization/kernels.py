@@ -104,6 +104,15 @@ def absmax_accumulate(x: torch.Tensor, acc: torch.Tensor, layout, reread: bool =
     return _hip.absmax_into(x, acc, outer, axis, inner, reread=reread)
 
 
+def absmax_of(x: torch.Tensor, out_dtype: torch.dtype, reread: bool = False):
+    """The abs-max of all of ``x`` as one element of ``out_dtype``; None where ``_hip.absmax_tensor`` does not
+    apply (an accumulator and ``absmax_accumulate`` do)."""
+    if not x.is_contiguous():
+        flat = dense_flat_view(x)
+        x = flat if flat is not None else x.contiguous()
+    return _hip.absmax_tensor(x, out_dtype, reread=reread)
+
+
 def reduce_amax_gpu(x: torch.Tensor, reduce_dims, keepdims=True, reread: bool = False):
     """``reduce_amax`` on the device: abs-max over ``reduce_dims`` (None = all) in x.dtype."""
     nd = x.dim()
@@ -115,6 +124,10 @@ def reduce_amax_gpu(x: torch.Tensor, reduce_dims, keepdims=True, reread: bool = 
         out_shape = tuple(1 if d in red else x.shape[d] for d in range(nd)) if keepdims else tuple(
             x.shape[d] for d in keep)
     layout = amax_layout(tuple(x.shape), keep)
+    if layout is not None and layout[1] == 1 and x.is_cuda:
+        whole = absmax_of(x, x.dtype, reread=reread)
+        if whole is not None:
+            return whole.reshape(out_shape)
     src = x
     if layout is None and x.is_cuda and x.is_contiguous():
         # one abs-max per two-dimensional block of a matrix: a workgroup per block, no transposed copy

@@ -16,7 +16,7 @@ import torch.nn.functional as F
 from torch import nn
 from torch.nn.modules import module as _module_hooks
 
-from ... import calib, kernels, modes
+from ... import calib, kernels, modes, tensor_quant
 from ... import utils as quant_utils
 from ...config import QuantizerAttributeConfig
 from ...qtensor import (BaseQuantizedTensor, FP8QTensor, INT4QTensor, INT8QTensor, MXFP4QTensor,
@@ -440,10 +440,37 @@ class TensorQuantizer(nn.Module):
                                                self._narrow_range)
         return None if done is None else done[0]
 
+    def _dynamic_fake_quant(self, inputs):
+        """Fake quantisation with the abs-max of the input itself in two launches (the maxima of parts of
+        the tensor, folded by the launch that quantises): an accumulator would be filled, reduced into
+        by atomics and converted first.  For plain tensors that are not differentiated, traced or
+        transformed; None for all else."""
+        bs, bits = self._block_sizes, self._num_bits
+        if (hasattr(self, "_amax") or self._axis is not None or not inputs.is_cuda
+                or type(inputs) not in (torch.Tensor, nn.Parameter) or modes.strict_checks()
+                or (inputs.requires_grad and torch.is_grad_enabled())
+                or kernels.torch_is_intercepted()):
+            return None
+        if bs is None:
+            if type(bits) is int and 1 <= bits <= 24:
+                return kernels._hip.dynamic_qdq(inputs, kernels._hip.MO_ROW_INT, bits, bool(self._unsigned),
+                                                bool(self._narrow_range))
+            if bits == (4, 3):
+                # a per-tensor amax clamps unless "nan" is selected
+                return kernels._hip.dynamic_qdq(inputs, kernels._hip.MO_ROW_FP8,
+                                                get_fp8_overflow_behavior() != "nan")
+        elif (bs.get("type", "static") == "dynamic" and bits == (2, 1) and bs.get("scale_bits") == (4, 3)
+                and bs.get(-1) in (8, 16, 32)):
+            return kernels._hip.dynamic_qdq(inputs, kernels._hip.MO_ROW_NVFP4, bs[-1],
+                                            tensor_quant.NVFP4_FAKE_QUANT_MODE)
+        return None
+
     def _fake_quantize(self, inputs):
-        fused = self._fused_dynamic_per_tensor(inputs)
-        if fused is not None:
-            return fused
+        done = self._fused_dynamic_per_tensor(inputs)
+        if done is None:
+            done = self._dynamic_fake_quant(inputs)
+        if done is not None:
+            return done
         amax = None if self.is_mx_format else self._get_amax(inputs)
         bs = self.block_sizes
         if bs is not None and bs.get("type", "static") == "dynamic":

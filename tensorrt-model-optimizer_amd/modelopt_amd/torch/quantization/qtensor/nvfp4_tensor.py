@@ -146,6 +146,11 @@ class NVFP4QTensor(BaseQuantizedTensor):
             if fused is not None:
                 packed, wsf, wsf2, _ = fused
                 return cls(shape, dtype, packed), wsf, wsf2
+        if weights_scaling_factor_2 is None and weights_scaling_factor is None:
+            whole = _hip.nvfp4_quantize_dynamic(x, block_size, nvfp4_quantize_flags())
+            if whole is not None:
+                packed, wsf, wsf2 = whole
+                return cls(shape, dtype, packed), wsf, wsf2
         if weights_scaling_factor_2 is None:
             acc = torch.zeros(1, dtype=torch.float32, device=x.device)
             _hip.absmax_into(x, acc, 1, 1, x.numel(), reread=True)   # the quantize pass reads x next
