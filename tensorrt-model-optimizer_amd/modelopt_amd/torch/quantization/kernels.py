@@ -205,8 +205,12 @@ def fake_quant_fp8(x, amax=None, saturate=False):
 
 def ste_mask(x, amax, grad):
     """``torch.where(x.abs() <= amax, grad, 0)`` in one pass, or None where the kernel does not apply:
-    mixed types, a gradient in another memory order, an amax on two separated runs of dims."""
-    if (not (x.is_cuda and grad.is_cuda and amax.is_cuda) or x.dtype != grad.dtype or x.dim() == 0
+    mixed types, a gradient in another memory order, an amax on two separated runs of dims, a gradient
+    that is itself differentiated (``create_graph``), batched or traced."""
+    if (torch_is_intercepted() or (grad.requires_grad and torch.is_grad_enabled())
+            or not torch._C._has_storage(grad)):
+        return None
+    if (type(grad) is not torch.Tensor or not (x.is_cuda and grad.is_cuda and amax.is_cuda) or x.dtype != grad.dtype or x.dim() == 0
             or x.shape != grad.shape or x.dtype not in _hip._DTYPES or amax.dtype not in _hip._DTYPES
             or not x.is_contiguous() or not grad.is_contiguous()):
         return None
@@ -237,9 +241,11 @@ def fake_quant_block_fp(x, block_size, fmt, scale_fmt="E8M0", global_amax=None):
 
 
 def torch_is_intercepted() -> bool:
-    """Whether something follows the tensor operations of this thread (a dispatch or function mode,
-    a functorch transform, forward-mode differentiation, a trace):
+    """Whether something follows the tensor operations of this thread (a compiler, a dispatch or
+    function mode, a functorch transform, forward-mode differentiation, a trace):
     a shortcut past an operator that it would see is not taken then."""
+    if torch.compiler.is_compiling():
+        return True
     return bool(torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None)
