@@ -450,14 +450,13 @@ __device__ __forceinline__ void qdq_block16_bf16(const uint32_t (&w)[8], float g
 
 // RP = pairs of 16-byte loads per lane (a workgroup handles RP * 256 blocks).  Measured: one pair
 // beats four from 50 MB of input (8192 x 4096: 5.4 - 5.7 TB/s against 5.0; 537 MB: 6.45 against
-// 6.0) and ties at 34 MB; smaller tensors keep four (fewer workgroups to launch).
+// 6.0) and ties at 34 MB; smaller tensors go row by row.
 template <int MODE, int RP>
 __global__ __launch_bounds__(256) void nvfp4_qdq_fast_kernel(const uint16_t* __restrict__ x,
                                                              uint16_t* __restrict__ y,
                                                              int64_t nblocks, const void* amax,
                                                              int amax_dtype) {
-    __shared__ uint32_t smem[4];
-    const float gs = tensor_amax(amax, amax_dtype, smem) / 2688.0f;
+    const float gs = load_scalar(amax, amax_dtype, 0) / 2688.0f;
     const float gs_safe = gs > 0.0f ? gs : 1e-12f;
     const int64_t nchunks = nblocks * 2;
     const int64_t c0 = (int64_t)blockIdx.x * (RP * 512) + threadIdx.x;
@@ -655,42 +654,31 @@ extern "C" int mo_nvfp4_dequantize(const uint8_t* packed, const uint8_t* wsf, co
     return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
 }
 
-namespace mo {
-// amax_dtype: a type, or parts (kAmaxParts + their number)
-int nvfp4_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* amax, int amax_dtype,
-              int block_size, int mode, hipStream_t s) {
-    const int64_t kp = (k + block_size - 1) / block_size * block_size;
-    if (dtype == MO_BF16 && block_size == 16 && k == kp &&
-        ((((uintptr_t)x | (uintptr_t)y) & 15u) == 0)) {
-        const int64_t nblocks = rows * k / 16;
-        const bool big = nblocks >= tuned("nvfp4_qdq_big_blocks", 1ll << 20);   // 16 Mi elements = 32 MB of bf16
-        const int64_t per_tile = (big ? 1 : 4) * 256;         // blocks per workgroup
-        const int64_t tiles = (nblocks + per_tile - 1) / per_tile;
-        if (tiles > 0x7FFFFFFF) return MO_ERR_UNSUPPORTED;
-        const unsigned g = (unsigned)tiles;
-        const size_t cap = ballast_bytes("nvfp4_qdq_fast_kernel", 0);
-        const uint16_t* xi = (const uint16_t*)x;
-        uint16_t* yo = (uint16_t*)y;
-        if (mode == 0 && big) nvfp4_qdq_fast_kernel<0, 1><<<g, 256, cap, s>>>(xi, yo, nblocks, amax, amax_dtype);
-        else if (mode == 0) nvfp4_qdq_fast_kernel<0, 4><<<g, 256, cap, s>>>(xi, yo, nblocks, amax, amax_dtype);
-        else if (big) nvfp4_qdq_fast_kernel<1, 1><<<g, 256, cap, s>>>(xi, yo, nblocks, amax, amax_dtype);
-        else nvfp4_qdq_fast_kernel<1, 4><<<g, 256, cap, s>>>(xi, yo, nblocks, amax, amax_dtype);
-        return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
-    }
-    // every other type, block size and layout
-    return row_qdq(x, y, rows, k, dtype, nullptr, MO_ROW_NVFP4, block_size, mode, 0, amax, amax_dtype, s);
-}
-}  // namespace mo
-
 extern "C" int mo_nvfp4_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype,
                             const void* amax, int amax_dtype, int block_size, int mode,
                             void* stream) {
     if (rows < 0 || k < 0 || (mode != 0 && mode != 1)) return MO_ERR_ARG;
     if (block_size != 8 && block_size != 16 && block_size != 32) return MO_ERR_UNSUPPORTED;
-    if (dtype < MO_F32 || dtype > MO_BF16 || amax_dtype < MO_F32 || amax_dtype > MO_BF16) return MO_ERR_DTYPE;
+    if (amax_dtype < MO_F32 || amax_dtype > MO_BF16) return MO_ERR_DTYPE;
     if (rows == 0 || k == 0) return MO_OK;
-    if (!x || !y || !amax || (((uintptr_t)x | (uintptr_t)y) & (dtype == MO_F32 ? 3u : 1u))) return MO_ERR_ARG;
-    return mo::nvfp4_qdq(x, y, rows, k, dtype, amax, amax_dtype, block_size, mode, (hipStream_t)stream);
+    if (!x || !y || !amax) return MO_ERR_ARG;
+    hipStream_t s = (hipStream_t)stream;
+    const int64_t nblocks = rows * k / 16;
+    // from 32 MB the two kernels tie (8192 x 8192 43.1 and 43.2 us), below it the row-wise one is faster
+    // (64 x 4096 3.0 us against 4.4)
+    if (dtype == MO_BF16 && block_size == 16 && k % 16 == 0 && nblocks >= (1ll << 20) &&
+        ((((uintptr_t)x | (uintptr_t)y) & 15u) == 0)) {
+        const int64_t tiles = (nblocks + 255) / 256;
+        if (tiles > 0x7FFFFFFF) return MO_ERR_UNSUPPORTED;
+        const unsigned g = (unsigned)tiles;
+        const uint16_t* xi = (const uint16_t*)x;
+        uint16_t* yo = (uint16_t*)y;
+        if (mode == 0) mo::nvfp4_qdq_fast_kernel<0, 1><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
+        else mo::nvfp4_qdq_fast_kernel<1, 1><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
+        return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
+    }
+    // every other size, type, block size and layout
+    return mo_row_qdq(x, y, rows, k, dtype, nullptr, MO_ROW_NVFP4, block_size, mode, 0, amax, amax_dtype, stream);
 }
 
 extern "C" int mo_nvfp4_quantize_multi(const mo_nvfp4_job* jobs_dev, int njobs,

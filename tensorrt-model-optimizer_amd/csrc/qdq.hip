@@ -30,10 +30,7 @@ __global__ __launch_bounds__(256) void qdq_kernel(const void* __restrict__ x, vo
     const int64_t chunks = n >> 3;
     const int64_t c0 = (int64_t)blockIdx.x * kTileChunks + threadIdx.x;
     typename Op::Scale s0 = {};
-    if constexpr (KIND == TENSOR) {
-        __shared__ uint32_t smem[4];
-        if (amax) s0 = op.make(tensor_amax(amax, amax_dtype, smem));
-    }
+    if (KIND == TENSOR && amax) s0 = op.make(load_scalar(amax, amax_dtype, 0));
     if (chunks > 0) {
         // All loads of the lane (the per-chunk amax too) come first, in straight-line code: a
         // chunk past the end re-reads the last one and is not stored.  Loads inside per-chunk
@@ -85,8 +82,9 @@ __global__ __launch_bounds__(256) void qdq_kernel(const void* __restrict__ x, vo
     // tail (n % 8 elements): the first lanes of the last workgroup
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x < (n & 7)) {
         const int64_t i = (chunks << 3) + threadIdx.x;
-        typename Op::Scale s = s0;
-        if (KIND != TENSOR && amax) s = op.make(load_scalar(amax, amax_dtype, (i / inner) % axis));
+        const int64_t a = KIND == TENSOR ? 0 : (i / inner) % axis;
+        typename Op::Scale s = {};
+        if (amax) s = op.make(load_scalar(amax, amax_dtype, a));
         store_elem<DT>(y, i, op.template apply<FLAG>(load_elem<DT>(x, i), s));
     }
 }
@@ -387,9 +385,13 @@ static int check_common(const void* x, void* y, int64_t outer, int64_t axis, int
     return MO_OK;
 }
 
-static int fp8_qdq(const void* x, void* y, int64_t outer, int64_t axis, int64_t inner, int dtype,
-                   const void* amax, int amax_dtype, int saturate, hipStream_t s) {
-    int rc;
+extern "C" int mo_fp8_qdq(const void* x, void* y, int64_t outer, int64_t axis, int64_t inner,
+                          int dtype, const void* amax, int amax_dtype, int saturate,
+                          void* stream) {
+    int rc = check_common(x, y, outer, axis, inner, amax_dtype);
+    if (rc != MO_OK) return rc;
+    if (outer == 0 || axis == 0 || inner == 0) return MO_OK;
+    hipStream_t s = (hipStream_t)stream;
 #define CALL2(DT, SAT)                                                                                 \
     rc = amax ? mo::launch_qdq<DT, SAT>(x, y, outer, axis, inner, amax, amax_dtype,                    \
                                         mo::Fp8Op<true>(), s)                                          \
@@ -409,18 +411,14 @@ static int fp8_qdq(const void* x, void* y, int64_t outer, int64_t axis, int64_t 
     return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
 }
 
-extern "C" int mo_fp8_qdq(const void* x, void* y, int64_t outer, int64_t axis, int64_t inner,
-                          int dtype, const void* amax, int amax_dtype, int saturate,
-                          void* stream) {
-    const int rc = check_common(x, y, outer, axis, inner, amax_dtype);
-    if (rc != MO_OK || outer == 0 || axis == 0 || inner == 0) return rc;
-    return fp8_qdq(x, y, outer, axis, inner, dtype, amax, amax_dtype, saturate, (hipStream_t)stream);
-}
-
-static int int_qdq(const void* x, void* y, int64_t outer, int64_t axis, int64_t inner, int dtype,
-                   const void* amax, int amax_dtype, int num_bits, int is_unsigned, int narrow_range,
-                   hipStream_t s) {
-    int rc;
+extern "C" int mo_int_qdq(const void* x, void* y, int64_t outer, int64_t axis, int64_t inner,
+                          int dtype, const void* amax, int amax_dtype, int num_bits,
+                          int is_unsigned, int narrow_range, void* stream) {
+    int rc = check_common(x, y, outer, axis, inner, amax_dtype);
+    if (rc != MO_OK) return rc;
+    if (!amax || num_bits < 1 || num_bits > 24) return MO_ERR_ARG;
+    if (outer == 0 || axis == 0 || inner == 0) return MO_OK;
+    hipStream_t s = (hipStream_t)stream;
     mo::IntOp op;
     op.bound = (float)((1 << (num_bits - 1 + (is_unsigned ? 1 : 0))) - 1);
     op.lo = is_unsigned ? 0.0f : (narrow_range ? -op.bound : -op.bound - 1.0f);
@@ -432,45 +430,6 @@ static int int_qdq(const void* x, void* y, int64_t outer, int64_t axis, int64_t 
     }
     if (rc != MO_OK) return rc;
     return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
-}
-
-extern "C" int mo_int_qdq(const void* x, void* y, int64_t outer, int64_t axis, int64_t inner,
-                          int dtype, const void* amax, int amax_dtype, int num_bits,
-                          int is_unsigned, int narrow_range, void* stream) {
-    const int rc = check_common(x, y, outer, axis, inner, amax_dtype);
-    if (rc != MO_OK) return rc;
-    if (!amax || num_bits < 1 || num_bits > 24) return MO_ERR_ARG;
-    if (outer == 0 || axis == 0 || inner == 0) return MO_OK;
-    return int_qdq(x, y, outer, axis, inner, dtype, amax, amax_dtype, num_bits, is_unsigned, narrow_range,
-                   (hipStream_t)stream);
-}
-
-// The abs-max parts and the fake quantisation that folds them: two launches, nothing to clear.
-// 4096 x 4096 bf16 to FP8: 18.9 us, 33.2 as four launches (fill, abs-max, conversion, quantise).
-extern "C" int mo_dynamic_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, int kind, int p0, int p1,
-                              int p2, void* parts, void* stream) {
-    if (rows < 0 || k < 0) return MO_ERR_ARG;
-    if (dtype < MO_F32 || dtype > MO_BF16) return MO_ERR_DTYPE;
-    switch (kind) {
-        case MO_ROW_INT: if (p0 < 1 || p0 > 24) return MO_ERR_ARG; break;
-        case MO_ROW_FP8: break;
-        case MO_ROW_NVFP4:
-            if (p1 != 0 && p1 != 1) return MO_ERR_ARG;
-            if (p0 != 8 && p0 != 16 && p0 != 32) return MO_ERR_UNSUPPORTED;
-            break;
-        default: return MO_ERR_UNSUPPORTED;
-    }
-    if (rows == 0 || k == 0) return MO_OK;
-    if (!x || !y || !parts) return MO_ERR_ARG;
-    if (((uintptr_t)x | (uintptr_t)y) & 15u) return MO_ERR_UNSUPPORTED;
-    hipStream_t s = (hipStream_t)stream;
-    int nparts = 0;
-    const int rc = mo::launch_absmax_parts(x, rows * k, dtype, true, (uint32_t*)parts, &nparts, s);
-    if (rc != MO_OK) return rc;
-    const int amax_dtype = mo::kAmaxParts + nparts;
-    if (kind == MO_ROW_FP8) return fp8_qdq(x, y, 1, 1, rows * k, dtype, parts, amax_dtype, p0, s);
-    if (kind == MO_ROW_INT) return int_qdq(x, y, 1, 1, rows * k, dtype, parts, amax_dtype, p0, p1, p2, s);
-    return mo::nvfp4_qdq(x, y, rows, k, dtype, parts, amax_dtype, p0, p1, s);
 }
 
 extern "C" int mo_fp8_qdq_blocks2d(const void* x, void* y, int64_t rows, int64_t cols,

@@ -118,11 +118,11 @@ def dtype_code(dt: torch.dtype) -> int:
 
 def _stream(t: torch.Tensor):
     """torch's current stream on the device of ``t`` as the C ABI takes it."""
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(t.device.index))
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _require_device(*tensors):
@@ -188,8 +188,8 @@ class KernelTimer:
 
 def call(name: str, anchor: torch.Tensor, *args):
     """Invoke ``name`` with the device of ``anchor`` current; raise on a non-zero status."""
-    lib = load()
-    if _timer is None and anchor.device.index == torch.cuda.current_device():
+    lib = _lib if _lib is not None else load()
+    if _timer is None and anchor.get_device() == torch._C._cuda_getDevice():
         rc = getattr(lib, name)(*args)   # the common case, without the context manager's cost
     else:
         with torch.cuda.device(anchor.device):
@@ -451,13 +451,14 @@ def row_qdq(x, pre_scale, kind, p0=0, p1=0, p2=0, amax=None):
     """Fake quantisation of ``T(x * pre_scale)`` (``x`` itself when ``pre_scale`` is None) along the last dim
     in one pass; ``kind`` and ``p0`` .. ``p2`` as in ``mo_row_qdq``, ``amax`` one device element (None for
     ``MO_ROW_MX``)."""
-    _require_device(x, pre_scale, amax)
+    if not x.is_cuda or pre_scale is not None or amax is not None:
+        _require_device(x, pre_scale, amax)
     assert x.is_contiguous() and (pre_scale is None or (pre_scale.is_contiguous() and pre_scale.dtype == x.dtype
                                                         and pre_scale.numel() == x.shape[-1]))
     k = x.shape[-1]
     y = torch.empty_like(x)
-    call("mo_row_qdq", x, _ptr(x), _ptr(y), x.numel() // k if k else 0, k, dtype_code(x.dtype), _ptr(pre_scale),
-         kind, int(p0), int(p1), int(p2), _ptr(amax), MO_F32 if amax is None else dtype_code(amax.dtype), _stream(x))
+    call("mo_row_qdq", x, x.data_ptr(), y.data_ptr(), x.numel() // k if k else 0, k, dtype_code(x.dtype),
+         _ptr(pre_scale), kind, p0, p1, p2, _ptr(amax), MO_F32 if amax is None else dtype_code(amax.dtype), _stream(x))
     return y
 
 

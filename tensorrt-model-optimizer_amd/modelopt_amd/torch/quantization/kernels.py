@@ -9,12 +9,11 @@ import math
 import torch
 
 from ... import _hip
-from .overflow import fp8_saturates
 
 __all__ = [
     "amax_layout", "kept_dims_first", "dense_flat_view", "absmax_accumulate", "reduce_amax_gpu", "fake_quant_int", "fake_quant_fp8",
-    "ste_mask", "fake_quant_nvfp4", "fake_quant_block_fp", "fake_quant_prescaled",
-    "mul_last_dim", "torch_is_intercepted",
+    "ste_mask", "fake_quant_nvfp4", "fake_quant_block_fp", "mul_last_dim",
+    "torch_is_intercepted",
 ]
 
 
@@ -249,37 +248,6 @@ def torch_is_intercepted() -> bool:
     return bool(torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None)
-
-
-_BLOCK_FORMATS = {(4, 3): "E4M3", (5, 2): "E5M2", 8: "INT8", (0, 3): "E0M3", (1, 2): "E1M2", (3, 0): "E3M0",
-                  (2, 1): "E2M1", (3, 2): "E3M2", (2, 3): "E2M3"}
-
-
-def fake_quant_prescaled(x, scale, amax, kind, *args):
-    """Fake quantisation of ``x * scale`` (``scale`` one element per column) in one pass:
-    ``kind`` "int" (num_bits, unsigned, narrow_range), "fp8", or "block" (block size, element bits,
-    scale bits) with NVFP4 or power-of-two block scales.  None where the kernel has no such form."""
-    if x.dtype not in _hip._DTYPES or (amax is not None and (amax.dtype not in _hip._DTYPES or not amax.is_cuda)):
-        return None
-    if kind == "int":
-        if not 1 <= args[0] <= 24:
-            return None
-        form = (_hip.MO_ROW_INT, args[0], bool(args[1]), bool(args[2]))
-    elif kind == "fp8":
-        form = (_hip.MO_ROW_FP8, fp8_saturates(amax), 0, 0)
-    else:
-        block, bits, scale_bits = args
-        if block not in (8, 16, 32) or type(bits) not in (int, tuple):
-            return None
-        if scale_bits == (8, 0) and bits in _BLOCK_FORMATS:
-            form = (_hip.MO_ROW_MX, block, _hip.ELEM_FORMATS.index(_BLOCK_FORMATS[bits]), 0)
-        elif scale_bits == (4, 3) and bits == (2, 1):
-            from . import tensor_quant
-            form = (_hip.MO_ROW_NVFP4, block, tensor_quant.NVFP4_FAKE_QUANT_MODE, 0)
-        else:
-            return None
-    x = x if x.is_contiguous() else x.contiguous()
-    return _hip.row_qdq(x, scale.reshape(-1).contiguous(), *form, amax)
 
 
 def mul_last_dim(x, scale):

@@ -16,6 +16,7 @@ import torch.nn.functional as F
 from torch import nn
 from torch.nn.modules import module as _module_hooks
 
+from ..... import _hip
 from ... import calib, kernels, modes, tensor_quant
 from ... import utils as quant_utils
 from ...config import QuantizerAttributeConfig
@@ -26,6 +27,10 @@ from ...tensor_quant import dynamic_block_quant, fake_tensor_quant, scaled_e4m3
 
 __all__ = ["SequentialQuantizer", "TensorQuantizer"]
 
+_PLAIN_TENSORS = (torch.Tensor, nn.Parameter)   # no subclass, packed tensors among them
+# element formats of the MX block kernel by their bits
+_MX_ELEMENTS = {bits: _hip.ELEM_FORMATS.index(name) for bits, name in tensor_quant.mx_format_map.items()
+                if name != "E8M0"}
 _DEFAULT_CONFIG = []
 
 
@@ -440,37 +445,10 @@ class TensorQuantizer(nn.Module):
                                                self._narrow_range)
         return None if done is None else done[0]
 
-    def _dynamic_fake_quant(self, inputs):
-        """Fake quantisation with the abs-max of the input itself in two launches (the maxima of parts of
-        the tensor, folded by the launch that quantises): an accumulator would be filled, reduced into
-        by atomics and converted first.  For plain tensors that are not differentiated, traced or
-        transformed; None for all else."""
-        bs, bits = self._block_sizes, self._num_bits
-        if (hasattr(self, "_amax") or self._axis is not None or not inputs.is_cuda
-                or type(inputs) not in (torch.Tensor, nn.Parameter) or modes.strict_checks()
-                or (inputs.requires_grad and torch.is_grad_enabled())
-                or kernels.torch_is_intercepted()):
-            return None
-        if bs is None:
-            if type(bits) is int and 1 <= bits <= 24:
-                return kernels._hip.dynamic_qdq(inputs, kernels._hip.MO_ROW_INT, bits, bool(self._unsigned),
-                                                bool(self._narrow_range))
-            if bits == (4, 3):
-                # a per-tensor amax clamps unless "nan" is selected
-                return kernels._hip.dynamic_qdq(inputs, kernels._hip.MO_ROW_FP8,
-                                                get_fp8_overflow_behavior() != "nan")
-        elif (bs.get("type", "static") == "dynamic" and bits == (2, 1) and bs.get("scale_bits") == (4, 3)
-                and bs.get(-1) in (8, 16, 32)):
-            return kernels._hip.dynamic_qdq(inputs, kernels._hip.MO_ROW_NVFP4, bs[-1],
-                                            tensor_quant.NVFP4_FAKE_QUANT_MODE)
-        return None
-
     def _fake_quantize(self, inputs):
-        done = self._fused_dynamic_per_tensor(inputs)
-        if done is None:
-            done = self._dynamic_fake_quant(inputs)
-        if done is not None:
-            return done
+        fused = self._fused_dynamic_per_tensor(inputs)
+        if fused is not None:
+            return fused
         amax = None if self.is_mx_format else self._get_amax(inputs)
         bs = self.block_sizes
         if bs is not None and bs.get("type", "static") == "dynamic":
@@ -612,51 +590,81 @@ class TensorQuantizer(nn.Module):
             return kernels.mul_last_dim(inputs, pqs.to(inputs.device))
         return inputs * pqs  # other shapes / mixed dtypes: torch broadcasting and type promotion
 
-    def _prescaled_fake_quant(self, inputs, scale):
-        """The scale and the quantizer in one launch: the product alone is a pass over the tensor
-        (2048 x 14336 bf16 to INT8: 43.2 us in two launches, 22.7 in one = 5.2 TB/s; a decode-sized
-        input saves a launch).  For one calibrated abs-max or block scales of a power of two, on
-        plain tensors that are not differentiated, traced or transformed; None for all else."""
-        if (type(self) is not TensorQuantizer or type(inputs) not in (torch.Tensor, nn.Parameter)
-                or self._disabled or not self._if_quant or not self._fake_quant or self._rotate
-                or (self._if_calib and not self._dynamic) or modes.strict_checks()
-                or not inputs.is_cuda or inputs.dim() == 0
-                or (torch.is_grad_enabled() and (inputs.requires_grad or scale.requires_grad))
-                or scale.dtype != inputs.dtype or scale.device != inputs.device
-                or scale.numel() != inputs.shape[-1] or scale.shape[-1] != inputs.shape[-1]
+    def _direct_fake_quant(self, inputs):
+        """Fake quantisation with one abs-max for the tensor or with dynamic block scales, straight to
+        the kernel: a plain tensor in GPU memory that is not differentiated, traced or transformed,
+        no statistics to collect.  None for all else (``forward`` goes on, step by step).
+
+        The steps of ``forward`` and the operator behind them cost the host 17 us, more than the
+        kernel up to some 4 million elements; this way 10.5.  A pre-quant scale is multiplied in
+        the quantizer's launch (the product alone is a pass over the tensor: 2048 x 14336 bf16 to
+        INT8 43.2 us in two launches, 22.7 in one = 5.2 TB/s), and a missing abs-max is taken as
+        maxima of parts that the quantising launch folds (an accumulator would be filled, reduced
+        into by atomics and converted first)."""
+        own = self.__dict__
+        if (own["_disabled"] or not own["_if_quant"] or not own["_fake_quant"] or own["_rotate"]
+                or (own["_if_calib"] and not own["_dynamic"]) or type(self) is not TensorQuantizer
+                or not inputs.is_cuda or modes.strict_checks() or modes.one_launch_dynamic_quant()):
+            return None
+        bs, bits = own["_block_sizes"], own["_num_bits"]
+        p1 = p2 = 0
+        if bs is None:
+            if type(bits) is int and 1 <= bits <= 24:
+                kind, p0, p1, p2 = _hip.MO_ROW_INT, bits, bool(own["_unsigned"]), bool(own["_narrow_range"])
+            elif bits == (4, 3):   # a per-tensor amax clamps unless "nan" is selected
+                kind, p0 = _hip.MO_ROW_FP8, get_fp8_overflow_behavior() != "nan"
+            else:
+                return None
+        else:
+            p0, scale_bits = bs.get(-1), bs.get("scale_bits")
+            if bs.get("type") != "dynamic" or p0 not in (8, 16, 32):
+                return None
+            if scale_bits == (4, 3) and bits == (2, 1):
+                kind, p1 = _hip.MO_ROW_NVFP4, tensor_quant.NVFP4_FAKE_QUANT_MODE
+            elif scale_bits == (8, 0) and type(bits) in (int, tuple) and bits in _MX_ELEMENTS:
+                kind, p1 = _hip.MO_ROW_MX, _MX_ELEMENTS[bits]
+            else:
+                return None
+        buffers = own["_buffers"]
+        scale = buffers.get("_pre_quant_scale") if own["_enable_pre_quant_scale"] else None
+        amax = buffers.get("_amax")
+        for name in ("_amax", "_pre_quant_scale"):   # kept as anything but a buffer with a tensor
+            if name in own or name in own["_parameters"] or buffers.get(name, self) is None:
+                return None
+        if (inputs.dtype not in _hip._DTYPES or inputs.dim() == 0 or inputs.numel() == 0
+                or (torch.is_grad_enabled() and (inputs.requires_grad or (scale is not None and scale.requires_grad)))
                 or kernels.torch_is_intercepted()):
             return None
-        bs, bits, args = self._block_sizes, self._num_bits, None
-        if bs is None:
-            if type(bits) is int:
-                args = ("int", bits, self._unsigned, self._narrow_range)
-            elif bits == (4, 3):
-                args = ("fp8",)
-        elif bs.get("type", "static") == "dynamic":
-            args = ("block", bs.get(-1), bits, bs.get("scale_bits"))
-        if args is None:
-            return None
-        amax = None
-        if not self.is_mx_format:
-            if not hasattr(self, "_amax") or self._amax.numel() != 1:
+        if scale is not None:
+            k = inputs.shape[-1]
+            if (scale.dtype != inputs.dtype or scale.device != inputs.device or scale.numel() != k
+                    or scale.shape[-1] != k):
                 return None
-            amax = self._get_amax(inputs)
-        return kernels.fake_quant_prescaled(inputs, scale, amax, *args)
+            scale = scale.reshape(-1).contiguous()
+        if kind == _hip.MO_ROW_MX:
+            amax = None
+        elif amax is None:
+            if scale is not None or own["_axis"] is not None:
+                return None
+            return _hip.dynamic_qdq(inputs if inputs.is_contiguous() else inputs.contiguous(), kind, p0, p1, p2)
+        elif amax.numel() != 1 or amax.device != inputs.device or amax.dtype not in _hip._DTYPES:
+            return None
+        return _hip.row_qdq(inputs if inputs.is_contiguous() else inputs.contiguous(), scale, kind, p0, p1, p2, amax)
 
     def forward(self, inputs):
         """Scale -> (calibrate) -> (quantise); returns a tensor of the input dtype for fake
         quantisation, a ``QTensorWrapper``-able packed tensor for real quantisation."""
+        if type(inputs) in _PLAIN_TENSORS and not torch.compiler.is_compiling():
+            outputs = self._direct_fake_quant(inputs)
+            if outputs is not None:
+                return outputs
         if isinstance(inputs, (BaseQuantizedTensor, QTensorWrapper)):
             assert self._dequantize, "No dequantization stats in the tensor quantizer."
             return self.dequantize(inputs)
         if inputs.numel() == 0:  # e.g. an MoE expert that saw no token
             return inputs
         source = inputs
-        scale = self.pre_quant_scale
-        if scale is not None:
-            outputs = self._prescaled_fake_quant(inputs, scale)
-            if outputs is not None:
-                return outputs
+        if self.pre_quant_scale is not None:
             inputs = self._apply_pre_quant_scale(inputs)
         if self._rotate:
             raise NotImplementedError("Hadamard rotation is outside the hot path built here")

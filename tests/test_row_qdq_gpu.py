@@ -121,3 +121,36 @@ def test_a_pre_quant_scale_equals_the_scaled_input(name, dtype, form):
     assert torch.equal(torch.isnan(got), torch.isnan(want))
     keep = ~torch.isnan(want)
     assert torch.equal(got[keep], want[keep])
+
+
+@pytest.mark.parametrize("name", FORMATS)
+@pytest.mark.parametrize("dtype", DTYPES + [torch.float64])
+@pytest.mark.parametrize("form", ["plain", "one_dim", "strided", "unaligned", "parameter", "scaled", "dynamic", "amax_1x1",
+                                  "amax_on_cpu", "nan_overflow", "inference"])
+def test_the_direct_route_equals_the_steps_of_forward(name, dtype, form, monkeypatch):
+    from modelopt_amd.torch.quantization.config import QuantizerAttributeConfig
+    from modelopt_amd.torch.quantization.nn import TensorQuantizer
+    from modelopt_amd.torch.quantization.overflow import set_fp8_overflow_behavior
+
+    if dtype == torch.float64 and (FORMATS[name].get("block_sizes") or form == "scaled"):
+        pytest.skip("neither the block formats nor the scale take float64")
+    flat = torch.randn(11 * 96 + 1, generator=torch.Generator().manual_seed(6)).mul_(3).to(dtype).to(DEV)
+    x = (flat[1:] if form == "unaligned" else flat[:-1]).view(11, 96)
+    x = {"one_dim": x[3], "strided": x[:, :].t().contiguous().t(), "parameter": torch.nn.Parameter(x)}.get(form, x)
+    q = TensorQuantizer(QuantizerAttributeConfig(**FORMATS[name]))
+    if form == "scaled":
+        q.pre_quant_scale = torch.linspace(0.5, 2, 96).to(dtype).to(DEV)
+    if form != "dynamic" and not q.is_mx_format:
+        q.amax = torch.full((1, 1) if form == "amax_1x1" else (), 2.5, dtype=dtype,
+                            device="cpu" if form == "amax_on_cpu" else DEV)
+    previous = set_fp8_overflow_behavior("nan" if form == "nan_overflow" else "auto")
+    try:
+        with torch.inference_mode(form == "inference"), torch.no_grad():
+            got = q(x)
+            monkeypatch.setattr(TensorQuantizer, "_direct_fake_quant", lambda self, inputs: None)
+            want = q(x)
+    finally:
+        set_fp8_overflow_behavior(previous)
+    assert got.shape == want.shape and got.dtype == want.dtype and got.is_contiguous() == want.is_contiguous()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got.nan_to_num(nan=0.0), want.nan_to_num(nan=0.0))
