@@ -245,6 +245,14 @@ int mo_row_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const
 int mo_dynamic_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, int kind, int p0, int p1, int p2,
                    void* parts, void* stream);
 
+/* Weight gradient of a linear layer whose weight is fake-quantised (F.linear behind the straight-through
+ * estimator of TQ/tensor_quant.py:315-319): dw[n, k] = |w[n, k]| <= amax[(n * K + k) / inner] ?
+ * T(sum over t of dy[t, n] * x[t, k]) : 0, sums in fp32; inner = 0: one amax.  dy [tokens, n], x [tokens, k],
+ * w and dw [n, k], all of type dtype (fp16 or bf16), 16-byte aligned, n, k and inner multiples of 8,
+ * k a multiple of inner (MO_ERR_UNSUPPORTED otherwise).  narrow_amax: the amax is rounded to dtype before the comparison. */
+int mo_wgrad_masked(const void* dy, const void* x, const void* w, void* dw, int64_t tokens, int64_t n, int64_t k,
+                    int dtype, const void* amax, int amax_dtype, int64_t inner, int narrow_amax, void* stream);
+
 /* ------------------------------------------------------------------ real quantize + pack */
 
 /* Squared fake-quantisation error for n_cand candidate amax values in one pass over x viewed

@@ -43,6 +43,7 @@ SIGNATURES = {
     "mo_fp8_qdq": [_P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _P],
     "mo_int_qdq": [_P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _P],
     "mo_ste_mask": [_P, _P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _P],
+    "mo_wgrad_masked": [_P, _P, _P, _P, _I64, _I64, _I64, _INT, _P, _INT, _I64, _INT, _P],
     "mo_row_qdq": [_P, _P, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _P, _INT, _P],
     "mo_nvfp4_qdq": [_P, _P, _I64, _I64, _INT, _P, _INT, _INT, _INT, _P],
     "mo_qdq_sq_err": [_P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _INT, _INT, _P, _P],
@@ -375,6 +376,24 @@ def ste_mask(x, grad, amax, outer, axis, inner, narrow_amax=False):
     call("mo_ste_mask", x, _ptr(x), _ptr(grad), _ptr(out), outer, axis, inner, dtype_code(x.dtype),
          _ptr(amax), dtype_code(amax.dtype), int(narrow_amax), _stream(x))
     return out
+
+
+def wgrad_masked(dy, x, w, amax, inner=0, narrow_amax=False):
+    """``where(|w| <= amax, dy.T @ x, 0)`` in the dtype of ``w`` with sums in fp32 (``dy`` [tokens, n], ``x``
+    [tokens, k], ``w`` [n, k]); ``inner`` elements of ``w`` in a row share an amax (0: all).  None, with
+    nothing launched, where the kernel has no such form."""
+    _require_device(dy, x, w, amax)
+    tokens, n, k = dy.shape[0], dy.shape[1], x.shape[1]
+    if (w.dtype not in (torch.bfloat16, torch.float16) or dy.dtype != w.dtype or x.dtype != w.dtype
+            or tokens == 0 or n % 8 or k % 8 or inner % 8 or (inner and k % inner) or w.numel() == 0
+            or (dy.data_ptr() | x.data_ptr() | w.data_ptr()) % 16):
+        return None
+    assert dy.is_contiguous() and x.is_contiguous() and w.is_contiguous() and amax.is_contiguous()
+    assert x.shape[0] == tokens and w.shape == (n, k) and amax.numel() == (w.numel() // inner if inner else 1)
+    dw = torch.empty_like(w)
+    call("mo_wgrad_masked", w, _ptr(dy), _ptr(x), _ptr(w), _ptr(dw), tokens, n, k, dtype_code(w.dtype), _ptr(amax),
+         dtype_code(amax.dtype), inner, int(narrow_amax), _stream(w))
+    return dw
 
 
 def blocks2d_covered(x, rows, cols, block_rows, block_cols) -> bool:

@@ -1,11 +1,15 @@
 """Quantised ``nn.Linear`` (reference: nn/modules/quant_linear.py:39-115)."""
 
+import torch
 import torch.nn.functional as F
 from torch import nn
 
+from ... import kernels
 from ...config import QuantizerAttributeConfig
 from ...qtensor.base_qtensor import QTensorWrapper
+from ...tensor_quant import MaskedGradientLinear
 from .quant_module import QuantLinearConvBase, QuantModule, QuantModuleRegistry
+from .tensor_quantizer import TensorQuantizer, quantizer_has_hooks
 
 __all__ = ["Linear", "QuantLinear", "RealQuantLinear"]
 
@@ -18,9 +22,33 @@ class _QuantLinear(QuantLinearConvBase):
 
     def forward(self, input, *args, **kwargs):
         input = self.input_quantizer(input)
-        weight = self.weight_quantizer(self.weight)
-        output = F.linear(input, weight, self.bias)
+        output = self._masked_gradient_linear(input) if torch.is_grad_enabled() else None
+        if output is None:
+            weight = self.weight_quantizer(self.weight)
+            output = F.linear(input, weight, self.bias)
         return self.output_quantizer(output)
+
+    def _masked_gradient_linear(self, input):
+        """The weight quantizer and the linear layer as one autograd function, whose weight gradient is
+        masked by the kernel that computes it.  For a trained 16-bit weight behind a plain, calibrated
+        quantizer with a clipping backward; None for all else: hooks on the quantizer (which would see
+        its output with a graph), autocast, transforms, traces, and shapes with nothing to gain."""
+        weight, quantizer = self._parameters.get("weight"), self._modules.get("weight_quantizer")
+        if (type(quantizer) is not TensorQuantizer or type(weight) is not nn.Parameter
+                or self.weight is not weight or type(input) is not torch.Tensor
+                or not weight.requires_grad or not weight.is_cuda or not input.is_cuda
+                or weight.dim() != 2 or input.dim() < 2
+                or input.dtype != weight.dtype or weight.dtype not in (torch.bfloat16, torch.float16)
+                or not weight.is_contiguous() or input.shape[-1] != weight.shape[1]
+                or not kernels.wgrad_mask_pays(input.numel() // weight.shape[1], *weight.shape)
+                or torch.is_autocast_enabled("cuda") or quantizer_has_hooks(quantizer)
+                or torch.compiler.is_compiling() or kernels.torch_is_intercepted()
+                or (self.bias is not None and type(self.bias) is not nn.Parameter)):
+            return None
+        amax = quantizer.clipping_amax(weight)
+        if amax is None:
+            return None
+        return MaskedGradientLinear.apply(input, weight, self.bias, quantizer, *amax)
 
 
 class QuantLinear(_QuantLinear, nn.Linear):

@@ -747,6 +747,35 @@ class TensorQuantizer(nn.Module):
             return x0, x1
         return first(x0), second(x1)
 
+    def clipping_amax(self, weight):
+        """``(amax, inner)`` -- one amax for every ``inner`` elements in a row of the contiguous matrix ``weight``,
+        or for all of them where ``inner`` is 0 -- when the backward of this quantizer is its gradient
+        where ``|weight| <= amax`` and zero elsewhere; None when it is not (or not that simply)."""
+        own = self.__dict__
+        if (type(self) is not TensorQuantizer or own["_disabled"] or not own["_if_quant"] or not own["_fake_quant"]
+                or own["_rotate"] or own["_if_calib"] or own["_pass_through_bwd"] or "_pre_quant_scale" in own["_buffers"]
+                or modes.strict_checks()):
+            return None
+        amax = own["_buffers"].get("_amax")
+        if amax is None or amax.device != weight.device or amax.dtype not in _hip._DTYPES or amax.dim() > 2:
+            return None
+        bs, bits = own["_block_sizes"], own["_num_bits"]
+        n, k = weight.shape
+        if bs is not None and bs.get("type") == "dynamic":
+            # the global amax of the two-level formats clips; power-of-two scales pass all gradients
+            return (amax.data, 0) if bs.get("scale_bits") != (8, 0) and amax.numel() == 1 else None
+        if type(bits) is not int and bits != (4, 3):
+            return None
+        if bs is None:
+            if amax.numel() == 1:
+                return amax.data, 0
+            return (amax.data, k) if tuple(amax.shape) == (n, 1) else None
+        block = bs.get(-1)
+        if (not block or any(isinstance(d, int) and d != -1 for d in bs) or k % block or amax.dim() != 2
+                or tuple(amax.shape) != (n * (k // block), 1)):
+            return None
+        return (amax.data, block) if amax.numel() > 1 else (amax.data, 0)
+
     # ------------------------------------------------------------------ representation / state
     def _short_amax(self, fmt=".4f"):
         if self.is_mx_format:
@@ -823,6 +852,12 @@ class TensorQuantizer(nn.Module):
             setattr(self, key, value)
         else:
             self.register_buffer(key, value)
+
+
+def quantizer_has_hooks(module) -> bool:
+    """Whether a hook looks at the calls of this module (its own or a global one)."""
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                or module._backward_pre_hooks or _module_hooks._has_any_global_hook())
 
 
 class SequentialQuantizer(nn.Sequential):

@@ -265,6 +265,55 @@ class DynamicBlockQuantizationFunction(Function):
         return _backward(ctx, grad_outputs, 9)
 
 
+class MaskedGradientLinear(Function):
+    """``F.linear(x, quantizer(weight), bias)`` for a weight quantizer whose backward keeps the gradient
+    where ``|weight| <= amax``: the weight gradient is computed and masked in one pass
+    (``_hip.wgrad_masked``) instead of written, read back with the weight and written again."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, quantizer, amax, inner):
+        quantized = quantizer(weight)          # grad mode is off here
+        ctx.save_for_backward(x, weight, quantized, amax)
+        ctx.inner, ctx.has_bias = inner, bias is not None
+        return torch.nn.functional.linear(x, quantized, bias)
+
+    @staticmethod
+    def backward(ctx, grad):
+        x, weight, quantized, amax = ctx.saved_tensors
+        n, k = weight.shape
+        if ctx.inner:
+            mask_amax = amax.reshape(n, k // ctx.inner, 1)
+        else:   # a 0-dim amax takes the type of the weight in the comparison, one with dims widens the weight
+            mask_amax = amax
+        narrow = amax.dim() == 0 and amax.dtype != weight.dtype
+        rows = grad.reshape(-1, n)
+        differentiated = torch.is_grad_enabled() and (grad.requires_grad or x.requires_grad or weight.requires_grad)
+        plain = not (differentiated or kernels.torch_is_intercepted() or type(grad) is not torch.Tensor
+                     or not torch._C._has_storage(grad))
+
+        def masked(w, g):
+            shape = (n, k // ctx.inner, ctx.inner) if ctx.inner else (n, k)
+            kept = torch.where(w.reshape(shape).abs() <= mask_amax, g.reshape(shape), g.new_zeros(1))
+            return kept.reshape(n, k)
+
+        grads = [None, None, None]
+        if ctx.needs_input_grad[0]:
+            used = quantized
+            if differentiated:   # its value, with the straight-through path back to the weight
+                used = quantized + masked(weight, weight - weight.detach())
+            grads[0] = (rows @ used).reshape(x.shape)
+        if ctx.needs_input_grad[1]:
+            x2 = x.reshape(-1, k)
+            if plain:
+                grads[1] = _hip.wgrad_masked(rows.contiguous(), x2.contiguous(), weight.detach(),
+                                             amax.reshape(-1).contiguous(), ctx.inner, narrow)
+            if grads[1] is None:
+                grads[1] = masked(weight, rows.t() @ x2)
+        if ctx.has_bias and ctx.needs_input_grad[2]:
+            grads[2] = rows.sum(0)
+        return (*grads, None, None, None)
+
+
 class _NoGraph:
     """Stands in for the autograd context when nothing will be differentiated."""
 
