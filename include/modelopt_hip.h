@@ -644,6 +644,12 @@ int mo_awq_clip_losses(const void* x, int64_t tokens, const void* w, int64_t n, 
                        const float* ratios, int n_ratios, int num_bits, int is_unsigned,
                        int narrow_range, float* loss, void* stream);
 
+/* What the loop over the clip ratios leaves (model_calib.py:958-966) from the stacked losses
+ * loss[n_ratios, blocks]: best_loss[b] the smallest (infinity if none is below it; a NaN never is), clip[b] =
+ * T(amax[b] * ratios[first index of it]), 0 where best_loss is infinite.  amax and clip of type dtype. */
+int mo_awq_best_clip(const float* loss, int64_t n_ratios, int64_t blocks, const float* ratios, const void* amax,
+                     int dtype, float* best_loss, void* clip, void* stream);
+
 /* acc[0] += sum of f32(T(a[i] - b[i]))^2 in double: the numerator of update_loss
  * (TQ/model_calib.py:623-627). */
 int mo_sq_diff_sum(const void* a, const void* b, int64_t n, int dtype, double* acc, void* stream);

@@ -77,6 +77,7 @@ SIGNATURES = {
     "mo_awq_scale_activations": [_P, _P, _I64, _I64, _I64, _INT, _P, _P],
     "mo_awq_search_losses": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _INT, _I64, _INT, _INT, _INT, _P, _P],
     "mo_awq_search_losses_biased": [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _INT, _I64, _INT, _INT, _INT, _P, _P],
+    "mo_awq_best_clip": [_P, _I64, _I64, _P, _P, _INT, _P, _P, _P],
     "mo_awq_clip_losses": [_P, _I64, _P, _I64, _I64, _INT, _I64, _P, _INT, _P, _INT, _INT, _INT, _INT, _P, _P],
     "mo_abs_colsum": [_P, _I64, _I64, _INT, _P, _I64, _P, _P],
     "mo_abs_colsum_staged": [_P, _I64, _I64, _INT, _P, _I64, _P, _P, _I64, _P],
@@ -856,6 +857,19 @@ def int4_pack_rows(w, ws, via_dtype=torch.float32):
     call("mo_int4_pack_rows_via", w, _ptr(w), batch, n, k, bs, dtype_code(w.dtype), _ptr(ws),
          dtype_code(via_dtype), _ptr(out), _stream(w))
     return out
+
+
+def awq_best_clip(loss: torch.Tensor, ratios: torch.Tensor, amax: torch.Tensor):
+    """``(best_loss, clip)``, shaped like ``amax``: per block the smallest of fp32 ``loss`` [ratios, blocks] and
+    ``amax * ratio`` for the first ratio that has it (zero where no loss is below infinity)."""
+    _require_device(loss, ratios, amax)
+    assert loss.dtype == ratios.dtype == torch.float32 and loss.is_contiguous() and amax.is_contiguous()
+    assert loss.numel() == ratios.numel() * amax.numel() and ratios.is_contiguous()
+    best = torch.empty(amax.shape, dtype=torch.float32, device=amax.device)
+    clip = torch.empty_like(amax)
+    call("mo_awq_best_clip", loss, _ptr(loss), ratios.numel(), amax.numel(), _ptr(ratios), _ptr(amax),
+         dtype_code(amax.dtype), _ptr(best), _ptr(clip), _stream(loss))
+    return best, clip
 
 
 def awq_pick_scale(loss: torch.Tensor, scales: torch.Tensor, dtype: torch.dtype):

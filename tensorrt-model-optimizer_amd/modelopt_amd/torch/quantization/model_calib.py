@@ -336,10 +336,11 @@ def _best_clip(helper):
     """``(best_loss, best_clip_val)`` as the reference's loop over the ratios leaves them
     (model_calib.py:958-966: a ratio replaces the running best when its loss is strictly smaller,
     so the first smallest loss wins, a NaN never does, and a block for which no loss is below
-    infinity keeps a clip value of zero) -- from the stacked losses in a handful of launches
-    instead of three per ratio."""
+    infinity keeps a clip value of zero) -- from the stacked losses in one launch on the device."""
     ratios = tuple(helper.loss)
     w_amax = helper.w_amax
+    if w_amax.is_cuda and w_amax.dtype in _hip._DTYPES and w_amax.is_contiguous():
+        return _hip.awq_best_clip(helper.loss_all, _ratio_column(ratios, w_amax.device), w_amax)
     loss = helper.loss_all.view(len(ratios), *w_amax.shape)
     inf = torch.full((), float("inf"), dtype=loss.dtype, device=loss.device)
     best_loss, index = torch.where(torch.isnan(loss), inf, loss).min(dim=0)

@@ -68,3 +68,22 @@ def test_shares_of_the_ratios_give_the_same_bits(dtype):
         assert torch.equal(_losses(w[rows].contiguous(), x, 16), whole[:, rows])
         one = _losses(w[rows].contiguous(), x, 16, ratios=RATIOS[3:4])
         assert torch.equal(one[0], whole[3, rows])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("ratios,blocks", [(1, 1), (11, 255), (11, 257), (3, 5000)])
+def test_best_clip_is_what_the_loop_over_the_ratios_leaves(dtype, ratios, blocks):
+    g = torch.Generator().manual_seed(blocks)
+    loss = torch.rand(ratios, blocks, generator=g).mul_(4).round_()      # many equal losses
+    loss[torch.rand(ratios, blocks, generator=g) < 0.2] = float("nan")
+    loss[torch.rand(ratios, blocks, generator=g) < 0.2] = float("inf")
+    loss[:, 0] = float("nan")
+    loss[:, -1] = float("inf") if blocks > 1 else loss[:, -1]
+    amax, table = torch.rand(blocks, 1, generator=g).to(dtype), torch.linspace(0.5, 1, ratios)
+    best, clip = torch.full((blocks, 1), float("inf")), torch.zeros(blocks, 1, dtype=dtype)
+    for r in range(ratios):
+        better = loss[r].view(-1, 1) < best
+        best = torch.where(better, loss[r].view(-1, 1), best)
+        clip = torch.where(better, (amax.float() * table[r]).to(dtype), clip)
+    got_best, got_clip = _hip.awq_best_clip(loss.to("cuda"), table.to("cuda"), amax.to("cuda"))
+    assert torch.equal(got_best.cpu(), best) and torch.equal(got_clip.cpu(), clip)
