@@ -67,6 +67,47 @@ __device__ __forceinline__ float clip_qdq_fast(const IntOp& op, float v, const I
     return exact_quotient_short(q, s.div, s.rdiv);
 }
 
+// A selection by zeros does not select among products that are not finite: inf * 0 is NaN in every sum of
+// its matrix row, the sums of other weight rows among them.  Any such sum ends the quick form of a
+// wavefront before the losses of that step are written, and the careful form goes on from there: over
+// the products of a step twice, once for their kinds and once without those that are not finite, so that
+// the rows without any get the bits they would have alone.  A kind is a power of two whose sums over a block
+// (128 at most of each) stay apart in 24 bits; two words of 16 bits at a time, E the exponent mask of the type.
+// The forms come one after the other, not one within the other, which would cost the quick one registers.
+struct ClipStep {
+    int token, ratio;   // first token of the pass, index of the ratio (that of the unclipped block: before the first)
+};
+
+template <uint32_t E, uint32_t POS, uint32_t NEG, uint32_t NAN_>
+__device__ __forceinline__ uint32_t clip_kinds(uint32_t w, bool kinds) {
+    uint32_t out = 0;
+#pragma unroll
+    for (int h = 0; h < 32; h += 16) {
+        const uint32_t v = (w >> h) & 0xFFFFu;
+        const bool finite = (v & E) != E;
+        const uint32_t kind = (v & 0x7FFFu) != E ? NAN_ : (v & 0x8000u) ? NEG : POS;
+        out |= (kinds ? (finite ? 0u : kind) : (finite ? v : 0u)) << h;
+    }
+    return out;
+}
+// 2^-8 for +inf, 1 for -inf, 2^8 for NaN
+__device__ __forceinline__ uint32_t clip_kinds_bf16(uint32_t w, bool kinds) {
+    return clip_kinds<0x7F80u, 0x3B80u, 0x3F80u, 0x4380u>(w, kinds);
+}
+__device__ __forceinline__ uint32_t clip_kinds_f16(uint32_t w, bool kinds) {
+    return clip_kinds<0x7C00u, 0x1C00u, 0x3C00u, 0x5C00u>(w, kinds);
+}
+// The sum of the products without those, given the kinds among them: 0 none, 1 +inf, 2 -inf, 3 NaN or both
+__device__ __forceinline__ uint32_t clip_sum_kind(float kinds) {
+    const uint32_t c = (uint32_t)(kinds * 256.0f);
+    const uint32_t k = ((c & 0xFFu) ? 1u : 0u) | ((c & 0xFF00u) ? 2u : 0u);
+    return c >> 16 ? 3u : k;
+}
+__device__ __forceinline__ float clip_with_kind(float sum, uint32_t kind) {
+    const uint32_t special = kind == 3 ? 0x7FC00000u : 0x7F800000u | (kind & 2u) << 30;
+    return kind ? u2f(special) : sum;
+}
+
 // ------------------------------------------------------------------------------------- bf16
 // A wavefront owns 32 rows of one weight block and all tokens of a pass, in two tiles of 32.  For two
 // columns (j, j + 8) of the block, v_mfma_f32_32x32x4_2b_bf16 with the tokens as A, reduced to one of
@@ -80,19 +121,19 @@ __device__ __forceinline__ float clip_qdq_fast(const IntOp& op, float v, const I
 // of the tile.  The partial outputs of the unclipped block stay in registers in the same places.
 // The weights are quantised as they are used, 16 columns at a time, by the lane that supplies them to
 // the matrix instruction; no LDS and no barrier anywhere.
-template <int BS>
-__device__ __forceinline__ void clip_losses_bf16(const uint16_t* __restrict__ x, int tokens,
+template <int BS, bool CAREFUL>
+__device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x, int tokens,
                                                  const uint16_t* __restrict__ w, int n, int k,
                                                  const void* __restrict__ w_amax, int amax_dtype,
                                                  const ClipRatios& ratios, int r0, int r1,
-                                                 const IntOp& op, float* __restrict__ loss) {
+                                                 const IntOp& op, float* __restrict__ loss, ClipStep& at) {
     constexpr int NC = BS / 16;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fr = lane & 31, kg = lane >> 5;
     const int nblk = k / BS, b = blockIdx.y;
     const int row0 = (blockIdx.x * kClipWaves + wave) * 32;
-    if (row0 >= n) return;
+    if (row0 >= n) return true;
     int row = row0 + fr < n ? row0 + fr : n - 1;
     const float amax = load_scalar(w_amax, amax_dtype, (int64_t)row * nblk + b);
     bf16x8_t pair_sum;
@@ -105,7 +146,7 @@ __device__ __forceinline__ void clip_losses_bf16(const uint16_t* __restrict__ x,
     f32x32_t zero;
 #pragma unroll
     for (int i = 0; i < 32; ++i) zero[i] = 0.0f;
-    for (int t0 = 0; t0 < tokens; t0 += kClipTokens) {
+    for (int t0 = CAREFUL ? __builtin_amdgcn_readfirstlane(at.token) : 0; t0 < tokens; t0 += kClipTokens) {
         int xrow[2];
         bool live[2];   // a token past the end counts as a row of zeros
 #pragma unroll
@@ -127,6 +168,7 @@ __device__ __forceinline__ void clip_losses_bf16(const uint16_t* __restrict__ x,
         fetch(0);
         uint32_t org[2][8];   // rounded partial outputs of the unclipped block, two a word
         for (int v = r0 - 1; v < r1; ++v) {   // r0 - 1: the unclipped block
+            if (CAREFUL && v >= r0 && t0 == at.token && v < at.ratio) continue;   // in the losses already
             IntOp::Scale s = {};
             if (v >= r0) s = clip_scale(op, amax, amax_dtype, ratios.r[v]);
             f32x4 acc[2][4];
@@ -134,9 +176,9 @@ __device__ __forceinline__ void clip_losses_bf16(const uint16_t* __restrict__ x,
             for (int m = 0; m < 2; ++m)
 #pragma unroll
                 for (int a = 0; a < 4; ++a) acc[m][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-            for (int c = 0; c < NC; ++c) {
-                uint32_t wb[4] = {wraw.x, wraw.y, wraw.z, wraw.w};
+            // the operands of the chunk that was fetched: the weights quantised, the tokens that exist
+            auto operands = [&](uint32_t (&wb)[4], uint32_t (&xb)[2][4]) {
+                wb[0] = wraw.x, wb[1] = wraw.y, wb[2] = wraw.z, wb[3] = wraw.w;
                 if (v >= r0) {
                     float q[8];
 #pragma unroll
@@ -156,7 +198,6 @@ __device__ __forceinline__ void clip_losses_bf16(const uint16_t* __restrict__ x,
 #pragma unroll
                     for (int j = 0; j < 4; ++j) wb[j] = f32x2_to_bf16x2(q[2 * j], q[2 * j + 1]);
                 }
-                uint32_t xb[2][4];
 #pragma unroll
                 for (int m = 0; m < 2; ++m) {
                     xb[m][0] = live[m] ? xraw[m].x : 0u;
@@ -164,36 +205,96 @@ __device__ __forceinline__ void clip_losses_bf16(const uint16_t* __restrict__ x,
                     xb[m][2] = live[m] ? xraw[m].z : 0u;
                     xb[m][3] = live[m] ? xraw[m].w : 0u;
                 }
-                fetch(c + 1 < NC ? c + 1 : 0);   // the first one again for the next ratio
-                auto products = [&](int q) {   // column q & 7 of either half of the chunk, tile q >> 3
-                    const int m = q >> 3, e = q & 7;
-                    const uint32_t one = xb[m][e >> 1] & ((e & 1) ? 0xFFFF0000u : 0x0000FFFFu);
-                    const uint32_t aw[2] = {(e & 2) ? 0u : one, (e & 2) ? one : 0u};
-                    const uint32_t bw[2] = {wb[(e >> 2) * 2], wb[(e >> 2) * 2 + 1]};
-                    s16x4_t av, bv;
-                    __builtin_memcpy(&av, aw, 8);
-                    __builtin_memcpy(&bv, bw, 8);
-                    return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(av, bv, zero, 0, 0, 0);
-                };
-                f32x32_t d = products(0);
+            };
+            // column q & 7 of either half of the chunk, tile q >> 3
+            auto products = [&](const uint32_t (&wb)[4], const uint32_t (&xb)[2][4], int q) {
+                const int m = q >> 3, e = q & 7;
+                const uint32_t one = xb[m][e >> 1] & ((e & 1) ? 0xFFFF0000u : 0x0000FFFFu);
+                const uint32_t aw[2] = {(e & 2) ? 0u : one, (e & 2) ? one : 0u};
+                const uint32_t bw[2] = {wb[(e >> 2) * 2], wb[(e >> 2) * 2 + 1]};
+                s16x4_t av, bv;
+                __builtin_memcpy(&av, aw, 8);
+                __builtin_memcpy(&bv, bw, 8);
+                return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(av, bv, zero, 0, 0, 0);
+            };
+            if constexpr (CAREFUL) {
+                uint32_t kind[2] = {0, 0};   // two bits an output
+#pragma unroll 1
+                for (int pass = 0; pass < 2; ++pass) {
 #pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    f32x32_t ahead;   // the next products run under this step's conversions
-                    if (q + 1 < 16) ahead = products(q + 1);
-                    __builtin_amdgcn_sched_barrier(0);
+                    for (int m = 0; m < 2; ++m)
 #pragma unroll
-                    for (int a = 0; a < 4; ++a) {
-                        uint32_t pw[4];
+                        for (int a = 0; a < 4; ++a) acc[m][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+                    for (int c = 0; c < NC; ++c) {
+                        uint32_t wb[4], xb[2][4];
+                        fetch(c);
+                        operands(wb, xb);
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) pw[i] = f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]);
-                        bf16x8_t pv;
-                        __builtin_memcpy(&pv, pw, 16);
-                        acc[q >> 3][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pv, pair_sum, acc[q >> 3][a], 0, 0, 0);
+                        for (int q = 0; q < 16; ++q) {
+                            const f32x32_t d = products(wb, xb, q);
+#pragma unroll
+                            for (int a = 0; a < 4; ++a) {
+                                uint32_t pw[4];
+#pragma unroll
+                                for (int i = 0; i < 4; ++i)
+                                    pw[i] = clip_kinds_bf16(f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]), pass == 0);
+                                bf16x8_t pv;
+                                __builtin_memcpy(&pv, pw, 16);
+                                acc[q >> 3][a] =
+                                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(pv, pair_sum, acc[q >> 3][a], 0, 0, 0);
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
                     }
-                    if (q + 1 < 16) d = ahead;
-                    // Steps stay apart: left alone, the scheduler converts the first of the products
-                    // ahead within this step and waits out the matrix instruction that makes them.
-                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int m = 0; m < 2; ++m)
+#pragma unroll
+                        for (int a = 0; a < 4; ++a)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const int bit = 2 * (4 * a + i);
+                                if (pass == 0) kind[m] |= clip_sum_kind(acc[m][a][i]) << bit;
+                                else acc[m][a][i] = clip_with_kind(acc[m][a][i], (kind[m] >> bit) & 3u);
+                            }
+                }
+            } else {
+#pragma unroll 1
+                for (int c = 0; c < NC; ++c) {
+                    uint32_t wb[4], xb[2][4];
+                    operands(wb, xb);
+                    fetch(c + 1 < NC ? c + 1 : 0);   // the first one again for the next ratio
+                    f32x32_t d = products(wb, xb, 0);
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) {
+                        f32x32_t ahead;   // the next products run under this step's conversions
+                        if (q + 1 < 16) ahead = products(wb, xb, q + 1);
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int a = 0; a < 4; ++a) {
+                            uint32_t pw[4];
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) pw[i] = f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]);
+                            bf16x8_t pv;
+                            __builtin_memcpy(&pv, pw, 16);
+                            acc[q >> 3][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pv, pair_sum, acc[q >> 3][a], 0, 0, 0);
+                        }
+                        if (q + 1 < 16) d = ahead;
+                        // Steps stay apart: left alone, the scheduler converts the first of the products
+                        // ahead within this step and waits out the matrix instruction that makes them.
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                bool lost = false;
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+#pragma unroll
+                    for (int a = 0; a < 4; ++a)
+#pragma unroll
+                        for (int i = 0; i < 4; i += 2) lost |= __builtin_isunordered(acc[m][a][i], acc[m][a][i + 1]);
+                if (__any(lost)) {
+                    at = {t0, v};
+                    return false;
                 }
             }
             if (v < r0) {
@@ -236,6 +337,7 @@ __device__ __forceinline__ void clip_losses_bf16(const uint16_t* __restrict__ x,
             }
         }
     }
+    return true;
 }
 
 // ------------------------------------------------------------------------------------- fp16
@@ -244,19 +346,19 @@ __device__ __forceinline__ void clip_losses_bf16(const uint16_t* __restrict__ x,
 // two rounded products; the words of four tokens are an A operand of v_mfma_f32_16x16x32_f16 and are
 // summed as in the bf16 form: lane l, register i holds row 4 (l >> 4) + i + 16 ((l >> 2) & 3), token
 // l & 3 of the four.  The partial outputs of the unclipped block stay in LDS.
-template <int BS>
-__device__ __forceinline__ void clip_losses_f16(const uint16_t* __restrict__ x, int tokens,
+template <int BS, bool CAREFUL>
+__device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, int tokens,
                                                 const uint16_t* __restrict__ w, int n, int k,
                                                 const void* __restrict__ w_amax, int amax_dtype,
                                                 const ClipRatios& ratios, int r0, int r1, const IntOp& op,
-                                                float* __restrict__ loss, u32x2* __restrict__ org) {
+                                                float* __restrict__ loss, u32x2* __restrict__ org, ClipStep& at) {
     constexpr int GW = 4;            // words of a token read ahead together (8 columns)
     constexpr int NG = BS / 2 / GW;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nblk = k / BS, b = blockIdx.y;
     const int row0 = (blockIdx.x * kClipWaves + wave) * kClipLanes;
-    if (row0 >= n) return;
+    if (row0 >= n) return true;
     org += (size_t)wave * (kClipTokens / 4) * kClipLanes + lane;
     const int row = row0 + lane < n ? row0 + lane : n - 1;
     const uint16_t* wp = w + (int64_t)row * k + b * BS;
@@ -271,9 +373,19 @@ __device__ __forceinline__ void clip_losses_f16(const uint16_t* __restrict__ x, 
     const uint32_t* xw = (const uint32_t*)(x + b * BS);
     const int xstride = k / 2;
     uint32_t wq[BS / 2];
-    for (int t0 = 0; t0 < tokens; t0 += kClipTokens) {
+    auto product = [](uint32_t xs, uint32_t ws) {   // of two pairs, each rounded
+        f16x2_t a, c;
+        __builtin_memcpy(&a, &xs, 4);
+        __builtin_memcpy(&c, &ws, 4);
+        const f16x2_t p = a * c;
+        uint32_t out;
+        __builtin_memcpy(&out, &p, 4);
+        return out;
+    };
+    for (int t0 = CAREFUL ? __builtin_amdgcn_readfirstlane(at.token) : 0; t0 < tokens; t0 += kClipTokens) {
         const int tc = tokens - t0 < kClipTokens ? tokens - t0 : kClipTokens;
         for (int v = r0 - 1; v < r1; ++v) {   // r0 - 1: the unclipped block
+            if (CAREFUL && v >= r0 && t0 == at.token && v < at.ratio) continue;   // in the losses already
             IntOp::Scale s = {};
             if (v >= r0) s = clip_scale(op, amax, amax_dtype, ratios.r[v]);
             // opaque to the optimiser, which would otherwise keep the block live beside its
@@ -310,6 +422,7 @@ __device__ __forceinline__ void clip_losses_f16(const uint16_t* __restrict__ x, 
                     }
                 }
             }
+            bool lost = false;
             float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
             for (int g4 = 0; g4 * 4 < tc; ++g4) {
                 const uint32_t* xr[4];   // past the end: the last token again, left out below
@@ -319,47 +432,72 @@ __device__ __forceinline__ void clip_losses_f16(const uint16_t* __restrict__ x, 
                     xr[i] = xw + (int64_t)(t0 + t) * xstride;
                 }
                 f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
-                uint32_t cur[4][GW];
+                f32x4 total;
+                if constexpr (CAREFUL) {
+                    uint32_t kind[4] = {0, 0, 0, 0};
+#pragma unroll 1
+                    for (int pass = 0; pass < 2; ++pass) {
+                        acc[0] = acc[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                        for (int j = 0; j < BS / 2; ++j) {
+                            // opaque, or the products would be kept from one pass for the other and the
+                            // activations be read many steps ahead
+                            int at_j = j;
+                            asm volatile("" : "+s"(at_j));
+                            uint32_t pw[4];
 #pragma unroll
-                    for (int j = 0; j < GW; ++j) cur[i][j] = xr[i][j];
-#pragma unroll
-                for (int g = 0; g < NG; ++g) {
-                    uint32_t next[4][GW];
-                    if (g + 1 < NG) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-#pragma unroll
-                            for (int j = 0; j < GW; ++j) next[i][j] = xr[i][GW * (g + 1) + j];
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int j = 0; j < GW; ++j) {
-                        uint32_t pw[4];
+                            for (int i = 0; i < 4; ++i) pw[i] = clip_kinds_f16(product(xr[i][at_j], wq[j]), pass == 0);
+                            f16x8_t pv;
+                            __builtin_memcpy(&pv, pw, 16);
+                            acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pv, pair_sum, acc[j & 1], 0, 0, 0);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                        total = acc[0] + acc[1];
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            f16x2_t a, c;
-                            __builtin_memcpy(&a, &cur[i][j], 4);
-                            __builtin_memcpy(&c, &wq[GW * g + j], 4);
-                            const f16x2_t p = a * c;
-                            __builtin_memcpy(&pw[i], &p, 4);
+                            if (pass == 0) kind[i] = clip_sum_kind(total[i]);
+                            else total[i] = clip_with_kind(total[i], kind[i]);
                         }
-                        f16x8_t pv;
-                        __builtin_memcpy(&pv, pw, 16);
-                        acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pv, pair_sum, acc[j & 1], 0, 0, 0);
                     }
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (g + 1 < NG) {
+                } else {
+                    uint32_t cur[4][GW];
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
+                    for (int i = 0; i < 4; ++i)
 #pragma unroll
-                            for (int j = 0; j < GW; ++j) cur[i][j] = next[i][j];
+                        for (int j = 0; j < GW; ++j) cur[i][j] = xr[i][j];
+#pragma unroll
+                    for (int g = 0; g < NG; ++g) {
+                        uint32_t next[4][GW];
+                        if (g + 1 < NG) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                                for (int j = 0; j < GW; ++j) next[i][j] = xr[i][GW * (g + 1) + j];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int j = 0; j < GW; ++j) {
+                            uint32_t pw[4];
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) pw[i] = product(cur[i][j], wq[GW * g + j]);
+                            f16x8_t pv;
+                            __builtin_memcpy(&pv, pw, 16);
+                            acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pv, pair_sum, acc[j & 1], 0, 0, 0);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (g + 1 < NG) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                                for (int j = 0; j < GW; ++j) cur[i][j] = next[i][j];
+                        }
                     }
+                    total = acc[0] + acc[1];
+                    lost |= __builtin_isunordered(total[0], total[1]) | __builtin_isunordered(total[2], total[3]);
                 }
                 float out[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) out[i] = clip_round<MO_F16>(acc[0][i] + acc[1][i]);
+                for (int i = 0; i < 4; ++i) out[i] = clip_round<MO_F16>(total[i]);
                 if (v < r0) {
                     u32x2 o;
                     o.x = f32_to_f16_bits(out[0]) | (f32_to_f16_bits(out[1]) << 16);
@@ -377,6 +515,10 @@ __device__ __forceinline__ void clip_losses_f16(const uint16_t* __restrict__ x, 
                     }
                 }
             }
+            if (!CAREFUL && __any(lost)) {
+                at = {t0, v};
+                return false;
+            }
             if (v < r0) continue;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {   // the other tokens of the rows: lane bits 0 and 1
@@ -392,6 +534,7 @@ __device__ __forceinline__ void clip_losses_f16(const uint16_t* __restrict__ x, 
             }
         }
     }
+    return true;
 }
 
 // ------------------------------------------------------------------------------------- fp32
@@ -532,13 +675,20 @@ __global__ __launch_bounds__(kClipLanes * kClipWaves, DT == MO_BF16 ? 3 : 2) voi
     extern __shared__ __align__(16) unsigned char clip_smem[];
     const int r0 = (int)(blockIdx.z * (unsigned)ratios.count / gridDim.z);
     const int r1 = (int)((blockIdx.z + 1) * (unsigned)ratios.count / gridDim.z);
-    if constexpr (DT == MO_BF16)
-        clip_losses_bf16<BS>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype, ratios,
-                             r0, r1, op, loss);
-    else if constexpr (DT == MO_F16)
-        clip_losses_f16<BS>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype, ratios,
-                            r0, r1, op, loss, (u32x2*)clip_smem);
-    else
+    if constexpr (DT == MO_BF16) {
+        ClipStep at;
+        if (!clip_losses_bf16<BS, false>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype,
+                                         ratios, r0, r1, op, loss, at))
+            clip_losses_bf16<BS, true>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype,
+                                       ratios, r0, r1, op, loss, at);
+    } else if constexpr (DT == MO_F16) {
+        ClipStep at;
+        u32x2* org = (u32x2*)clip_smem;
+        if (!clip_losses_f16<BS, false>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype,
+                                        ratios, r0, r1, op, loss, org, at))
+            clip_losses_f16<BS, true>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype,
+                                      ratios, r0, r1, op, loss, org, at);
+    } else
         clip_losses_f32<BS>((const float*)x, tokens, (const float*)w, n, k, w_amax, amax_dtype, ratios, r0, r1,
                             op, loss, (float*)clip_smem);
 }

@@ -1,6 +1,6 @@
 """The 16-bit clip search at the edges of its tiles: 32 rows (bf16) or 64 rows (fp16) per wavefront, tiles
 of 32 tokens or groups of 4, passes of 64, shares of the ratios, codes too wide for the short
-quotient, blocks whose scale leaves the range of the reciprocal."""
+quotient, blocks whose scale leaves the range of the reciprocal, products that overflow."""
 
 import pytest
 import torch
@@ -68,6 +68,40 @@ def test_shares_of_the_ratios_give_the_same_bits(dtype):
         assert torch.equal(_losses(w[rows].contiguous(), x, 16), whole[:, rows])
         one = _losses(w[rows].contiguous(), x, 16, ratios=RATIOS[3:4])
         assert torch.equal(one[0], whole[3, rows])
+
+
+# rows in the first and the last place of a tile and in the part of one at the end, tokens in the first and a
+# later pass and in the part of a group at the end
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("kind", ["overflow", "clipped_overflow", "both_signs", "inf", "nan"])
+@pytest.mark.parametrize("n,k,tokens,block,rows,token", [
+    (96, 64, 8, 32, (21,), 3), (129, 128, 66, 128, (0, 63, 128), 65), (70, 32, 70, 16, (5, 37, 64), 31), (64, 64, 1, 64, (33,), 0)])
+def test_a_row_that_is_not_finite_leaves_the_others_alone(dtype, kind, n, k, tokens, block, rows, token):
+    """Products of finite values that overflow, and weights that are not finite: the losses of all other rows
+    are to the bit those of the same weight without them, and the row's own are what the CPU makes of it."""
+    w, x = _case(n, k, tokens, dtype, n)
+    clean, col = w.clone(), k - 3
+    # times 4096 past 65504, times 64 past 2^128; the last one only where clipping widens it (code -8 of 7)
+    scale, x_large = (1.0, 4096.0) if dtype == torch.float16 else (2.0 ** 118, 64.0)
+    values = {"overflow": (0.0, 20.0), "both_signs": (-20.0, 20.0), "clipped_overflow": (0.0, -15.875)}
+    for r in rows:
+        w[r, col - 1:col + 1] = torch.tensor(values[kind]) * scale if kind in values else float(kind)
+        clean[r, col - 1:col + 1] = 0.0
+    if kind in values:
+        x[token, col - 1:col + 1] = x_large
+    got, other = _losses(w, x, block), _losses(clean, x, block)
+    want, _ = oawq.awq_clip_search(w, [x], block, 4, max_tokens_per_batch=1 << 20)
+    healthy = torch.ones(n, dtype=torch.bool)
+    healthy[list(rows)] = False
+    assert torch.isfinite(other[:, healthy]).all() and torch.equal(got[:, healthy], other[:, healthy])
+    assert torch.equal(got[:, :, :col // block], other[:, :, :col // block])      # the other blocks of the row
+    for i, r in enumerate(RATIOS):
+        mine, cpu = got[i][~healthy][:, col // block], want[r][~healthy][:, col // block]
+        assert kind == "clipped_overflow" or not torch.isfinite(cpu).any()
+        assert torch.equal(mine.isnan(), cpu.isnan()) and torch.equal(mine.isinf(), cpu.isinf()), r
+        # what is finite and large is one token's error, above 1700: two outputs in steps of 32
+        large = torch.isfinite(cpu) & (cpu * tokens > 3e6)
+        torch.testing.assert_close(mine[large], cpu[large], rtol=0.08, atol=0.0)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
