@@ -20,6 +20,11 @@
 //   fp16: v_pk_mul_f16 rounds two products at once, sums on the matrix cores (clip_losses_f16): 0.5
 //         vector instructions per product where multiply, round and add took about 4.
 //   fp32: no rounding to do, one multiply and one add per product (clip_losses_f32).
+// The instruction adds a pair of products to an output with one rounding, as v_dot2c does.  Its sums are made
+// in chains of a quarter of a block (but for blocks of 16), as four chains of v_dot2c made them: one
+// chain through a block of 128 rounds at twice the magnitude, and measured against sums in 64 bits 41 % more
+// blocks had an output that fell on the other side of a rounding to bf16 (1199 of 1.57 million; 852 with
+// quarters, 856 with v_dot2c).  What that costs: bf16 blocks of 128 3 %, of 64 and of 32 5 %.
 // Measured figures stand at the launch below.
 #include "common.h"
 #include "qdq_ops.h"
@@ -118,16 +123,20 @@ __device__ __forceinline__ float clip_with_kind(float sum, uint32_t kind) {
 // B operand, constant through the kernel, sends pair p to output column p, so the instruction adds
 // lo + hi of each of the 64 x 4 words to a sum of its own: lane l, register i of group a holds
 //   row 4 (l >> 4) + i + 16 ((l >> 2) & 1), token 8 a + 4 ((l >> 3) & 1) + (l & 3)
-// of the tile.  The partial outputs of the unclipped block stay in registers in the same places.
-// The weights are quantised as they are used, 16 columns at a time, by the lane that supplies them to
-// the matrix instruction; no LDS and no barrier anywhere.
+// of the tile.  The sums of the chains that have ended and the partial outputs of the unclipped block lie in
+// LDS, each lane's own: no barrier anywhere.  Folding stands where the products before it are used up, or
+// its operands would not fit the registers.  The weights are quantised as they are used, 16 columns at a
+// time, by the lane that supplies them to the matrix instruction.
 template <int BS, bool CAREFUL>
 __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x, int tokens,
                                                  const uint16_t* __restrict__ w, int n, int k,
                                                  const void* __restrict__ w_amax, int amax_dtype,
                                                  const ClipRatios& ratios, int r0, int r1,
-                                                 const IntOp& op, float* __restrict__ loss, ClipStep& at) {
+                                                 const IntOp& op, float* __restrict__ loss,
+                                                 f32x4* __restrict__ parts, u32x2* __restrict__ org, ClipStep& at) {
     constexpr int NC = BS / 16;
+    constexpr int HALVES = BS >= 32 ? BS / 32 : 2;   // of a chunk, in a chain of sums
+    constexpr int RUN = HALVES >= 2 ? HALVES / 2 : 1;   // chunks until the chains of both tiles have ended
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fr = lane & 31, kg = lane >> 5;
@@ -166,16 +175,28 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
             for (int m = 0; m < 2; ++m) xraw[m] = *(const u32x4*)(x + ((int64_t)xrow[m] * k + col));
         };
         fetch(0);
-        uint32_t org[2][8];   // rounded partial outputs of the unclipped block, two a word
         for (int v = r0 - 1; v < r1; ++v) {   // r0 - 1: the unclipped block
             if (CAREFUL && v >= r0 && t0 == at.token && v < at.ratio) continue;   // in the losses already
             IntOp::Scale s = {};
             if (v >= r0) s = clip_scale(op, amax, amax_dtype, ratios.r[v]);
             f32x4 acc[2][4];
+            auto clear = [&]() {
 #pragma unroll
-            for (int m = 0; m < 2; ++m)
+                for (int m = 0; m < 2; ++m)
 #pragma unroll
-                for (int a = 0; a < 4; ++a) acc[m][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    for (int a = 0; a < 4; ++a) parts[(4 * m + a) * 64] = acc[m][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            };
+            // the end of the chains: their sums go to those of the chains before them
+            auto fold = [&]() {
+                if (HALVES == 2 * NC) return;
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) {
+                        acc[m][a] = parts[(4 * m + a) * 64] + acc[m][a];
+                        parts[(4 * m + a) * 64] = acc[m][a];
+                    }
+            };
             // the operands of the chunk that was fetched: the weights quantised, the tokens that exist
             auto operands = [&](uint32_t (&wb)[4], uint32_t (&xb)[2][4]) {
                 wb[0] = wraw.x, wb[1] = wraw.y, wb[2] = wraw.z, wb[3] = wraw.w;
@@ -206,9 +227,10 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                     xb[m][3] = live[m] ? xraw[m].w : 0u;
                 }
             };
-            // column q & 7 of either half of the chunk, tile q >> 3
+            // Step q of a chunk: four columns of its lower half and the same of its upper half, of either
+            // tile of tokens in turn, then the other four
             auto products = [&](const uint32_t (&wb)[4], const uint32_t (&xb)[2][4], int q) {
-                const int m = q >> 3, e = q & 7;
+                const int m = (q >> 2) & 1, e = (q >> 3) * 4 + (q & 3);
                 const uint32_t one = xb[m][e >> 1] & ((e & 1) ? 0xFFFF0000u : 0x0000FFFFu);
                 const uint32_t aw[2] = {(e & 2) ? 0u : one, (e & 2) ? one : 0u};
                 const uint32_t bw[2] = {wb[(e >> 2) * 2], wb[(e >> 2) * 2 + 1]};
@@ -217,14 +239,17 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                 __builtin_memcpy(&bv, bw, 8);
                 return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(av, bv, zero, 0, 0, 0);
             };
+            auto sum_words = [&](const uint32_t (&pw)[4], int m, int a, bool opens) {
+                bf16x8_t pv;
+                __builtin_memcpy(&pv, pw, 16);
+                const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+                acc[m][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pv, pair_sum, opens ? none : acc[m][a], 0, 0, 0);
+            };
             if constexpr (CAREFUL) {
                 uint32_t kind[2] = {0, 0};   // two bits an output
 #pragma unroll 1
                 for (int pass = 0; pass < 2; ++pass) {
-#pragma unroll
-                    for (int m = 0; m < 2; ++m)
-#pragma unroll
-                        for (int a = 0; a < 4; ++a) acc[m][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    clear();
 #pragma unroll 1
                     for (int c = 0; c < NC; ++c) {
                         uint32_t wb[4], xb[2][4];
@@ -232,19 +257,20 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                         operands(wb, xb);
 #pragma unroll
                         for (int q = 0; q < 16; ++q) {
+                            const int m = (q >> 2) & 1;
+                            const bool opens = (c * 2 + (q >> 3)) % HALVES == 0 && (q & 3) == 0;
                             const f32x32_t d = products(wb, xb, q);
 #pragma unroll
                             for (int a = 0; a < 4; ++a) {
+                                if (opens) acc[m][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                                 uint32_t pw[4];
 #pragma unroll
                                 for (int i = 0; i < 4; ++i)
                                     pw[i] = clip_kinds_bf16(f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]), pass == 0);
-                                bf16x8_t pv;
-                                __builtin_memcpy(&pv, pw, 16);
-                                acc[q >> 3][a] =
-                                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(pv, pair_sum, acc[q >> 3][a], 0, 0, 0);
+                                sum_words(pw, m, a, false);
                             }
                             __builtin_amdgcn_sched_barrier(0);
+                            if ((c * 2 + (q >> 3)) % HALVES == HALVES - 1 && (q & 7) == 7) fold();
                         }
                     }
 #pragma unroll
@@ -259,62 +285,66 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                             }
                 }
             } else {
+                clear();
 #pragma unroll 1
-                for (int c = 0; c < NC; ++c) {
-                    uint32_t wb[4], xb[2][4];
-                    operands(wb, xb);
-                    fetch(c + 1 < NC ? c + 1 : 0);   // the first one again for the next ratio
-                    f32x32_t d = products(wb, xb, 0);
+                for (int c = 0; c < NC; c += RUN) {
 #pragma unroll
-                    for (int q = 0; q < 16; ++q) {
-                        f32x32_t ahead;   // the next products run under this step's conversions
-                        if (q + 1 < 16) ahead = products(wb, xb, q + 1);
-                        __builtin_amdgcn_sched_barrier(0);
+                    for (int cc = 0; cc < RUN; ++cc) {
+                        uint32_t wb[4], xb[2][4];
+                        operands(wb, xb);
+                        f32x32_t d = products(wb, xb, 0);
 #pragma unroll
-                        for (int a = 0; a < 4; ++a) {
-                            uint32_t pw[4];
+                        for (int q = 0; q < 16; ++q) {
+                            const int m = (q >> 2) & 1, half = cc * 2 + (q >> 3);
+                            f32x32_t ahead;   // the next products run under this step's conversions
+                            if (q + 1 < 16) ahead = products(wb, xb, q + 1);
+                            // half a chunk ahead; the first one again for the next ratio
+                            if (q == 8) fetch(c + cc + 1 < NC ? c + cc + 1 : 0);
+                            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) pw[i] = f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]);
-                            bf16x8_t pv;
-                            __builtin_memcpy(&pv, pw, 16);
-                            acc[q >> 3][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pv, pair_sum, acc[q >> 3][a], 0, 0, 0);
+                            for (int a = 0; a < 4; ++a) {
+                                uint32_t pw[4];
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) pw[i] = f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]);
+                                sum_words(pw, m, a, half % HALVES == 0 && (q & 3) == 0);
+                            }
+                            if (q + 1 < 16) d = ahead;
+                            // Steps stay apart: left alone, the scheduler converts the first of the products
+                            // ahead within this step and waits out the matrix instruction that makes them.
+                            __builtin_amdgcn_sched_barrier(0);
+                            if (half % HALVES == HALVES - 1 && (q & 7) == 7) fold();
                         }
-                        if (q + 1 < 16) d = ahead;
-                        // Steps stay apart: left alone, the scheduler converts the first of the products
-                        // ahead within this step and waits out the matrix instruction that makes them.
-                        __builtin_amdgcn_sched_barrier(0);
                     }
                 }
-                bool lost = false;
-#pragma unroll
-                for (int m = 0; m < 2; ++m)
-#pragma unroll
-                    for (int a = 0; a < 4; ++a)
-#pragma unroll
-                        for (int i = 0; i < 4; i += 2) lost |= __builtin_isunordered(acc[m][a][i], acc[m][a][i + 1]);
-                if (__any(lost)) {
-                    at = {t0, v};
-                    return false;
-                }
             }
+            bool lost = false;
             if (v < r0) {
 #pragma unroll
                 for (int m = 0; m < 2; ++m)
 #pragma unroll
                     for (int a = 0; a < 4; ++a) {
-                        org[m][2 * a] = f32x2_to_bf16x2(acc[m][a][0], acc[m][a][1]);
-                        org[m][2 * a + 1] = f32x2_to_bf16x2(acc[m][a][2], acc[m][a][3]);
+                        lost |= __builtin_isunordered(acc[m][a][0], acc[m][a][1]) |
+                                __builtin_isunordered(acc[m][a][2], acc[m][a][3]);
+                        u32x2 o;
+                        o.x = f32x2_to_bf16x2(acc[m][a][0], acc[m][a][1]);
+                        o.y = f32x2_to_bf16x2(acc[m][a][2], acc[m][a][3]);
+                        org[(4 * m + a) * 64] = o;
                     }
+                if (!CAREFUL && __any(lost)) {
+                    at = {t0, v};
+                    return false;
+                }
                 continue;
             }
             float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int m = 0; m < 2; ++m)
 #pragma unroll
-                for (int a = 0; a < 4; ++a)
+                for (int a = 0; a < 4; ++a) {
+                    const u32x2 of = org[(4 * m + a) * 64];
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
-                        const uint32_t o = org[m][2 * a + h];
+                        const uint32_t o = h ? of.y : of.x;
                         const uint32_t cur = f32x2_to_bf16x2(acc[m][a][2 * h], acc[m][a][2 * h + 1]);
                         const uint32_t dd = f32x2_to_bf16x2(u2f(cur << 16) - u2f(o << 16),
                                                             u2f(cur & 0xFFFF0000u) - u2f(o & 0xFFFF0000u));
@@ -322,6 +352,13 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                         sum[2 * h] += lo * lo;
                         sum[2 * h + 1] += hi * hi;
                     }
+                }
+            // a NaN output leaves a NaN here
+            lost = __builtin_isunordered(sum[0], sum[1]) | __builtin_isunordered(sum[2], sum[3]);
+            if (!CAREFUL && __any(lost)) {
+                at = {t0, v};
+                return false;
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {   // the other tokens of the rows: lane bits 0, 1 and 3
                 sum[i] += __shfl_xor(sum[i], 1, kWave);
@@ -329,9 +366,11 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                 sum[i] += __shfl_xor(sum[i], 8, kWave);
             }
             if ((lane & 11) == 0) {
+                int r0_lane = row0 + 4 * (lane >> 4) + 16 * ((lane >> 2) & 1);
+                asm volatile("" : "+v"(r0_lane));   // or four addresses are kept through the sums
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int r = row0 + 4 * (lane >> 4) + i + 16 * ((lane >> 2) & 1);
+                    const int r = r0_lane + i;
                     if (r < n) loss[((int64_t)v * n + r) * nblk + b] += sum[i] / (float)tokens;
                 }
             }
@@ -354,6 +393,7 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                                                 float* __restrict__ loss, u32x2* __restrict__ org, ClipStep& at) {
     constexpr int GW = 4;            // words of a token read ahead together (8 columns)
     constexpr int NG = BS / 2 / GW;
+    constexpr int CHAINS = BS >= 32 ? 4 : 2;   // of sums, as independent as they are short
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nblk = k / BS, b = blockIdx.y;
@@ -431,14 +471,25 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                     const int t = 4 * g4 + i < tc ? 4 * g4 + i : tc - 1;
                     xr[i] = xw + (int64_t)(t0 + t) * xstride;
                 }
-                f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+                f32x4 acc[CHAINS];
+                auto sum_words = [&](const uint32_t (&pw)[4], int j) {
+                    f16x8_t pv;
+                    __builtin_memcpy(&pv, pw, 16);
+                    const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+                    f32x4& c = acc[j % CHAINS];
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(pv, pair_sum, j < CHAINS ? none : c, 0, 0, 0);
+                };
+                auto sum_chains = [&]() {
+                    f32x4 t = acc[0] + acc[1];
+                    if constexpr (CHAINS == 4) t = t + (acc[2] + acc[3]);
+                    return t;
+                };
                 f32x4 total;
                 if constexpr (CAREFUL) {
                     uint32_t kind[4] = {0, 0, 0, 0};
 #pragma unroll 1
                     for (int pass = 0; pass < 2; ++pass) {
-                        acc[0] = acc[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
+                        #pragma unroll
                         for (int j = 0; j < BS / 2; ++j) {
                             // opaque, or the products would be kept from one pass for the other and the
                             // activations be read many steps ahead
@@ -447,12 +498,10 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                             uint32_t pw[4];
 #pragma unroll
                             for (int i = 0; i < 4; ++i) pw[i] = clip_kinds_f16(product(xr[i][at_j], wq[j]), pass == 0);
-                            f16x8_t pv;
-                            __builtin_memcpy(&pv, pw, 16);
-                            acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pv, pair_sum, acc[j & 1], 0, 0, 0);
+                            sum_words(pw, j);
                             __builtin_amdgcn_sched_barrier(0);
                         }
-                        total = acc[0] + acc[1];
+                        total = sum_chains();
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             if (pass == 0) kind[i] = clip_sum_kind(total[i]);
@@ -480,9 +529,7 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                             uint32_t pw[4];
 #pragma unroll
                             for (int i = 0; i < 4; ++i) pw[i] = product(cur[i][j], wq[GW * g + j]);
-                            f16x8_t pv;
-                            __builtin_memcpy(&pv, pw, 16);
-                            acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pv, pair_sum, acc[j & 1], 0, 0, 0);
+                            sum_words(pw, GW * g + j);
                         }
                         __builtin_amdgcn_sched_barrier(0);
                         if (g + 1 < NG) {
@@ -492,13 +539,13 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                                 for (int j = 0; j < GW; ++j) cur[i][j] = next[i][j];
                         }
                     }
-                    total = acc[0] + acc[1];
-                    lost |= __builtin_isunordered(total[0], total[1]) | __builtin_isunordered(total[2], total[3]);
+                    total = sum_chains();
                 }
                 float out[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) out[i] = clip_round<MO_F16>(total[i]);
                 if (v < r0) {
+                    lost |= __builtin_isunordered(total[0], total[1]) | __builtin_isunordered(total[2], total[3]);
                     u32x2 o;
                     o.x = f32_to_f16_bits(out[0]) | (f32_to_f16_bits(out[1]) << 16);
                     o.y = f32_to_f16_bits(out[2]) | (f32_to_f16_bits(out[3]) << 16);
@@ -515,6 +562,8 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                     }
                 }
             }
+            // a NaN output leaves a NaN here (a token past the end is the last one again)
+            if (v >= r0) lost = __builtin_isunordered(sum[0], sum[1]) | __builtin_isunordered(sum[2], sum[3]);
             if (!CAREFUL && __any(lost)) {
                 at = {t0, v};
                 return false;
@@ -677,10 +726,13 @@ __global__ __launch_bounds__(kClipLanes * kClipWaves, DT == MO_BF16 ? 3 : 2) voi
     const int r1 = (int)((blockIdx.z + 1) * (unsigned)ratios.count / gridDim.z);
     if constexpr (DT == MO_BF16) {
         ClipStep at;
+        // of a lane: 8 words of four partial sums, and 8 of four rounded outputs of the unclipped block
+        f32x4* parts = (f32x4*)clip_smem + (threadIdx.x >> 6) * 512 + (threadIdx.x & 63);
+        u32x2* org = (u32x2*)((f32x4*)clip_smem + kClipWaves * 512) + (threadIdx.x >> 6) * 512 + (threadIdx.x & 63);
         if (!clip_losses_bf16<BS, false>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype,
-                                         ratios, r0, r1, op, loss, at))
+                                         ratios, r0, r1, op, loss, parts, org, at))
             clip_losses_bf16<BS, true>((const uint16_t*)x, tokens, (const uint16_t*)w, n, k, w_amax, amax_dtype,
-                                       ratios, r0, r1, op, loss, at);
+                                       ratios, r0, r1, op, loss, parts, org, at);
     } else if constexpr (DT == MO_F16) {
         ClipStep at;
         u32x2* org = (u32x2*)clip_smem;
@@ -733,17 +785,18 @@ extern "C" int mo_awq_clip_losses(const void* x, int64_t tokens, const void* w, 
         smem = (size_t)waves * mo::kClipTokens * mo::kClipLanes * 4 +
                (waves > 1 ? (size_t)2 * waves * mo::kClipLanes * sizeof(float) : 0);
     } else {
-        if (dtype == MO_F16) smem = (size_t)mo::kClipWaves * mo::kClipTokens * mo::kClipLanes * 2;
+        smem = (size_t)mo::kClipWaves * mo::kClipLanes * (dtype == MO_F16 ? mo::kClipTokens * 2 : 8 * (16 + 8));
         // A wavefront goes through all ratios unless there are too few of them to fill the chip; then
         // 2 to 11 of them share the ratios, each scoring the unclipped block once more.  11 ratios, 64
         // tokens, blocks of 128 (before: one vector-ALU kernel for both types, 1070 / 2160 us on the
         // first line):
-        //   bf16  4096 x 4096, 4096 wavefronts: 464 us (2 shares: 488); 1024 x 4096, 1024: 147, 137 with 2,
-        //         138 with 3; 1024 x 1024, 256: 143, 86 with 2, 50 with 4, 55 with 8
-        //   fp16  4096 x 4096, 2048 wavefronts: 496 us, 430 with 2 shares, 450 with 4; 1024 x 4096, 512:
-        //         307, 143 with 4, 156 with 8; 1024 x 1024, 128: 272, 95 with 4, 71 with 8, 69 with 11
-        // What bounds the bf16 form: a step of 2048 products is 128 cycles of matrix instructions and
-        // about 110 of vector instructions plus 40 of the port that issues both; measured 180.
+        //   bf16  4096 x 4096, 4096 wavefronts: 484 us, 503 with 2 shares; 1024 x 4096, 1024: 157, 145 with 2,
+        //         142 with 3, 149 with 4; 1024 x 1024, 256: 156, 91 with 2, 56 with 4, 59 with 8
+        //   fp16  4096 x 4096, 2048 wavefronts: 506 us, 444 with 2 shares, 465 with 4; 1024 x 4096, 512:
+        //         313, 148 with 4, 162 with 8; 1024 x 1024, 128: 280, 99 with 4, 76 with 8, 72 with 11
+        // (boxes differ by some 8 %.)  What bounds the bf16 form: a step of 2048 products is 128 cycles of
+        // matrix instructions and about 110 of vector instructions plus 40 of the port that issues both;
+        // measured 180.
         const int64_t sets = (int64_t)grid.x * grid.y * mo::kClipWaves;
         int64_t share = ((dtype == MO_BF16 ? 2048 : 3072) + sets - 1) / sets;
         if (dtype == MO_BF16 && share > 4) share = 4;

@@ -104,6 +104,19 @@ def test_a_row_that_is_not_finite_leaves_the_others_alone(dtype, kind, n, k, tok
         torch.testing.assert_close(mine[large], cpu[large], rtol=0.08, atol=0.0)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("block", [32, 64, 128])
+def test_sums_are_made_in_chains_of_a_quarter_of_a_block(dtype, block):
+    """One large weight at either end of a block, small ones between: 2^24 + 1 is 2^24 in fp32, so that the
+    chains with the large ones lose small ones, and no other chain does.  Quantised, the small ones are zero and
+    the large ones themselves: the loss is the square of what the sum of the block has kept, half of it at least."""
+    w = torch.full((96, 2 * block), 2.0 ** -11).to(dtype)      # a pair of products: 2^-10
+    w.view(96, 2, block)[..., 0], w.view(96, 2, block)[..., -1] = 2.0 ** 14, -2.0 ** 14
+    kept = block / 2 * 2.0 ** -11
+    loss = _losses(w, torch.ones(1, 2 * block).to(dtype), block, ratios=[1.0])
+    assert (loss >= kept * kept).all() and (loss <= (2 * kept) ** 2).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("ratios,blocks", [(1, 1), (11, 255), (11, 257), (3, 5000)])
 def test_best_clip_is_what_the_loop_over_the_ratios_leaves(dtype, ratios, blocks):
