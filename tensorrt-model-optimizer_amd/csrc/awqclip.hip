@@ -139,7 +139,7 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
     constexpr int RUN = HALVES >= 2 ? HALVES / 2 : 1;   // chunks until the chains of both tiles have ended
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int fr = lane & 31, kg = lane >> 5;
+    const int fr = lane & 31;
     const int nblk = k / BS, b = blockIdx.y;
     const int row0 = (blockIdx.x * kClipWaves + wave) * 32;
     if (row0 >= n) return true;
@@ -156,23 +156,22 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
 #pragma unroll
     for (int i = 0; i < 32; ++i) zero[i] = 0.0f;
     for (int t0 = CAREFUL ? __builtin_amdgcn_readfirstlane(at.token) : 0; t0 < tokens; t0 += kClipTokens) {
-        int xrow[2];
         bool live[2];   // a token past the end counts as a row of zeros
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            const int t = t0 + 32 * m + fr;
-            live[m] = t < tokens;
-            xrow[m] = live[m] ? t : tokens - 1;
-        }
-        // The addresses are made anew for every chunk from a row number: three 64-bit addresses kept
-        // across the chunk loop would cost the third wavefront of a SIMD.
+        for (int m = 0; m < 2; ++m) live[m] = t0 + 32 * m + fr < tokens;
+        // The addresses are made anew for every chunk from the lane's number: what is kept across the
+        // chunk loop beside the sums and the products would cost the third wavefront of a SIMD.
         u32x4 wraw, xraw[2];
         auto fetch = [&](int c) {
-            asm volatile("" : "+v"(row), "+v"(xrow[0]), "+v"(xrow[1]));
-            const int col = b * BS + c * 16 + kg * 8;
+            int l = lane;
+            asm volatile("" : "+v"(l), "+v"(row));
+            const int col = b * BS + c * 16 + (l >> 5) * 8;
             wraw = *(const u32x4*)(w + ((int64_t)row * k + col));
 #pragma unroll
-            for (int m = 0; m < 2; ++m) xraw[m] = *(const u32x4*)(x + ((int64_t)xrow[m] * k + col));
+            for (int m = 0; m < 2; ++m) {
+                const int t = t0 + 32 * m + (l & 31);
+                xraw[m] = *(const u32x4*)(x + ((int64_t)(t < tokens ? t : tokens - 1) * k + col));
+            }
         };
         fetch(0);
         for (int v = r0 - 1; v < r1; ++v) {   // r0 - 1: the unclipped block
