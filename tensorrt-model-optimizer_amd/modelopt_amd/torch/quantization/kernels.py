@@ -225,10 +225,19 @@ def ste_mask(x, amax, grad):
 
 def wgrad_mask_pays(tokens: int, n: int, k: int) -> bool:
     """Whether the weight gradient [n, k] over ``tokens`` is computed and masked in one pass.  The pass
-    saved over the gradient outweighs the library's faster product up to 1024 tokens (bf16, one pass
-    against two: 14336 x 4096 179 us and 200, at 2048 tokens 321 and 314; 2048 x 7168 52 and 54), with fewer
-    than 256 workgroups of 128 x 128 results up to 512 (512 x 512 11 us and 11, at 1024 tokens 17 and 14)."""
-    return 1 <= tokens <= (1024 if n * k >= 1 << 22 else 512) and n % 8 == 0 and k % 8 == 0
+    saved over the gradient outweighs the library's faster product up to 1024 tokens (one pass against two:
+    14336 x 4096 bf16 165 us and 192, fp16 165 and 195; 4096 x 4096 57 and 57; at 2048 tokens 321 and 314), with
+    fewer than 256 workgroups of 128 x 128 results up to 512 (512 x 512 10.7 us and 11.1, at 1024 tokens 17
+    and 14; 16384 x 128 11.3 and 14.5, 18.5 and 17).  A tile that is mostly padding pays for less: 8 rows up to
+    256 tokens (8 x 4096 fp16 6.8 us and 8.0, at 512 tokens 10.0 and 9.9), 8 or 16 columns, whose rows of the
+    weight are 16 or 32 bytes, up to 64 (65536 x 8 bf16 7.6 us and 8.5, at 128 tokens 9.7 and 9.2; 24 columns 17
+    and 21 at 512)."""
+    most = 1024 if n * k >= 1 << 22 else 512
+    if k < 24:
+        most = 64
+    elif n < 16:
+        most = 256
+    return 1 <= tokens <= most and n % 8 == 0 and k % 8 == 0
 
 
 def fake_quant_nvfp4(x, global_amax, block_size=16, mode=0):
