@@ -265,6 +265,17 @@ class DynamicBlockQuantizationFunction(Function):
         return _backward(ctx, grad_outputs, 9)
 
 
+def _is_wanted(ctx, index):
+    """Whether the backward pass that runs goes on to tensor input ``index`` of the function: a gradient
+    that ``needs_input_grad`` allows need not be asked for (``torch.autograd.grad(y, x)`` leaves the weight's)."""
+    if not ctx.needs_input_grad[index]:
+        return False
+    try:
+        return torch._C._will_engine_execute_node(ctx.next_functions[index][0])
+    except RuntimeError:   # no answer for a leaf that is asked for itself
+        return True
+
+
 class MaskedGradientLinear(Function):
     """``F.linear(x, quantizer(weight), bias)`` for a weight quantizer whose backward keeps the gradient
     where ``|weight| <= amax``: the weight gradient is computed and masked in one pass
@@ -297,19 +308,19 @@ class MaskedGradientLinear(Function):
             return kept.reshape(n, k)
 
         grads = [None, None, None]
-        if ctx.needs_input_grad[0]:
+        if _is_wanted(ctx, 0):
             used = quantized
             if differentiated:   # its value, with the straight-through path back to the weight
                 used = quantized + masked(weight, weight - weight.detach())
             grads[0] = (rows @ used).reshape(x.shape)
-        if ctx.needs_input_grad[1]:
+        if _is_wanted(ctx, 1):
             x2 = x.reshape(-1, k)
             if plain:
                 grads[1] = _hip.wgrad_masked(rows.contiguous(), x2.contiguous(), weight.detach(),
                                              amax.reshape(-1).contiguous(), ctx.inner, narrow)
             if grads[1] is None:
                 grads[1] = masked(weight, rows.t() @ x2)
-        if ctx.has_bias and ctx.needs_input_grad[2]:
+        if ctx.has_bias and _is_wanted(ctx, 2):
             grads[2] = rows.sum(0)
         return (*grads, None, None, None)
 

@@ -2,8 +2,12 @@
 backward computes, with the kernel's place taken by the tensor expression (no GPU needed)."""
 
 import pytest
+import torch
+import torch.nn.functional as F
 
+from modelopt_amd import _hip
 from modelopt_amd.torch.quantization import kernels
+from modelopt_amd.torch.quantization.tensor_quant import MaskedGradientLinear
 
 
 @pytest.mark.parametrize("n,k,most", [
@@ -14,3 +18,66 @@ def test_the_sizes_at_which_one_pass_pays(n, k, most):
     """By the tokens up to which it was measured to be no slower than the product and the mask."""
     for tokens in (0, 1, most, most + 1, 4096):
         assert kernels.wgrad_mask_pays(tokens, n, k) == (1 <= tokens <= most), tokens
+
+
+def _halves(w):   # a quantizer of the CPU: to steps of a half within +-1
+    return (w.clamp(-1, 1) * 2).round() / 2
+
+
+@pytest.fixture
+def made(monkeypatch):
+    """The weight gradients that were computed."""
+    done = []
+
+    def wgrad_masked(dy, x, w, amax, inner=0, narrow_amax=False):
+        done.append("weight")
+        return torch.where(w.abs() <= amax.reshape(-1, 1), dy.t() @ x, torch.zeros(()))
+
+    monkeypatch.setattr(_hip, "wgrad_masked", wgrad_masked)
+    return done
+
+
+def _case(leaf=True, bias=True):
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(5, 8, generator=g, requires_grad=True)
+    w = torch.randn(16, 8, generator=g, requires_grad=True)
+    b = torch.randn(16, generator=g, requires_grad=True) if bias else None
+    seen = x if leaf else x * 1.0
+    return x, w, b, seen, MaskedGradientLinear.apply(seen, w, b, _halves, torch.ones(()), 0)
+
+
+@pytest.mark.parametrize("leaf", [True, False])
+@pytest.mark.parametrize("bias", [True, False])
+def test_only_the_gradients_that_are_asked_for_are_computed(made, leaf, bias):
+    x, w, b, seen, y = _case(leaf, bias)
+    dy = torch.randn(5, 16, generator=torch.Generator().manual_seed(4))
+    products = []
+
+    class Count(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func is torch.ops.aten.mm.default:
+                products.append(tuple(args[1].shape))
+            return func(*args, **(kwargs or {}))
+
+    want = {"x": dy @ _halves(w.detach()), "w": torch.where(w.detach().abs() <= 1, dy.t() @ x.detach(), torch.zeros(())),
+            "b": dy.sum(0)}
+    tensors = {"x": x, "w": w, "b": b}
+    for names in (("x",), ("w",), ("b",), ("x", "w"), ("w", "b"), ("x", "w", "b")):
+        if b is None and "b" in names:
+            continue
+        made.clear()
+        got = torch.autograd.grad(y, [tensors[n] for n in names], dy, retain_graph=True)
+        for n, t in zip(names, got):
+            assert torch.equal(t, want[n])
+        assert made == (["weight"] if "w" in names else [])
+        with Count():
+            products.clear()
+            torch.autograd.grad(y, [tensors[n] for n in names], dy, retain_graph=True)
+        # [16, 8] for the input; the tensor expression of the weight's under a dispatch mode
+        assert products == [(16, 8)] * ("x" in names) + [(5, 8)] * ("w" in names)
+    made.clear()
+    y.backward(dy, inputs=[w], retain_graph=True)
+    assert made == ["weight"] and x.grad is None and torch.equal(w.grad, want["w"])
+    w.grad = None
+    y.backward(dy)
+    assert torch.equal(x.grad, want["x"]) and torch.equal(w.grad, want["w"]) and (b is None or torch.equal(b.grad, want["b"]))
