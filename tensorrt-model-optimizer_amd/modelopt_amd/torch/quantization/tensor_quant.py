@@ -284,7 +284,8 @@ class MaskedGradientLinear(Function):
     @staticmethod
     def forward(ctx, x, weight, bias, quantizer, amax, inner):
         quantized = quantizer(weight)          # grad mode is off here
-        ctx.save_for_backward(x, weight, quantized, amax)
+        # the quantised weight is for the input's gradient: of an input without one it is not kept
+        ctx.save_for_backward(x, weight, quantized if ctx.needs_input_grad[0] else None, amax)
         ctx.inner, ctx.has_bias = inner, bias is not None
         return torch.nn.functional.linear(x, quantized, bias)
 

@@ -81,3 +81,16 @@ def test_only_the_gradients_that_are_asked_for_are_computed(made, leaf, bias):
     w.grad = None
     y.backward(dy)
     assert torch.equal(x.grad, want["x"]) and torch.equal(w.grad, want["w"]) and (b is None or torch.equal(b.grad, want["b"]))
+
+
+@pytest.mark.parametrize("trained_input", [True, False])
+def test_the_quantised_weight_is_kept_for_the_gradient_of_the_input_only(made, trained_input):
+    x = torch.randn(5, 8, requires_grad=trained_input)
+    w = torch.randn(16, 8, requires_grad=True)
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(t) or t, lambda t: t):
+        y = MaskedGradientLinear.apply(x, w, None, _halves, torch.ones(()), 0)
+    quantized = [t for t in kept if t.shape == w.shape and t is not w and torch.equal(t, _halves(w.detach()))]
+    assert len(quantized) == trained_input
+    y.sum().backward()
+    assert w.grad is not None and (x.grad is not None) == trained_input
