@@ -7,6 +7,7 @@ functions take and return torch tensors and never synchronise with the host.
 import math
 
 import torch
+from torch.utils._device import DeviceContext
 
 from ... import _hip
 
@@ -258,12 +259,15 @@ def fake_quant_block_fp(x, block_size, fmt, scale_fmt="E8M0", global_amax=None):
 
 def torch_is_intercepted() -> bool:
     """Whether something follows the tensor operations of this thread (a compiler, a dispatch or
-    function mode, a functorch transform, forward-mode differentiation, a trace):
-    a shortcut past an operator that it would see is not taken then."""
+    function mode, a functorch transform, forward-mode differentiation, a trace): a shortcut past an
+    operator that it would see is not taken then.  The mode behind ``torch.set_default_device`` is no such
+    thing: it is on the stack for a whole program and only says where new tensors go that name no device."""
     if torch.compiler.is_compiling():
         return True
-    return bool(torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch._C._functorch.peek_interpreter_stack() is not None
+    for i in range(torch._C._len_torch_function_stack()):
+        if type(torch._C._get_function_stack_at(i)) is not DeviceContext:
+            return True
+    return bool(torch._C._len_torch_dispatch_stack() or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None)
 
 

@@ -1,9 +1,9 @@
 """The linear layer whose weight gradient is computed and masked in one pass: which calls take it and what its
-backward computes, with the kernel's place taken by the tensor expression (no GPU needed)."""
+backward computes, with the kernel's place taken by the tensor expression; what the shortcuts past the operators take for an
+interception (no GPU needed)."""
 
 import pytest
 import torch
-import torch.nn.functional as F
 
 from modelopt_amd import _hip
 from modelopt_amd.torch.quantization import kernels
@@ -94,3 +94,22 @@ def test_the_quantised_weight_is_kept_for_the_gradient_of_the_input_only(made, t
     assert len(quantized) == trained_input
     y.sum().backward()
     assert w.grad is not None and (x.grad is not None) == trained_input
+
+
+def test_a_default_device_is_no_interception():
+    class Follows(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert not kernels.torch_is_intercepted()
+    with torch.device("cpu"):
+        assert not kernels.torch_is_intercepted()
+        with Follows():
+            assert kernels.torch_is_intercepted()
+    with Follows(), torch.device("meta"):
+        assert kernels.torch_is_intercepted()
+    torch.set_default_device("cpu")
+    try:
+        assert not kernels.torch_is_intercepted()
+    finally:
+        torch.set_default_device(None)
