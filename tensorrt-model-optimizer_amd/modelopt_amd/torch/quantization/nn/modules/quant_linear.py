@@ -22,7 +22,10 @@ class _QuantLinear(QuantLinearConvBase):
 
     def forward(self, input, *args, **kwargs):
         input = self.input_quantizer(input)
-        output = self._masked_gradient_linear(input) if torch.is_grad_enabled() else None
+        output = None
+        # a compiler would follow every step of the choice
+        if torch.is_grad_enabled() and not torch.compiler.is_compiling():
+            output = self._masked_gradient_linear(input)
         if output is None:
             weight = self.weight_quantizer(self.weight)
             output = F.linear(input, weight, self.bias)
@@ -42,7 +45,7 @@ class _QuantLinear(QuantLinearConvBase):
                 or not weight.is_contiguous() or input.shape[-1] != weight.shape[1]
                 or not kernels.wgrad_mask_pays(input.numel() // weight.shape[1], *weight.shape)
                 or torch.is_autocast_enabled("cuda") or quantizer_has_hooks(quantizer)
-                or torch.compiler.is_compiling() or kernels.torch_is_intercepted()
+                or kernels.torch_is_intercepted()
                 or (self.bias is not None and type(self.bias) is not nn.Parameter)):
             return None
         amax = quantizer.clipping_amax(weight)

@@ -7,6 +7,7 @@ import torch
 
 from modelopt_amd import _hip
 from modelopt_amd.torch.quantization import kernels
+from modelopt_amd.torch.quantization.nn import QuantLinear
 from modelopt_amd.torch.quantization.tensor_quant import MaskedGradientLinear
 
 
@@ -113,3 +114,16 @@ def test_a_default_device_is_no_interception():
         assert not kernels.torch_is_intercepted()
     finally:
         torch.set_default_device(None)
+
+
+def test_a_compiler_does_not_follow_the_choice_of_the_route(monkeypatch):
+    layer = QuantLinear(8, 8)
+    for quantizer in (layer.input_quantizer, layer.weight_quantizer, layer.output_quantizer):
+        quantizer.disable()
+    asked = []
+    monkeypatch.setattr(type(layer), "_masked_gradient_linear", lambda self, x: asked.append(x))
+    x = torch.randn(4, 8)
+    want = layer(x)
+    assert len(asked) == 1
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    assert torch.equal(layer(x), want) and len(asked) == 1
