@@ -110,9 +110,18 @@ __device__ __forceinline__ uint32_t nvfp4_codes(const float (&v)[8], uint32_t bm
     const float r = 1.0f / s;
     uint32_t c = 0;
     if (!exact && nvfp4_scale_fast(s, bmax_bits, r)) {
+        float q[8];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            c = fp4_pair(c, quotient_of<DT>(v[2 * j], s, r), quotient_of<DT>(v[2 * j + 1], s, r), j);
+        for (int j = 0; j < 8; ++j) q[j] = quotient_of<DT>(v[j], s, r);
+        if constexpr (DT == MO_F32) {
+            // The code keeps the sign of the quotient.  m smallest denormals over s round to a zero, which has
+            // no sign here, where m <= s / 2; the short form may leave either neighbour.
+            const float least = u2f((uint32_t)(0.5f * s));
+#pragma unroll
+            for (int j = 0; j < 8; ++j) q[j] = __builtin_fabsf(v[j]) > least ? q[j] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c = fp4_pair(c, q[2 * j], q[2 * j + 1], j);
         return c;
     }
     keep_branch();

@@ -125,6 +125,24 @@ def test_all_bf16_patterns_against_oracle():
         assert_bits_equal(p.cpu(), po, f"packed pilot={pilot}")
 
 
+@pytest.mark.parametrize("block", [8, 16, 32])
+@pytest.mark.parametrize("wsf2", [1.0, 0.37, 4.0])
+def test_quotients_that_round_to_zero_have_no_sign(block, wsf2):
+    """fp32 elements of a few smallest denormals in blocks whose scale is above 2: a negative one rounds to zero
+    up to half the scale, and to a denormal with a code that keeps the sign beyond."""
+    g = torch.Generator().manual_seed(block)
+    x = torch.randint(-600, 601, (2048, 128), generator=g).float() * 2.0 ** -149
+    x[0] = torch.arange(-64, 64) * 2.0 ** -149
+    top = torch.exp(torch.rand(2048, 128 // block, generator=g) * 6.2 + 2.5) * wsf2
+    top[0] = torch.tensor([12.0, 18.0, 24.0, 36.0]).repeat(4)[:128 // block] * wsf2   # scales 2, 3, 4, 6 of wsf2
+    x.view(2048, -1, block)[..., 5] = top
+    packed_o, wsf_o, _ = qtensor.nvfp4_quantize(x, block, wsf2=torch.tensor(wsf2))
+    for flags in (0, _hip.MO_FLAG_FORCE_EXACT):
+        packed, wsf, _ = _hip.nvfp4_quantize(x.to(DEV), torch.tensor(wsf2, device=DEV), block, amax_is_wsf2=True, flags=flags)
+        assert_bits_equal(wsf.cpu(), wsf_o, "wsf")
+        assert_bits_equal(packed.cpu(), packed_o, "packed")
+
+
 def test_fast_path_equals_exact_division_on_large_input():
     """Same GPU, same input: multiply-and-verify codes == literal per-element division codes."""
     g = torch.Generator(device=DEV).manual_seed(11)
