@@ -448,10 +448,9 @@ __device__ __forceinline__ void qdq_block16_bf16(const uint32_t (&w)[8], float g
     for (int j = 0; j < 8; ++j) { lo[j] = o[j]; hi[j] = o[8 + j]; }
 }
 
-// RP = pairs of 16-byte loads per lane (a workgroup handles RP * 256 blocks).  Measured: one pair
-// beats four from 50 MB of input (8192 x 4096: 5.4 - 5.7 TB/s against 5.0; 537 MB: 6.45 against
-// 6.0) and ties at 34 MB; smaller tensors go row by row.
-template <int MODE, int RP>
+// Two 16-byte loads a lane, in rounds of 256 so that a wavefront reads contiguous memory.  More in flight
+// per lane is slower (four times as much: 8192 x 4096 5.0 TB/s, 5.4 - 5.7 this way) and an occupancy cap wins nothing.
+template <int MODE>
 __global__ __launch_bounds__(256) void nvfp4_qdq_fast_kernel(const uint16_t* __restrict__ x,
                                                              uint16_t* __restrict__ y,
                                                              int64_t nblocks, const void* amax,
@@ -459,48 +458,39 @@ __global__ __launch_bounds__(256) void nvfp4_qdq_fast_kernel(const uint16_t* __r
     const float gs = load_scalar(amax, amax_dtype, 0) / 2688.0f;
     const float gs_safe = gs > 0.0f ? gs : 1e-12f;
     const int64_t nchunks = nblocks * 2;
-    const int64_t c0 = (int64_t)blockIdx.x * (RP * 512) + threadIdx.x;
+    const int64_t ca = (int64_t)blockIdx.x * 512 + threadIdx.x, cb = ca + 256;
     const bool odd = threadIdx.x & 1;
-    u32x4 a[RP], b[RP];
-#pragma unroll
-    for (int p = 0; p < RP; ++p) {
-        const int64_t ca = c0 + p * 512, cb = ca + 256;
-        const u32x4 zero = {0, 0, 0, 0};
-        a[p] = ca < nchunks ? __builtin_nontemporal_load((const u32x4*)(x + ca * 8)) : zero;
-        b[p] = cb < nchunks ? __builtin_nontemporal_load((const u32x4*)(x + cb * 8)) : zero;
-    }
-#pragma unroll
-    for (int p = 0; p < RP; ++p) {
-        const int64_t ca = c0 + p * 512, cb = ca + 256;
-        const u32x4 send = odd ? a[p] : b[p];
-        u32x4 recv;
-        recv.x = swap_adjacent_lanes(send.x);
-        recv.y = swap_adjacent_lanes(send.y);
-        recv.z = swap_adjacent_lanes(send.z);
-        recv.w = swap_adjacent_lanes(send.w);
-        const u32x4 first = odd ? recv : a[p], second = odd ? b[p] : recv;
-        const uint32_t w[8] = {first.x, first.y, first.z, first.w,
-                               second.x, second.y, second.z, second.w};
-        float lo[8], hi[8];
-        qdq_block16_bf16<MODE>(w, gs, gs_safe, lo, hi);
-        // back to the load layout, so that the stores are contiguous across the wavefront:
-        // the even lane hands over the second chunk of its round-A block and receives the
-        // first chunk of the neighbour's round-B block; the odd lane the other way round.
-        u32x4 o0, o1;
-        o0.x = f32x2_to_bf16x2(lo[0], lo[1]); o0.y = f32x2_to_bf16x2(lo[2], lo[3]);
-        o0.z = f32x2_to_bf16x2(lo[4], lo[5]); o0.w = f32x2_to_bf16x2(lo[6], lo[7]);
-        o1.x = f32x2_to_bf16x2(hi[0], hi[1]); o1.y = f32x2_to_bf16x2(hi[2], hi[3]);
-        o1.z = f32x2_to_bf16x2(hi[4], hi[5]); o1.w = f32x2_to_bf16x2(hi[6], hi[7]);
-        const u32x4 give = odd ? o0 : o1;
-        u32x4 got;
-        got.x = swap_adjacent_lanes(give.x);
-        got.y = swap_adjacent_lanes(give.y);
-        got.z = swap_adjacent_lanes(give.z);
-        got.w = swap_adjacent_lanes(give.w);
-        const u32x4 out_a = odd ? got : o0, out_b = odd ? o1 : got;
-        if (ca < nchunks) __builtin_nontemporal_store(out_a, (u32x4*)(y + ca * 8));
-        if (cb < nchunks) __builtin_nontemporal_store(out_b, (u32x4*)(y + cb * 8));
-    }
+    const u32x4 zero = {0, 0, 0, 0};
+    const u32x4 a = ca < nchunks ? __builtin_nontemporal_load((const u32x4*)(x + ca * 8)) : zero;
+    const u32x4 b = cb < nchunks ? __builtin_nontemporal_load((const u32x4*)(x + cb * 8)) : zero;
+    const u32x4 send = odd ? a : b;
+    u32x4 recv;
+    recv.x = swap_adjacent_lanes(send.x);
+    recv.y = swap_adjacent_lanes(send.y);
+    recv.z = swap_adjacent_lanes(send.z);
+    recv.w = swap_adjacent_lanes(send.w);
+    const u32x4 first = odd ? recv : a, second = odd ? b : recv;
+    const uint32_t w[8] = {first.x, first.y, first.z, first.w,
+                           second.x, second.y, second.z, second.w};
+    float lo[8], hi[8];
+    qdq_block16_bf16<MODE>(w, gs, gs_safe, lo, hi);
+    // back to the load layout, so that the stores are contiguous across the wavefront:
+    // the even lane hands over the second chunk of its round-A block and receives the
+    // first chunk of the neighbour's round-B block; the odd lane the other way round.
+    u32x4 o0, o1;
+    o0.x = f32x2_to_bf16x2(lo[0], lo[1]); o0.y = f32x2_to_bf16x2(lo[2], lo[3]);
+    o0.z = f32x2_to_bf16x2(lo[4], lo[5]); o0.w = f32x2_to_bf16x2(lo[6], lo[7]);
+    o1.x = f32x2_to_bf16x2(hi[0], hi[1]); o1.y = f32x2_to_bf16x2(hi[2], hi[3]);
+    o1.z = f32x2_to_bf16x2(hi[4], hi[5]); o1.w = f32x2_to_bf16x2(hi[6], hi[7]);
+    const u32x4 give = odd ? o0 : o1;
+    u32x4 got;
+    got.x = swap_adjacent_lanes(give.x);
+    got.y = swap_adjacent_lanes(give.y);
+    got.z = swap_adjacent_lanes(give.z);
+    got.w = swap_adjacent_lanes(give.w);
+    const u32x4 out_a = odd ? got : o0, out_b = odd ? o1 : got;
+    if (ca < nchunks) __builtin_nontemporal_store(out_a, (u32x4*)(y + ca * 8));
+    if (cb < nchunks) __builtin_nontemporal_store(out_b, (u32x4*)(y + cb * 8));
 }
 
 template <int DT, int BS>
@@ -673,8 +663,8 @@ extern "C" int mo_nvfp4_qdq(const void* x, void* y, int64_t rows, int64_t k, int
         const unsigned g = (unsigned)tiles;
         const uint16_t* xi = (const uint16_t*)x;
         uint16_t* yo = (uint16_t*)y;
-        if (mode == 0) mo::nvfp4_qdq_fast_kernel<0, 1><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
-        else mo::nvfp4_qdq_fast_kernel<1, 1><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
+        if (mode == 0) mo::nvfp4_qdq_fast_kernel<0><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
+        else mo::nvfp4_qdq_fast_kernel<1><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
         return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
     }
     // every other size, type, block size and layout

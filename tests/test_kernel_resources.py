@@ -79,7 +79,7 @@ def _vgprs(kernels, fragment):
     ("nvfp4_quantize_multi_kernel", 64, "eight wavefronts per SIMD, the occupancy cap decides"),
     ("absmax_multi_kernelILi2E", 64, "eight wavefronts per SIMD"),
     ("weight_scale_colsum8_kernelILi2E", 96, "five wavefronts per SIMD (three: 25 % slower)"),
-    ("nvfp4_qdq_fast_kernelILi0ELi1E", 64, "eight wavefronts per SIMD"),
+    ("nvfp4_qdq_fast_kernelILi0E", 64, "eight wavefronts per SIMD"),
     ("qdq_kernelILi2ELi0ELb0ENS_5Fp8OpILb1E", 64, "eight wavefronts per SIMD"),
 ])
 def test_register_budget(kernels, fragment, limit, why):
