@@ -343,6 +343,9 @@ __device__ __forceinline__ float tensor_amax(const void* amax, int dtype, uint32
 // launches: parts of x (16-byte aligned), their fold to one value of out_dtype
 int launch_absmax_parts(const void* x, int64_t n, int dtype, bool keep, uint32_t* parts, int* nparts, hipStream_t s);
 int launch_fold_parts(const uint32_t* parts, int nparts, void* out, int out_dtype, hipStream_t s);
+// mo_nvfp4_qdq of n elements in the form for large whole tensors, MO_ERR_UNSUPPORTED where that is not the faster one
+int nvfp4_qdq_whole(const void* x, void* y, int64_t n, int64_t k, int dtype, int block_size, int mode, const void* amax,
+                    int amax_dtype, hipStream_t s);
 // mo_row_qdq behind its checks, amax_dtype a type or parts
 int row_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* pre, int kind, int p0, int p1,
             int p2, const void* amax, int amax_dtype, hipStream_t s);

@@ -644,6 +644,23 @@ extern "C" int mo_nvfp4_dequantize(const uint8_t* packed, const uint8_t* wsf, co
     return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
 }
 
+// The kernel for whole bf16 blocks of 16, from one round of its workgroups on the chip (2^20 blocks, 32 MB:
+// 11.1 us, row by row 12.0; 64 MB 22.2 and 22.6; 24 MB 10.1 and 10.1, 64 x 4096 4.4 and 3.0) to 256 MB (81.9 and 82.5;
+// 512 MB 165 and 165, 2 GB 689 and 671).  MO_ERR_UNSUPPORTED for all else.
+int mo::nvfp4_qdq_whole(const void* x, void* y, int64_t n, int64_t k, int dtype, int block_size, int mode,
+                        const void* amax, int amax_dtype, hipStream_t s) {
+    const int64_t nblocks = n / 16;
+    if (dtype != MO_BF16 || block_size != 16 || k % 16 || nblocks < (1ll << 20) || nblocks > (1ll << 23) ||
+        (((uintptr_t)x | (uintptr_t)y) & 15u))
+        return MO_ERR_UNSUPPORTED;
+    const unsigned g = (unsigned)((nblocks + 255) / 256);
+    const uint16_t* xi = (const uint16_t*)x;
+    uint16_t* yo = (uint16_t*)y;
+    if (mode == 0) nvfp4_qdq_fast_kernel<0><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
+    else nvfp4_qdq_fast_kernel<1><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
+    return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
+}
+
 extern "C" int mo_nvfp4_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype,
                             const void* amax, int amax_dtype, int block_size, int mode,
                             void* stream) {
@@ -652,22 +669,6 @@ extern "C" int mo_nvfp4_qdq(const void* x, void* y, int64_t rows, int64_t k, int
     if (amax_dtype < MO_F32 || amax_dtype > MO_BF16) return MO_ERR_DTYPE;
     if (rows == 0 || k == 0) return MO_OK;
     if (!x || !y || !amax) return MO_ERR_ARG;
-    hipStream_t s = (hipStream_t)stream;
-    const int64_t nblocks = rows * k / 16;
-    // from 32 MB the two kernels tie (8192 x 8192 43.1 and 43.2 us), below it the row-wise one is faster
-    // (64 x 4096 3.0 us against 4.4)
-    if (dtype == MO_BF16 && block_size == 16 && k % 16 == 0 && nblocks >= (1ll << 20) &&
-        ((((uintptr_t)x | (uintptr_t)y) & 15u) == 0)) {
-        const int64_t tiles = (nblocks + 255) / 256;
-        if (tiles > 0x7FFFFFFF) return MO_ERR_UNSUPPORTED;
-        const unsigned g = (unsigned)tiles;
-        const uint16_t* xi = (const uint16_t*)x;
-        uint16_t* yo = (uint16_t*)y;
-        if (mode == 0) mo::nvfp4_qdq_fast_kernel<0><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
-        else mo::nvfp4_qdq_fast_kernel<1><<<g, 256, 0, s>>>(xi, yo, nblocks, amax, amax_dtype);
-        return hipGetLastError() == hipSuccess ? MO_OK : MO_ERR_LAUNCH;
-    }
-    // every other size, type, block size and layout
     return mo_row_qdq(x, y, rows, k, dtype, nullptr, MO_ROW_NVFP4, block_size, mode, 0, amax, amax_dtype, stream);
 }
 

@@ -6,11 +6,10 @@
 // twice as often.  A lane owns chunks of 8 columns of one row, all loads ahead of the first store; the
 // scales of a chunk come from L2.  The product is rounded to the tensor's type before it is quantised, as
 // the tensor expression rounds it.  Measured, each against the kernel it replaced: NVFP4 of fp16 1537 x 3000
-// 7.9 us (15.4 with element loads and a division per element), INT8 of a scaled bf16 2048 x 14336 22.7 us
+// 7.0 us (15.4 with element loads and a division per element), INT8 of a scaled bf16 2048 x 14336 22.7 us
 // (43.2 with the product in a launch of its own), NVFP4 of fp32 4096 x 8192 53 us (69), MX E4M3 of
 // bf16 3001 x 5001 15 us (43 with element loads) and of 8192 x 8192 43 us (47).  Without a scale and aligned
-// it equals the whole-tensor kernels or beats them: bf16 64 x 4096 2.6 - 3.0 us (INT8 3.2, FP8 2.9, NVFP4 4.4),
-// 4096 x 4096 12.7 - 13.2 (13.6, 13.1, 13.0), 8192 x 8192 42.9 - 43.6 (45.7, 44.4, 43.1).
+// it equals the whole-tensor kernels or beats them at most sizes; whole_is_faster says where it does not.
 #include "common.h"
 #include "blockfp_ops.h"
 #include "nvfp4_ops.h"
@@ -183,10 +182,34 @@ static int dispatch_row(const void* x, void* y, int64_t rows, int64_t k, const v
     return MO_OK;
 }
 
+// Where rows do not matter (no scale per column, 16-byte alignment, one amax at hand) and the kernels for whole
+// tensors are the faster ones.  A workgroup of theirs takes twice the chunks, so from 2^23 to 2^24 elements they fill
+// the chip in one round where the row kernel starts a second: bf16 32 MB FP8 11.1 us against 12.2, INT8 11.7 and
+// 12.0, fp16 11.5 and 12.5, 11.5 and 12.7.  In fp16, whose conversions cost the row kernel more, from 2^20 (4 MB
+// 3.6 and 3.8; 16 MB 7.0 and 6.9), and in fp32 as long as the tensor is below 1 GB (16 MB 7.4 and 7.3, 32 MB 13.8 and
+// 14.7, 128 MB 51.3 and 52.5, 512 MB 204 and 204, 1 GB 410 and 419, 4 GB 1737 and 1715).  Elsewhere the row kernel is equal or
+// faster (bf16 INT8 1 MB 3.2 and 2.7, 256 MB 86.6 and 82.4, FP8 84.5 and 83.4).  Same bits either way.
+static bool whole_is_faster(int64_t n, int dtype) {
+    if (dtype == MO_F32) return n >= (1ll << 22) && n <= (1ll << 28);
+    return n > (dtype == MO_F16 ? 1ll << 20 : 1ll << 23) && n <= (1ll << 24);
+}
+
 // amax_dtype: a type, or parts (kAmaxParts + their number)
 int row_qdq(const void* x, void* y, int64_t rows, int64_t k, int dtype, const void* pre, int kind, int p0, int p1,
             int p2, const void* amax, int amax_dtype, hipStream_t s) {
     int rc;
+    if (!pre && amax_dtype < kAmaxParts) {
+        const int64_t n = rows * k;
+        const bool aligned = (((uintptr_t)x | (uintptr_t)y) & 15u) == 0;
+        if (kind == MO_ROW_FP8 && aligned && whole_is_faster(n, dtype))
+            return mo_fp8_qdq(x, y, 1, 1, n, dtype, amax, amax_dtype, p0, s);
+        if (kind == MO_ROW_INT && aligned && whole_is_faster(n, dtype))
+            return mo_int_qdq(x, y, 1, 1, n, dtype, amax, amax_dtype, p0, p1, p2, s);
+        if (kind == MO_ROW_NVFP4) {
+            rc = nvfp4_qdq_whole(x, y, n, k, dtype, p0, p1, amax, amax_dtype, s);
+            if (rc != MO_ERR_UNSUPPORTED) return rc;
+        }
+    }
     switch (dtype) {
         case MO_F32: rc = dispatch_row<MO_F32>(x, y, rows, k, pre, kind, p0, p1, p2, amax, amax_dtype, s); break;
         case MO_F16: rc = dispatch_row<MO_F16>(x, y, rows, k, pre, kind, p0, p1, p2, amax, amax_dtype, s); break;

@@ -52,6 +52,25 @@ def test_equals_the_whole_tensor_kernels(dtype, kind, p0, p1, p2, rows, k, pre):
     assert torch.equal(_bits(got), _bits(_whole(seen, kind, p0, p1, p2, amax)))
 
 
+# both sides of the sizes between which a whole tensor without a scale goes to the kernel for whole tensors
+@pytest.mark.parametrize("dtype,line", [(torch.float32, 1 << 22), (torch.float32, 1 << 28), (torch.float16, 1 << 20),
+                                        (torch.float16, 1 << 24), (torch.bfloat16, 1 << 23), (torch.bfloat16, 1 << 24)])
+@pytest.mark.parametrize("kind,p0,p1,p2", KINDS[:5])
+def test_large_tensors_equal_their_parts(dtype, line, kind, p0, p1, p2):
+    g = torch.Generator(DEV).manual_seed(p0)
+    x = torch.randn(line + 8, device=DEV, generator=g).to(dtype)
+    if dtype != torch.float32:
+        x[:65536] = torch.arange(65536, device=DEV, dtype=torch.int32).to(torch.int16).view(dtype)   # every value
+    x[-3], x[-2] = float("nan"), float("inf")
+    amax = torch.full((1,), 2.5, device=DEV)
+    step = 1 << 19
+    parts = torch.cat([_hip.row_qdq(t.clone(), None, kind, p0, p1, p2, amax) for t in x.split(step)])
+    for n in (line - 8, line, line + 8):
+        got = _hip.row_qdq(x[:n], None, kind, p0, p1, p2, amax)
+        same = (got == parts[:n]) | (torch.isnan(got) & torch.isnan(parts[:n]))
+        assert bool(same.all()) and torch.equal(torch.signbit(got), torch.signbit(parts[:n]))
+
+
 @pytest.mark.parametrize("kind,p0,p1,p2", [(_hip.MO_ROW_FP8, 1, 0, 0), (_hip.MO_ROW_NVFP4, 16, 0, 0), (_hip.MO_ROW_MX, 32, 0, 0)])
 def test_unaligned_base_and_non_finite_blocks(kind, p0, p1, p2):
     g = torch.Generator().manual_seed(1)
