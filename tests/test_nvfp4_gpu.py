@@ -204,28 +204,51 @@ def test_multi_tensor_plan_matches_single_calls():
         assert_bits_equal(wsf[i].cpu(), wo, f"wsf {i}")
 
 
-@pytest.mark.parametrize("mode", [0, 1])
-def test_fake_quant_edge_cases_and_all_patterns(mode):
-    def want(x, amax):
-        if mode == 0:
-            return fake_quant.nvfp4_fake_quant(x, amax, 16)
-        wsf2 = amax.float() / 2688.0
-        wsf, _ = qtensor.nvfp4_block_scales(x, 16, wsf2)
-        p, _, _ = qtensor.nvfp4_quantize(x, 16, wsf, wsf2)
-        return qtensor.nvfp4_dequantize(p, wsf, wsf2, 16, x.shape, x.dtype)
+def _fake_quant_oracle(x, amax, mode):
+    if mode == 0:
+        return fake_quant.nvfp4_fake_quant(x, amax, 16)
+    wsf2 = amax.float() / 2688.0
+    wsf, _ = qtensor.nvfp4_block_scales(x, 16, wsf2)
+    p, _, _ = qtensor.nvfp4_quantize(x, 16, wsf, wsf2)
+    return qtensor.nvfp4_dequantize(p, wsf, wsf2, 16, x.shape, x.dtype)
 
-    x = _edge_tensor()
-    amax = reduce.reduce_amax(x)
-    assert_bits_equal(_hip.nvfp4_qdq(x.to(DEV), amax.to(DEV), 16, mode).cpu(), want(x, amax), "edge tensor")
+
+def _all_patterns(pilot):
+    """Every finite bf16 value in a block of 16 whose first element is ``pilot``."""
     allv = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
     finite = allv[torch.isfinite(allv.float())]
     finite = finite[: finite.numel() // 15 * 15].reshape(-1, 15)
+    return torch.cat([torch.full((finite.shape[0], 1), pilot, dtype=torch.bfloat16), finite], dim=1).contiguous()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_fake_quant_edge_cases_and_all_patterns(mode):
+    x = _edge_tensor()
+    amax = reduce.reduce_amax(x)
+    assert_bits_equal(_hip.nvfp4_qdq(x.to(DEV), amax.to(DEV), 16, mode).cpu(), _fake_quant_oracle(x, amax, mode), "edge tensor")
     for pilot in (1.0, 0.013):
-        col = torch.full((finite.shape[0], 1), pilot, dtype=torch.bfloat16)
-        x = torch.cat([col, finite], dim=1).contiguous()
+        x = _all_patterns(pilot)
         amax = torch.tensor(pilot * 4, dtype=torch.bfloat16)
-        assert_bits_equal(_hip.nvfp4_qdq(x.to(DEV), amax.to(DEV), 16, mode).cpu(), want(x, amax),
+        assert_bits_equal(_hip.nvfp4_qdq(x.to(DEV), amax.to(DEV), 16, mode).cpu(), _fake_quant_oracle(x, amax, mode),
                           f"all patterns pilot={pilot}")
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("blocks", [(1 << 20) - 1, 1 << 20, (1 << 20) + 77, 1 << 23, (1 << 23) + 1])
+def test_fake_quant_of_large_tensors(mode, blocks):
+    """The edge cases and all patterns over and over, at both ends of the sizes that take the kernel for whole
+    tensors, with a last workgroup of 1, 77 and 256 blocks."""
+    edge = _edge_tensor().reshape(-1, 16)
+    amax = reduce.reduce_amax(edge)
+    for part, amax in ((edge, amax), (_all_patterns(1.0), torch.tensor(4.0).bfloat16()),
+                       (_all_patterns(0.013), torch.tensor(0.052).bfloat16())):
+        want = _fake_quant_oracle(part, amax, mode).to(DEV)
+        times, rest = divmod(blocks, part.shape[0])
+        x = torch.cat([part.to(DEV).repeat(times, 1), part[:rest].to(DEV)])
+        got = _hip.nvfp4_qdq(x, amax.to(DEV), 16, mode)
+        for y, w in ((got[:blocks - rest].view(times, *part.shape), want), (got[blocks - rest:], want[:rest])):
+            same = (y.view(torch.int16) == w.view(torch.int16)) | (torch.isnan(y) & torch.isnan(w))
+            assert bool(same.all())
 
 
 def test_dequantize_every_code_and_scale():
