@@ -1,11 +1,14 @@
-"""Row-wise fake quantisation (pre-scaled, ragged or unaligned rows) against the kernels for whole tensors,
-which the oracle tests pin, on zero-padded copies; bit for bit."""
+"""Row-wise fake quantisation (pre-scaled, ragged or unaligned rows): integers and FP8 against the kernels for
+whole tensors, which the oracle tests pin, NVFP4 and the MX formats, whose other entry points run the same
+kernel, against the oracle; bit for bit."""
 
 import pytest
 import torch
 import torch.nn.functional as F
 
+from conftest import assert_bits_equal
 from modelopt_amd import _hip
+from oracle import fake_quant, mx, qtensor
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -13,19 +16,20 @@ DTYPES = [torch.bfloat16, torch.float16, torch.float32]
 MX = {name: i for i, name in enumerate(_hip.ELEM_FORMATS[:-1])}
 
 
-def _bits(t):
-    return t.contiguous().view(torch.int32 if t.element_size() == 4 else torch.int16)
-
-
 def _whole(x, kind, p0, p1, p2, amax):
     if kind == _hip.MO_ROW_INT:
         return _hip.int_qdq(x, amax, 1, 1, x.numel(), p0, p1, p2)
     if kind == _hip.MO_ROW_FP8:
         return _hip.fp8_qdq(x, amax, 1, 1, x.numel(), bool(p0))
-    k, block = x.shape[-1], p0
-    padded = F.pad(x, (0, -k % block)).contiguous()
-    y = _hip.nvfp4_qdq(padded, amax, block, p1) if kind == _hip.MO_ROW_NVFP4 else _hip.block_fp_qdq(padded, block, p1)
-    return y[..., :k]
+    x = x.cpu()
+    if kind == _hip.MO_ROW_MX:
+        return mx.block_fp_fake_quant(x, p0, _hip.ELEM_FORMATS[p1])
+    if p1 == 0:
+        return fake_quant.nvfp4_fake_quant(x, amax.cpu(), p0)
+    k = x.shape[-1]
+    padded, wsf2 = F.pad(x, (0, -k % p0)), amax.cpu().float().reshape(()) / 2688.0
+    packed, wsf, _ = qtensor.nvfp4_quantize(padded, p0, wsf2=wsf2)
+    return qtensor.nvfp4_dequantize(packed, wsf, wsf2, p0, padded.shape, x.dtype)[..., :k]
 
 
 KINDS = ([(_hip.MO_ROW_INT, 8, 0, 0), (_hip.MO_ROW_INT, 4, 1, 0), (_hip.MO_ROW_INT, 16, 0, 1),
@@ -49,7 +53,7 @@ def test_equals_the_whole_tensor_kernels(dtype, kind, p0, p1, p2, rows, k, pre):
     seen = x * s if pre else x
     amax = None if kind == _hip.MO_ROW_MX else (0.8 * seen.abs().amax()).float().reshape(1)
     got = _hip.row_qdq(x, s, kind, p0, p1, p2, amax)
-    assert torch.equal(_bits(got), _bits(_whole(seen, kind, p0, p1, p2, amax)))
+    assert_bits_equal(got.cpu(), _whole(seen, kind, p0, p1, p2, amax).cpu().contiguous(), "qdq")
 
 
 # both sides of the sizes between which a whole tensor without a scale goes to the kernel for whole tensors
@@ -71,18 +75,18 @@ def test_large_tensors_equal_their_parts(dtype, line, kind, p0, p1, p2):
         assert bool(same.all()) and torch.equal(torch.signbit(got), torch.signbit(parts[:n]))
 
 
-@pytest.mark.parametrize("kind,p0,p1,p2", [(_hip.MO_ROW_FP8, 1, 0, 0), (_hip.MO_ROW_NVFP4, 16, 0, 0), (_hip.MO_ROW_MX, 32, 0, 0)])
-def test_unaligned_base_and_non_finite_blocks(kind, p0, p1, p2):
+@pytest.mark.parametrize("kind,p0,p1,p2", [(_hip.MO_ROW_FP8, 1, 0, 0), (_hip.MO_ROW_MX, 32, 0, 0)]
+                         + [(_hip.MO_ROW_NVFP4, b, m, 0) for b in (8, 16, 32) for m in (0, 1)]
+                         + [(_hip.MO_ROW_MX, b, f, 0) for b, f in zip((8, 16, 32, 8, 16, 32, 8, 16), list(MX.values())[1:])])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_unaligned_base_and_non_finite_blocks(dtype, kind, p0, p1, p2):
     g = torch.Generator().manual_seed(1)
-    flat = torch.randn(40 * 96 + 1, generator=g).bfloat16()
+    flat = torch.randn(40 * 96 + 1, generator=g).to(dtype)
     flat[5], flat[700], flat[1500] = float("nan"), float("inf"), float("-inf")
-    x = flat.to(DEV)[1:].view(40, 96)                 # two bytes off a 16-byte boundary
+    x = flat.to(DEV)[1:].view(40, 96)                 # an element off a 16-byte boundary
     amax = torch.full((1,), 3.0, device=DEV)
     got = _hip.row_qdq(x, None, kind, p0, p1, p2, None if kind == _hip.MO_ROW_MX else amax)
-    want = _whole(x.clone(), kind, p0, p1, p2, amax)
-    assert torch.equal(torch.isnan(got), torch.isnan(want))
-    keep = ~torch.isnan(want)
-    assert torch.equal(_bits(got[keep]), _bits(want[keep]))
+    assert_bits_equal(got.cpu(), _whole(x.clone(), kind, p0, p1, p2, amax).cpu(), "qdq")
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -142,17 +146,19 @@ def test_a_pre_quant_scale_equals_the_scaled_input(name, dtype, form):
     assert torch.equal(got[keep], want[keep])
 
 
-@pytest.mark.parametrize("name", FORMATS)
-@pytest.mark.parametrize("dtype", DTYPES + [torch.float64])
-@pytest.mark.parametrize("form", ["plain", "one_dim", "strided", "unaligned", "parameter", "scaled", "dynamic", "amax_1x1",
-                                  "amax_on_cpu", "nan_overflow", "inference"])
+FORMS = ["plain", "one_dim", "strided", "unaligned", "parameter", "scaled", "dynamic", "amax_1x1", "amax_on_cpu",
+         "nan_overflow", "inference"]
+# float64 is taken with a calibrated abs-max only, without blocks and scales
+DIRECT = [(name, dtype, form) for name in FORMATS for dtype in DTYPES + [torch.float64] for form in FORMS
+          if dtype != torch.float64 or not (FORMATS[name].get("block_sizes") or form in ("scaled", "dynamic"))]
+
+
+@pytest.mark.parametrize("name,dtype,form", DIRECT)
 def test_the_direct_route_equals_the_steps_of_forward(name, dtype, form, monkeypatch):
     from modelopt_amd.torch.quantization.config import QuantizerAttributeConfig
     from modelopt_amd.torch.quantization.nn import TensorQuantizer
     from modelopt_amd.torch.quantization.overflow import set_fp8_overflow_behavior
 
-    if dtype == torch.float64 and (FORMATS[name].get("block_sizes") or form in ("scaled", "dynamic")):
-        pytest.skip("float64 is taken with a calibrated abs-max only, without blocks and scales")
     flat = torch.randn(11 * 96 + 1, generator=torch.Generator().manual_seed(6)).mul_(3).to(dtype).to(DEV)
     x = (flat[1:] if form == "unaligned" else flat[:-1]).view(11, 96)
     x = {"one_dim": x[3], "strided": x[:, :].t().contiguous().t(), "parameter": torch.nn.Parameter(x)}.get(form, x)
