@@ -33,7 +33,6 @@ __device__ __forceinline__ float row_round(float v) {
 // The formats: `start` once per lane, `chunk` for 8 elements (zeros where the row has ended).
 template <bool SAT>
 struct RowFp8 {
-    static constexpr int lanes_lg = 0;   // lanes that share a block, as a power of two
     Fp8Op<true> op;
     Fp8Op<true>::Scale s;
     __device__ __forceinline__ void start(float amax) { s = op.make(amax); }
@@ -49,7 +48,6 @@ struct RowFp8 {
 };
 
 struct RowInt {
-    static constexpr int lanes_lg = 0;
     IntOp op;
     IntOp::Scale s;
     __device__ __forceinline__ void start(float amax) { s = op.make(amax); }
@@ -68,7 +66,7 @@ struct RowInt {
 
 template <int BS, int MODE>
 struct RowNvfp4 {
-    static constexpr int lanes_lg = BS == 8 ? 0 : (BS == 16 ? 1 : 2);
+    static constexpr int lanes_lg = BS == 8 ? 0 : (BS == 16 ? 1 : 2);   // lanes that share a block, as a power of two
     float gs, gs_safe;
     __device__ __forceinline__ void start(float amax) {
         gs = amax / 2688.0f;
@@ -182,6 +180,19 @@ static int dispatch_row(const void* x, void* y, int64_t rows, int64_t k, const v
     return MO_OK;
 }
 
+static int check_row_format(int kind, int p0, int p1) {
+    const bool block = p0 == 8 || p0 == 16 || p0 == 32;
+    switch (kind) {
+        case MO_ROW_INT: return p0 < 1 || p0 > 24 ? MO_ERR_ARG : MO_OK;
+        case MO_ROW_FP8: return MO_OK;
+        case MO_ROW_NVFP4:
+            if (p1 != 0 && p1 != 1) return MO_ERR_ARG;
+            return block ? MO_OK : MO_ERR_UNSUPPORTED;
+        case MO_ROW_MX: return !block || p1 < MO_EF_E4M3 || p1 > MO_EF_E2M3 ? MO_ERR_UNSUPPORTED : MO_OK;
+        default: return MO_ERR_UNSUPPORTED;
+    }
+}
+
 // Where rows do not matter (no scale per column, 16-byte alignment, one amax at hand) and the kernels for whole
 // tensors are the faster ones.  A workgroup of theirs takes twice the chunks, so from 2^23 to 2^24 elements they fill
 // the chip in one round where the row kernel starts a second: bf16 32 MB FP8 11.1 us against 12.2, INT8 11.7 and
@@ -225,18 +236,8 @@ extern "C" int mo_row_qdq(const void* x, void* y, int64_t rows, int64_t k, int d
                           int kind, int p0, int p1, int p2, const void* amax, int amax_dtype, void* stream) {
     if (rows < 0 || k < 0) return MO_ERR_ARG;
     if (dtype < MO_F32 || dtype > MO_BF16 || amax_dtype < MO_F32 || amax_dtype > MO_BF16) return MO_ERR_DTYPE;
-    switch (kind) {
-        case MO_ROW_INT: if (p0 < 1 || p0 > 24) return MO_ERR_ARG; break;
-        case MO_ROW_FP8: break;
-        case MO_ROW_NVFP4:
-            if (p1 != 0 && p1 != 1) return MO_ERR_ARG;
-            if (p0 != 8 && p0 != 16 && p0 != 32) return MO_ERR_UNSUPPORTED;
-            break;
-        case MO_ROW_MX:
-            if ((p0 != 8 && p0 != 16 && p0 != 32) || p1 < MO_EF_E4M3 || p1 > MO_EF_E2M3) return MO_ERR_UNSUPPORTED;
-            break;
-        default: return MO_ERR_UNSUPPORTED;
-    }
+    const int format = mo::check_row_format(kind, p0, p1);
+    if (format != MO_OK) return format;
     if (rows == 0 || k == 0) return MO_OK;
     if (!x || !y || (kind != MO_ROW_MX && !amax)) return MO_ERR_ARG;
     const uintptr_t need = dtype == MO_F32 ? 3u : 1u;
@@ -250,15 +251,8 @@ extern "C" int mo_dynamic_qdq(const void* x, void* y, int64_t rows, int64_t k, i
                               int p2, void* parts, void* stream) {
     if (rows < 0 || k < 0) return MO_ERR_ARG;
     if (dtype < MO_F32 || dtype > MO_BF16) return MO_ERR_DTYPE;
-    switch (kind) {
-        case MO_ROW_INT: if (p0 < 1 || p0 > 24) return MO_ERR_ARG; break;
-        case MO_ROW_FP8: break;
-        case MO_ROW_NVFP4:
-            if (p1 != 0 && p1 != 1) return MO_ERR_ARG;
-            if (p0 != 8 && p0 != 16 && p0 != 32) return MO_ERR_UNSUPPORTED;
-            break;
-        default: return MO_ERR_UNSUPPORTED;
-    }
+    const int format = kind == MO_ROW_MX ? MO_ERR_UNSUPPORTED : mo::check_row_format(kind, p0, p1);
+    if (format != MO_OK) return format;
     if (rows == 0 || k == 0) return MO_OK;
     if (!x || !y || !parts) return MO_ERR_ARG;
     if (((uintptr_t)x | (uintptr_t)y) & 15u) return MO_ERR_UNSUPPORTED;

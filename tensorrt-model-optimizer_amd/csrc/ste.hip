@@ -132,11 +132,10 @@ static int launch_ste(const void* x, const void* dy, void* dx, int64_t outer, in
     int64_t tiles = ((n >> 3) + kSteTileChunks - 1) / kSteTileChunks;
     if (tiles < 1) tiles = 1;
     if (aligned && (axis == 1 || inner % 8 == 0) && tiles <= 0x7FFFFFFF) {
-        const size_t cap = mo::ballast_bytes("ste_mask_kernel", 0);
         if (axis == 1)
-            ste_mask_kernel<DT, STE_TENSOR><<<(unsigned)tiles, 256, cap, s>>>(x, dy, dx, n, axis, inner, amax, amax_dtype, narrow);
+            ste_mask_kernel<DT, STE_TENSOR><<<(unsigned)tiles, 256, 0, s>>>(x, dy, dx, n, axis, inner, amax, amax_dtype, narrow);
         else
-            ste_mask_kernel<DT, STE_CHUNK><<<(unsigned)tiles, 256, cap, s>>>(x, dy, dx, n, axis, inner, amax, amax_dtype, narrow);
+            ste_mask_kernel<DT, STE_CHUNK><<<(unsigned)tiles, 256, 0, s>>>(x, dy, dx, n, axis, inner, amax, amax_dtype, narrow);
         return MO_OK;
     }
     int64_t b = (n + 255) / 256;

@@ -20,7 +20,7 @@
 // Measured on a 14336 x 4096 bf16 weight with an amax a row, against the library's product and mo_ste_mask: 64
 // tokens 44 us (89) = 5.3 TB/s of weight and gradient, 256 tokens 67 (109), 512 tokens 96 (140) = 0.62
 // PFLOP/s, 1024 tokens 179 (200).  Up to some 100 tokens memory bounds it, beyond that the loads of the
-// operands: 64 KB in flight a compute unit, a quarter of them past L2.  More than three wavefronts a
+// operands: 96 KB in flight a compute unit (128 bytes a lane), a quarter of them past L2.  More than three wavefronts a
 // SIMD do not fit the registers (128 of them spill: 243 us at 512 tokens).
 #include "common.h"
 
