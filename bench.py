@@ -317,8 +317,8 @@ def single_tensor_configs(torch, steps, warmup):
             model = OneLinear(weight)
             # a few milliseconds of unrelated matrix work first, as the layers before this one
             # would be in a model-sized run.  (The clocks still fall back during the half
-            # millisecond of host work before the first big kernel: the clip search kernel, 1.35 ms
-            # in a train of launches, takes 1.85 ms inside this call.)
+            # millisecond of host work before the first big kernel: the clip search kernel, 0.49 ms
+            # in a train of launches, takes 0.56 ms inside this call.)
             for _ in range(12):
                 busy @ busy
             torch.cuda.synchronize()
@@ -367,9 +367,9 @@ def single_tensor_configs(torch, steps, warmup):
         "peak_TFLOPs": 2500.0, "frac": round(kflops / ms / 1e9 / 2500.0, 4)}
 
     # AWQ clip search on the same weight: 11 clip ratios x every 128-wide block, 64 calibration
-    # tokens, one launch.  Vector-ALU bound: two vector instructions per rounded product (one
-    # fp32 multiply each; one conversion to bf16 and one v_dot2c_f32_bf16 add per pair), against
-    # an issue peak of one instruction per lane and clock: 256 CUs x 64 lanes x 2.4 GHz
+    # tokens, one launch.  Bound by the issue of matrix instructions: 2048 rounded products are one
+    # outer-product instruction and four that sum, 128 cycles of a SIMD, beside 64 conversions on
+    # its vector ALU (half an instruction per product): 1024 SIMDs at 2.4 GHz
     ratios = [round(float(v), 2) for v in torch.arange(0.5, 1.0, 0.05)] + [1.0]
     x64 = x3[::8].contiguous()
     w_amax = w3.view(-1, 128).abs().amax(1, keepdim=True)
@@ -380,9 +380,9 @@ def single_tensor_configs(torch, steps, warmup):
     ms = train(clip, reps=20)
     products = 4096 * 4096 * 64 * (len(ratios) + 1)
     out["awq_clip_search_kernel_11_ratios_4096x4096_64_tokens"] = {
-        "ms": round(ms, 4), "rounded_products_per_s": round(products / ms * 1e3, 0), "bound": "valu",
-        "vector_instructions_per_product": 2.0, "peak_lane_instructions_per_s": 39.32e12,
-        "frac": round(2.0 * products / ms * 1e3 / 39.32e12, 4)}
+        "ms": round(ms, 4), "rounded_products_per_s": round(products / ms * 1e3, 0), "bound": "mfma",
+        "matrix_cycles_per_2048_products": 128, "peak_products_per_s": 39.32e12,
+        "frac": round(products / ms * 1e3 / 39.32e12, 4)}
     cfg = copy.deepcopy(mtq.INT4_AWQ_CFG)
     cfg["algorithm"] = {"method": "awq_clip"}
     out["awq_clip_4096x4096_end_to_end_ms"] = round(end_to_end(w3, x3, cfg) * 1e3, 3)
