@@ -7,7 +7,7 @@
 // contiguous bytes of codes.  No LDS, no cross-wave traffic.
 //
 // Algorithmic bytes per element (bf16 in): quantize 2 + 1/2 + 1/16; dequantize 1/2 + 1/16 + 2;
-// quantize-dequantize 2 + 2 (bf16 with whole 16-element blocks; everything else is in rowqdq.hip).
+// quantize-dequantize 2 + 2 (bf16 in whole blocks of 16, 32 to 256 MB; everything else is in rowqdq.hip).
 #include "common.h"
 #include "nvfp4_ops.h"
 
