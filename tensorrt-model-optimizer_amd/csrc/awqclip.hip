@@ -793,7 +793,7 @@ extern "C" int mo_awq_clip_losses(const void* x, int64_t tokens, const void* w, 
         //         142 with 3, 149 with 4; 1024 x 1024, 256: 156, 91 with 2, 56 with 4, 59 with 8
         //   fp16  4096 x 4096, 2048 wavefronts: 506 us, 444 with 2 shares, 465 with 4; 1024 x 4096, 512:
         //         313, 148 with 4, 162 with 8; 1024 x 1024, 128: 280, 99 with 4, 76 with 8, 72 with 11
-        // (boxes differ by some 8 %.)  What bounds the bf16 form: a step of 2048 products is 128 cycles of
+        // (cards differ by some 8 %.)  What bounds the bf16 form: a step of 2048 products is 128 cycles of
         // matrix instructions and about 110 of vector instructions plus 40 of the port that issues both;
         // measured 180.
         const int64_t sets = (int64_t)grid.x * grid.y * mo::kClipWaves;
