@@ -11,20 +11,28 @@
 // contraction; what the matrix cores can do is make the products (an outer product per column j,
 // whose fp32 result is exact for 16-bit operands) and add them up once they are rounded (a
 // contraction with a 0 / 1 matrix).  Issue costs, measured per wavefront instruction: 4.5 cycles for
-// v_mul_f32, v_cvt_pk_bf16_f32, v_pk_mul_f16 and v_dot2c, 16 cycles for a 16x16x32 and 32 for a
-// 32x32x16 matrix instruction, which run beside the vector instructions of other wavefronts and take
-// about 8 cycles of the issue port themselves.
+// v_mul_f32, v_cvt_pk_bf16_f32, v_pk_mul_f16 and v_dot2c, 16 cycles for a 16x16x32, 32 for a
+// 32x32x16 and 64 for a 32x32x4 (two blocks) matrix instruction, which run beside the vector instructions of
+// other wavefronts and take about 8 cycles of the issue port themselves.
 //   bf16: products on the matrix cores, one conversion per two products on the vector ALU, sums on the
 //         matrix cores (clip_losses_bf16): 0.5 vector instructions per product where multiply,
 //         convert and v_dot2c took 2.
 //   fp16: v_pk_mul_f16 rounds two products at once, sums on the matrix cores (clip_losses_f16): 0.5
 //         vector instructions per product where multiply, round and add took about 4.
 //   fp32: no rounding to do, one multiply and one add per product (clip_losses_f32).
+// A sum by selection leaves most of a matrix instruction idle: a dense one takes 512 products and adds two of them to
+// each of 256 sums.  The sparse form (v_smfmac, two of every four k) takes 1024 in the same 16 cycles: the
+// operand that says which is the sparse one, the products are the dense one.  It adds the two pairs of a sum one
+// after the other and leaves the bits of two dense instructions.
+// Measured, 4096 x 4096, 64 tokens, 11 ratios, dense / sparse: bf16 blocks of 128 495 / 400 - 414 us, of 64 520 / 425, of 16
+// 620 / 517; fp16 442 / 440, 436 / 418, 608 / 605.  bf16 blocks of 32 keep the dense form: their chains are so short
+// that the words held for the second step and the fold of the chains do not fit the registers of three wavefronts
+// a SIMD (50 spill: 1500 us against 537).
 // The instruction adds a pair of products to an output with one rounding, as v_dot2c does.  Its sums are made
 // in chains of a quarter of a block (but for blocks of 16), as four chains of v_dot2c made them: one
 // chain through a block of 128 rounds at twice the magnitude, and measured against sums in 64 bits 41 % more
 // blocks had an output that fell on the other side of a rounding to bf16 (1199 of 1.57 million; 852 with
-// quarters, 856 with v_dot2c).  What that costs: bf16 blocks of 128 3 %, of 64 and of 32 5 %.
+// quarters, 856 with v_dot2c).
 // Measured figures stand at the launch below.
 #include "common.h"
 #include "qdq_ops.h"
@@ -42,7 +50,9 @@ struct ClipRatios {
 };
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x16_t __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x16_t __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x32_t __attribute__((ext_vector_type(32)));
@@ -113,16 +123,33 @@ __device__ __forceinline__ float clip_with_kind(float sum, uint32_t kind) {
     return kind ? u2f(special) : sum;
 }
 
+// The 0 / 1 operand A of a sum, constant through a kernel.  As B the instruction takes eight words of a lane, four sums
+// with two words each: word i and word 4 + i.  Row 4 g + i of A picks them out of lane group g (16 lanes), so that
+// lane l, register i of the result is the sum of the words of lane l: no value changes its lane.
+// Dense (16x16x32): the first four words only.
+__device__ __forceinline__ void clip_sum_operand(uint32_t one, uint32_t (&m)[4]) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m[i] = (lane & 15) == 4 * (lane >> 4) + i ? one : 0u;
+}
+// Sparse (16x16x64, two of every four k): B has the first words of lane group g at k = 8 g .. 8 g + 7, the second ones 32
+// behind; lane (h, row) of A holds k = 16 h .. 16 h + 15 as four pairs, each pair with the same two places among its four.
+__device__ __forceinline__ int clip_sum_operand_sparse(uint32_t one, uint32_t (&m)[4]) {
+    const int lane = threadIdx.x & 63, h = lane >> 4, g = (lane >> 2) & 3, i = lane & 3;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) m[p] = (h & 1) == (g >> 1) && p == (g & 1) * 2 + (i >> 1) ? one : 0u;
+    return (i & 1) ? 0xEEEE : 0x4444;   // places 2 and 3, or 0 and 1
+}
+
 // ------------------------------------------------------------------------------------- bf16
 // A wavefront owns 32 rows of one weight block and all tokens of a pass, in two tiles of 32.  For two
 // columns (j, j + 8) of the block, v_mfma_f32_32x32x4_2b_bf16 with the tokens as A, reduced to one of
 // its four k by zeroing the others, and the weights as B gives the exact products of 32 tokens x 32
 // rows in 32 registers: register i of the first half and of the second half are the same token and
-// row under j and j + 8.  One conversion rounds the two into a word.  Four such words of a lane (four
-// tokens) are an A operand of v_mfma_f32_16x16x32_bf16 in which every word is a k pair of its own; the
-// B operand, constant through the kernel, sends pair p to output column p, so the instruction adds
-// lo + hi of each of the 64 x 4 words to a sum of its own: lane l, register i of group a holds
-//   row 4 (l >> 4) + i + 16 ((l >> 2) & 1), token 8 a + 4 ((l >> 3) & 1) + (l & 3)
+// row under j and j + 8.  One conversion rounds the two into a word.  The words of two steps are the B
+// operand of v_smfmac_f32_16x16x64_bf16 (those of one of v_mfma_f32_16x16x32_bf16), four tokens at a time, and
+// their lo + hi go to a sum of their own in the same lane: lane l, register i of group a holds
+//   row l & 31, token 8 a + 4 (l >> 5) + i
 // of the tile.  The sums of the chains that have ended and the partial outputs of the unclipped block lie in
 // LDS, each lane's own: no barrier anywhere.  Folding stands where the products before it are used up, or
 // its operands would not fit the registers.  The weights are quantised as they are used, 16 columns at a
@@ -136,6 +163,7 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                                                  f32x4* __restrict__ parts, u32x2* __restrict__ org, ClipStep& at) {
     constexpr int NC = BS / 16;
     constexpr int HALVES = BS >= 32 ? BS / 32 : 2;   // of a chunk, in a chain of sums
+    constexpr bool SPARSE = !CAREFUL && BS != 32;
     constexpr int RUN = HALVES >= 2 ? HALVES / 2 : 1;   // chunks until the chains of both tiles have ended
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -145,12 +173,13 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
     if (row0 >= n) return true;
     int row = row0 + fr < n ? row0 + fr : n - 1;
     const float amax = load_scalar(w_amax, amax_dtype, (int64_t)row * nblk + b);
-    bf16x8_t pair_sum;
+    bf16x8_t picks;
+    int places = 0;
     {
         uint32_t m[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) m[i] = (lane & 15) == 4 * (lane >> 4) + i ? 0x3F803F80u : 0u;
-        __builtin_memcpy(&pair_sum, m, 16);
+        if constexpr (!SPARSE) clip_sum_operand(0x3F803F80u, m);
+        else places = clip_sum_operand_sparse(0x3F803F80u, m);
+        __builtin_memcpy(&picks, m, 16);
     }
     f32x32_t zero;
 #pragma unroll
@@ -238,12 +267,6 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                 __builtin_memcpy(&bv, bw, 8);
                 return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(av, bv, zero, 0, 0, 0);
             };
-            auto sum_words = [&](const uint32_t (&pw)[4], int m, int a, bool opens) {
-                bf16x8_t pv;
-                __builtin_memcpy(&pv, pw, 16);
-                const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc[m][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pv, pair_sum, opens ? none : acc[m][a], 0, 0, 0);
-            };
             if constexpr (CAREFUL) {
                 uint32_t kind[2] = {0, 0};   // two bits an output
 #pragma unroll 1
@@ -266,7 +289,9 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
 #pragma unroll
                                 for (int i = 0; i < 4; ++i)
                                     pw[i] = clip_kinds_bf16(f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]), pass == 0);
-                                sum_words(pw, m, a, false);
+                                bf16x8_t pv;
+                                __builtin_memcpy(&pv, pw, 16);
+                                acc[m][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(picks, pv, acc[m][a], 0, 0, 0);
                             }
                             __builtin_amdgcn_sched_barrier(0);
                             if ((c * 2 + (q >> 3)) % HALVES == HALVES - 1 && (q & 7) == 7) fold();
@@ -292,6 +317,7 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                         uint32_t wb[4], xb[2][4];
                         operands(wb, xb);
                         f32x32_t d = products(wb, xb, 0);
+                        uint32_t pw[4][8];   // of two steps
 #pragma unroll
                         for (int q = 0; q < 16; ++q) {
                             const int m = (q >> 2) & 1, half = cc * 2 + (q >> 3);
@@ -302,10 +328,21 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                             for (int a = 0; a < 4; ++a) {
-                                uint32_t pw[4];
 #pragma unroll
-                                for (int i = 0; i < 4; ++i) pw[i] = f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]);
-                                sum_words(pw, m, a, half % HALVES == 0 && (q & 3) == 0);
+                                for (int i = 0; i < 4; ++i)
+                                    pw[a][(SPARSE ? q & 1 : 0) * 4 + i] = f32x2_to_bf16x2(d[4 * a + i], d[16 + 4 * a + i]);
+                                if constexpr (!SPARSE) {
+                                    const bool opens = half % HALVES == 0 && (q & 3) == 0;
+                                    const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+                                    bf16x8_t pv;
+                                    __builtin_memcpy(&pv, pw[a], 16);
+                                    acc[m][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(picks, pv, opens ? none : acc[m][a], 0, 0, 0);
+                                } else if (q & 1) {
+                                    if (half % HALVES == 0 && (q & 3) == 1) acc[m][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                                    bf16x16_t pv;
+                                    __builtin_memcpy(&pv, pw[a], 32);
+                                    acc[m][a] = __builtin_amdgcn_smfmac_f32_16x16x64_bf16(picks, pv, acc[m][a], places, 0, 0);
+                                }
                             }
                             if (q + 1 < 16) d = ahead;
                             // Steps stay apart: left alone, the scheduler converts the first of the products
@@ -358,21 +395,10 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
                 at = {t0, v};
                 return false;
             }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {   // the other tokens of the rows: lane bits 0, 1 and 3
-                sum[i] += __shfl_xor(sum[i], 1, kWave);
-                sum[i] += __shfl_xor(sum[i], 2, kWave);
-                sum[i] += __shfl_xor(sum[i], 8, kWave);
-            }
-            if ((lane & 11) == 0) {
-                int r0_lane = row0 + 4 * (lane >> 4) + 16 * ((lane >> 2) & 1);
-                asm volatile("" : "+v"(r0_lane));   // or four addresses are kept through the sums
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = r0_lane + i;
-                    if (r < n) loss[((int64_t)v * n + r) * nblk + b] += sum[i] / (float)tokens;
-                }
-            }
+            float total = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+            total += __shfl_xor(total, 32, kWave);   // the other tokens of the row
+            const int r = row0 + fr;
+            if (lane < 32 && r < n) loss[((int64_t)v * n + r) * nblk + b] += total / (float)tokens;
         }
     }
     return true;
@@ -381,9 +407,8 @@ __device__ __forceinline__ bool clip_losses_bf16(const uint16_t* __restrict__ x,
 // ------------------------------------------------------------------------------------- fp16
 // A lane owns one row of one weight block, its quantised weights in registers, two a word; the
 // activations are uniform over the wavefront (scalar loads, two columns a word).  One v_pk_mul_f16 gives
-// two rounded products; the words of four tokens are an A operand of v_mfma_f32_16x16x32_f16 and are
-// summed as in the bf16 form: lane l, register i holds row 4 (l >> 4) + i + 16 ((l >> 2) & 3), token
-// l & 3 of the four.  The partial outputs of the unclipped block stay in LDS.
+// two rounded products; the words of four tokens are summed as in the bf16 form, two steps of a chain an
+// instruction: lane l, register i holds row l, token i of the four.  The partial outputs of the unclipped block stay in LDS.
 template <int BS, bool CAREFUL>
 __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, int tokens,
                                                 const uint16_t* __restrict__ w, int n, int k,
@@ -402,12 +427,13 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
     const int row = row0 + lane < n ? row0 + lane : n - 1;
     const uint16_t* wp = w + (int64_t)row * k + b * BS;
     const float amax = load_scalar(w_amax, amax_dtype, (int64_t)row * nblk + b);
-    f16x8_t pair_sum;
+    f16x8_t picks;
+    int places = 0;
     {
         uint32_t m[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) m[i] = (lane & 15) == 4 * (lane >> 4) + i ? 0x3C003C00u : 0u;
-        __builtin_memcpy(&pair_sum, m, 16);
+        if constexpr (CAREFUL) clip_sum_operand(0x3C003C00u, m);
+        else places = clip_sum_operand_sparse(0x3C003C00u, m);
+        __builtin_memcpy(&picks, m, 16);
     }
     const uint32_t* xw = (const uint32_t*)(x + b * BS);
     const int xstride = k / 2;
@@ -471,13 +497,8 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                     xr[i] = xw + (int64_t)(t0 + t) * xstride;
                 }
                 f32x4 acc[CHAINS];
-                auto sum_words = [&](const uint32_t (&pw)[4], int j) {
-                    f16x8_t pv;
-                    __builtin_memcpy(&pv, pw, 16);
-                    const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
-                    f32x4& c = acc[j % CHAINS];
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(pv, pair_sum, j < CHAINS ? none : c, 0, 0, 0);
-                };
+#pragma unroll
+                for (int c = 0; c < CHAINS; ++c) acc[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 auto sum_chains = [&]() {
                     f32x4 t = acc[0] + acc[1];
                     if constexpr (CHAINS == 4) t = t + (acc[2] + acc[3]);
@@ -497,7 +518,11 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                             uint32_t pw[4];
 #pragma unroll
                             for (int i = 0; i < 4; ++i) pw[i] = clip_kinds_f16(product(xr[i][at_j], wq[j]), pass == 0);
-                            sum_words(pw, j);
+                            f16x8_t pv;
+                            __builtin_memcpy(&pv, pw, 16);
+                            if (j < CHAINS) acc[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};   // of either pass
+                            f32x4& c = acc[j % CHAINS];
+                            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(picks, pv, c, 0, 0, 0);
                             __builtin_amdgcn_sched_barrier(0);
                         }
                         total = sum_chains();
@@ -508,6 +533,7 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                         }
                     }
                 } else {
+                    uint32_t pw[CHAINS][8];   // two steps of every chain
                     uint32_t cur[4][GW];
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
@@ -525,10 +551,16 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                         for (int j = 0; j < GW; ++j) {
-                            uint32_t pw[4];
+                            const int step = GW * g + j, second = step / CHAINS & 1;
+                            f32x4& c = acc[step % CHAINS];
+                            uint32_t(&of)[8] = pw[step % CHAINS];
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) pw[i] = product(cur[i][j], wq[GW * g + j]);
-                            sum_words(pw, GW * g + j);
+                            for (int i = 0; i < 4; ++i) of[4 * second + i] = product(cur[i][j], wq[step]);
+                            if (second) {
+                                f16x16_t pv;
+                                __builtin_memcpy(&pv, of, 32);
+                                c = __builtin_amdgcn_smfmac_f32_16x16x64_f16(picks, pv, c, places, 0, 0);
+                            }
                         }
                         __builtin_amdgcn_sched_barrier(0);
                         if (g + 1 < NG) {
@@ -553,11 +585,10 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                     const u32x2 o = org[g4 * kClipLanes];
                     const float og[4] = {f16_bits_to_f32(o.x & 0xFFFFu), f16_bits_to_f32(o.x >> 16),
                                          f16_bits_to_f32(o.y & 0xFFFFu), f16_bits_to_f32(o.y >> 16)};
-                    const bool counts = 4 * g4 + (lane & 3) < tc;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float d = clip_round<MO_F16>(out[i] - og[i]);
-                        sum[i] += counts ? d * d : 0.0f;
+                        sum[i] += 4 * g4 + i < tc ? d * d : 0.0f;
                     }
                 }
             }
@@ -568,18 +599,8 @@ __device__ __forceinline__ bool clip_losses_f16(const uint16_t* __restrict__ x, 
                 return false;
             }
             if (v < r0) continue;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {   // the other tokens of the rows: lane bits 0 and 1
-                sum[i] += __shfl_xor(sum[i], 1, kWave);
-                sum[i] += __shfl_xor(sum[i], 2, kWave);
-            }
-            if ((lane & 3) == 0) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = row0 + 4 * (lane >> 4) + i + 16 * ((lane >> 2) & 3);
-                    if (r < n) loss[((int64_t)v * n + r) * nblk + b] += sum[i] / (float)tokens;
-                }
-            }
+            const float all = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+            if (row0 + lane < n) loss[((int64_t)v * n + row) * nblk + b] += all / (float)tokens;
         }
     }
     return true;
@@ -787,15 +808,15 @@ extern "C" int mo_awq_clip_losses(const void* x, int64_t tokens, const void* w, 
         smem = (size_t)mo::kClipWaves * mo::kClipLanes * (dtype == MO_F16 ? mo::kClipTokens * 2 : 8 * (16 + 8));
         // A wavefront goes through all ratios unless there are too few of them to fill the chip; then
         // 2 to 11 of them share the ratios, each scoring the unclipped block once more.  11 ratios, 64
-        // tokens, blocks of 128 (before: one vector-ALU kernel for both types, 1070 / 2160 us on the
-        // first line):
+        // tokens, blocks of 128 (with dense sums, where the lines were drawn):
         //   bf16  4096 x 4096, 4096 wavefronts: 484 us, 503 with 2 shares; 1024 x 4096, 1024: 157, 145 with 2,
         //         142 with 3, 149 with 4; 1024 x 1024, 256: 156, 91 with 2, 56 with 4, 59 with 8
         //   fp16  4096 x 4096, 2048 wavefronts: 506 us, 444 with 2 shares, 465 with 4; 1024 x 4096, 512:
         //         313, 148 with 4, 162 with 8; 1024 x 1024, 128: 280, 99 with 4, 76 with 8, 72 with 11
-        // (cards differ by some 8 %.)  What bounds the bf16 form: a step of 2048 products is 128 cycles of
-        // matrix instructions and about 110 of vector instructions plus 40 of the port that issues both;
-        // measured 180.
+        // (cards differ by some 8 %; 1024 x 1024 now 45 and 66.)  What bounds the bf16 form: a step of 2048 products is
+        // 96 cycles of matrix instructions (64 of products) and about 90 of vector instructions (72 of conversions) plus
+        // 24 of the port that issues both; measured 160.  Higher priority for the wavefront at its matrix
+        // instructions (402 us), sums between the conversions (424) or products behind the first of them (444) win nothing.
         const int64_t sets = (int64_t)grid.x * grid.y * mo::kClipWaves;
         int64_t share = ((dtype == MO_BF16 ? 2048 : 3072) + sets - 1) / sets;
         if (dtype == MO_BF16 && share > 4) share = 4;
