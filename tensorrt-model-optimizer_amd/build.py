@@ -18,6 +18,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libmodelopt_hip.so")
+LAUNCH_SRC = os.path.join(HERE, "binding", "launch.cpp")   # compiled calls of the C ABI for the Python layer
+LAUNCH_LIB = os.path.join(HERE, "modelopt_amd", "_launch.so")
 PROBE_SRC = os.path.join(HERE, "probe", "l2_read_probe.hip")   # measurement aid for bench.py: its own library, outside csrc/
 PROBE_LIB = os.path.join(HERE, "libmodelopt_probe.so")
 HEADERS = [os.path.join(CSRC, h) for h in ("common.h", "qdq_ops.h", "awq_ops.h", "nvfp4_ops.h", "blockfp_ops.h")] + [
@@ -54,13 +56,36 @@ def _compile(src, force, obj_dir, extra):
     return out
 
 
+def _build_launch():
+    """The Python extension module: host code only, against the installed torch's headers."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    include = [os.path.join(HERE, "..", "include"), os.path.join(root, "include"),
+               os.path.join(root, "include", "torch", "csrc", "api", "include"),
+               os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+    subprocess.run(
+        ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wno-unused-function",
+         "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
+         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+         "-I", include[0], *(f for d in include[1:] for f in ("-isystem", d)), LAUNCH_SRC, "-o", LAUNCH_LIB,
+         "-L", os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"], check=True)
+
+
 def build(force=False, jobs=4, tuning=False):
     obj_dir = os.path.join(OBJ, "tuning") if tuning else OBJ
     lib = LIB.replace(".so", "_tuning.so") if tuning else LIB
     extra = ["-DMO_TUNING"] if tuning else []
     os.makedirs(obj_dir, exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        launch = None
+        if not tuning and (force or _stale(LAUNCH_LIB, [LAUNCH_SRC, HEADERS[-1]])):
+            launch = ex.submit(_build_launch)
         objs = list(ex.map(lambda s: _compile(s, force, obj_dir, extra), _sources()))
+        if launch is not None:
+            launch.result()
     if force or _stale(lib, objs):
         subprocess.run(["hipcc", "-shared", "-fPIC", "--offload-arch=gfx950", *objs, "-o", lib],
                        check=True)

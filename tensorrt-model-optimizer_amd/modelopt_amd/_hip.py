@@ -1,10 +1,13 @@
-"""ctypes binding of ``libmodelopt_hip.so`` (the C ABI declared in ``include/modelopt_hip.h``).
+"""Binding of ``libmodelopt_hip.so`` (the C ABI declared in ``include/modelopt_hip.h``): loaded with ctypes,
+called through ``_launch.so`` (``binding/launch.cpp``) where an entry point has a compiled call.
 
 There is no CPU or eager fallback behind this module: if the library is missing or a call
 fails, a ``RuntimeError`` is raised.  PyTorch is used only for device memory and streams.
 """
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -13,6 +16,7 @@ _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 # MODELOPT_AMD_LIB names another build of the same library (e.g. the tuning build of build.py)
 LIB_PATH = os.environ.get("MODELOPT_AMD_LIB") or os.path.join(os.path.dirname(_PKG_DIR),
                                                               "libmodelopt_hip.so")
+_LAUNCH_PATH = os.path.join(_PKG_DIR, "_launch.so")
 
 MO_F32, MO_F16, MO_BF16 = 0, 1, 2
 # per-call flags of the NVFP4 quantize entry points (enum mo_quantize_flags)
@@ -86,29 +90,40 @@ SIGNATURES = {
 }
 
 _lib = None
+_launch = None   # the compiled calls (binding/launch.cpp)
+_entry = {}      # entry point -> how it is called: compiled, or through ctypes
 
 
 def load():
     """Load the shared library once; raise if it has not been built."""
-    global _lib
+    global _lib, _launch
     if _lib is not None:
         return _lib
-    if not os.path.exists(LIB_PATH):
-        raise RuntimeError(
-            f"{LIB_PATH} not found: build it with `python tensorrt-model-optimizer_amd/build.py` "
-            "(hipcc, gfx950).  There is no fallback path."
-        )
+    for path in (LIB_PATH, _LAUNCH_PATH):
+        if not os.path.exists(path):
+            raise RuntimeError(
+                f"{path} not found: build it with `python tensorrt-model-optimizer_amd/build.py` "
+                "(hipcc, gfx950).  There is no fallback path."
+            )
     lib = ctypes.CDLL(LIB_PATH)
     for name, argtypes in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = ctypes.c_char_p if name == "mo_error_string" else _INT
+        _entry[name] = fn
+    if _launch is None:
+        loader = importlib.machinery.ExtensionFileLoader("_launch", _LAUNCH_PATH)
+        spec = importlib.util.spec_from_loader("_launch", loader)
+        _launch = importlib.util.module_from_spec(spec)
+        loader.exec_module(_launch)
+    for name in _launch.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES}):
+        _entry[name] = getattr(_launch, name)
     _lib = lib
     return lib
 
 
 def is_available() -> bool:
-    return os.path.exists(LIB_PATH)
+    return os.path.exists(LIB_PATH) and os.path.exists(_LAUNCH_PATH)
 
 
 def dtype_code(dt: torch.dtype) -> int:
@@ -190,23 +205,28 @@ class KernelTimer:
 
 def call(name: str, anchor: torch.Tensor, *args):
     """Invoke ``name`` with the device of ``anchor`` current; raise on a non-zero status."""
-    lib = _lib if _lib is not None else load()
+    if _lib is None:
+        load()
+    fn = _entry[name]
     if _timer is None and anchor.get_device() == torch._C._cuda_getDevice():
-        rc = getattr(lib, name)(*args)   # the common case, without the context manager's cost
+        rc = fn(*args)   # the common case, without the context manager's cost
     else:
         with torch.cuda.device(anchor.device):
             if _timer is None:
-                rc = getattr(lib, name)(*args)
+                rc = fn(*args)
             else:
                 start = torch.cuda.Event(enable_timing=True)
                 end = torch.cuda.Event(enable_timing=True)
                 start.record()
-                rc = getattr(lib, name)(*args)
+                rc = fn(*args)
                 end.record()
                 _timer.pairs.append((name, start, end))
     if rc != 0:
-        msg = lib.mo_error_string(rc).decode()
-        raise RuntimeError(f"{name} failed: {msg} (status {rc})")
+        _raise(name, rc)
+
+
+def _raise(name, rc):
+    raise RuntimeError(f"{name} failed: {_lib.mo_error_string(rc).decode()} (status {rc})")
 
 
 # ----------------------------------------------------------------------------- thin wrappers
@@ -471,6 +491,10 @@ def row_qdq(x, pre_scale, kind, p0=0, p1=0, p2=0, amax=None):
     """Fake quantisation of ``T(x * pre_scale)`` (``x`` itself when ``pre_scale`` is None) along the last dim
     in one pass; ``kind`` and ``p0`` .. ``p2`` as in ``mo_row_qdq``, ``amax`` one device element (None for
     ``MO_ROW_MX``)."""
+    if _timer is None and _launch is not None:
+        y = _launch.row_qdq(x, pre_scale, kind, p0, p1, p2, amax)
+        if y is not None:
+            return y if type(y) is not int else _raise("mo_row_qdq", y)
     if not x.is_cuda or pre_scale is not None or amax is not None:
         _require_device(x, pre_scale, amax)
     assert x.is_contiguous() and (pre_scale is None or (pre_scale.is_contiguous() and pre_scale.dtype == x.dtype
@@ -485,6 +509,10 @@ def row_qdq(x, pre_scale, kind, p0=0, p1=0, p2=0, amax=None):
 def dynamic_qdq(x, kind, p0=0, p1=0, p2=0):
     """Fake quantisation with the abs-max of ``x`` itself (``kind`` and ``p0`` .. ``p2`` as in ``row_qdq``, no
     MX formats) in two launches; None, with nothing launched, for an empty or unaligned tensor."""
+    if _timer is None and _launch is not None:
+        y = _launch.dynamic_qdq(x, kind, p0, p1, p2, AMAX_PARTS_BYTES)
+        if y is not None:
+            return y if type(y) is not int else _raise("mo_dynamic_qdq", y)
     _require_device(x)
     if x.numel() == 0 or x.data_ptr() % 16 or x.dtype not in _DTYPES:
         return None

@@ -596,7 +596,7 @@ class TensorQuantizer(nn.Module):
         no statistics to collect.  None for all else (``forward`` goes on, step by step).
 
         The steps of ``forward`` and the operator behind them cost the host 17 us, more than the
-        kernel up to some 4 million elements; this way 10.5.  A pre-quant scale is multiplied in
+        kernel up to some 4 million elements; this way 8.  A pre-quant scale is multiplied in
         the quantizer's launch (the product alone is a pass over the tensor: 2048 x 14336 bf16 to
         INT8 43.2 us in two launches, 22.7 in one = 5.2 TB/s), and a missing abs-max is taken as
         maxima of parts that the quantising launch folds (an accumulator would be filled, reduced
