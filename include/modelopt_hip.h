@@ -116,6 +116,15 @@ int mo_value_ranges(const void* const* xs, const int64_t* counts, const int* dty
 int mo_absmax_tensor_parts(const void* x, int64_t n, int dtype, float* acc, uint32_t* parts,
                            int64_t parts_capacity, int64_t* parts_written, void* stream);
 
+/* The end of a max calibration for n per-tensor calibrators in one launch (up to 48 of them and 96 runs of parts each):
+ * *accs[i] = the largest of itself and parts[s][0 .. words[s]) for s in first[i] .. first[i + 1) (bit patterns of
+ * non-negative floats, as mo_absmax_tensor_parts leaves them; a NaN is the largest), *outs[i] = the same in
+ * out_dtypes[i].  Replaces the conversion of each calibrator's maximum (MaxCalibrator.compute_amax,
+ * TQ/calib/max.py:86-93).  accs, outs, out_dtypes, first (n + 1 entries, first[0] = 0), parts and words are host arrays;
+ * what they point to is device memory.  MO_ERR_TOO_LARGE for more than 96 runs of one calibrator. */
+int mo_amax_fold(float* const* accs, void* const* outs, const int* out_dtypes, const int* first,
+                 const uint32_t* const* parts, const int64_t* words, int n, void* stream);
+
 /* The per-column case of mo_absmax (x viewed as [outer, axis], inner == 1) in two passes through
  * a caller-provided workspace: row slabs are reduced to partial[slabs, axis] with plain stores
  * (slabs <= partial_rows, chosen by the library), then the columns of that matrix are folded

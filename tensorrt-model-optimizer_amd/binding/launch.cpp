@@ -19,6 +19,7 @@
 #include <tuple>
 #include <type_traits>
 #include <utility>
+#include <vector>
 
 #include "modelopt_hip.h"
 
@@ -40,15 +41,17 @@ namespace {
     X(mo_awq_scale_activations) X(mo_awq_search_losses) X(mo_awq_search_losses_biased) X(mo_awq_best_clip)    \
     X(mo_abs_colsum) X(mo_abs_colsum_staged) X(mo_weight_scale_colsum) X(mo_sq_diff_sum)
 
+// Of those the ones that the calls below make themselves
+#define MO_INSIDE(X) X(mo_value_ranges) X(mo_amax_fold)
+
 enum Slot {
 #define X(f) k_##f,
-    MO_FUNCTIONS(X)
+    MO_FUNCTIONS(X) kCalls, kBeforeInside = kCalls - 1, MO_INSIDE(X) kSlots
 #undef X
-    kSlots
 };
 const char* const kNames[] = {
 #define X(f) #f,
-    MO_FUNCTIONS(X)
+    MO_FUNCTIONS(X) MO_INSIDE(X)
 #undef X
 };
 void* g_address[kSlots];
@@ -185,7 +188,98 @@ PyObject* dynamic_qdq(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// bind({name: address}): where the calls go; a name left out has no compiled call.  Returns the names bound.
+// value_ranges(tensors, most tensors, elements of a chunk, most chunks): (the kernel's output, [chunks of each tensor]),
+// or None where the list is not covered
+PyObject* value_ranges(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    int64_t most, chunk, most_chunks;
+    if (n != 4 || !PyList_Check(a[0]) || !g_address[k_mo_value_ranges]) Py_RETURN_NONE;
+    if (!convert(a[1], most) || !convert(a[2], chunk) || !convert(a[3], most_chunks)) return nullptr;
+    const int64_t count = PyList_GET_SIZE(a[0]);
+    if (count == 0 || count > most || count > 64) Py_RETURN_NONE;
+    const void* xs[64];
+    int64_t counts[64], chunks[64], total = 0;
+    int dtypes[64];
+    std::vector<at::Tensor> held;
+    for (int64_t i = 0; i < count; ++i) {
+        const at::Tensor* t = plain(PyList_GET_ITEM(a[0], i));
+        if (!t) Py_RETURN_NONE;
+        held.push_back(*t);
+        xs[i] = t->const_data_ptr();
+        counts[i] = t->numel();
+        dtypes[i] = code_of(t->scalar_type());
+        chunks[i] = std::max<int64_t>(1, (counts[i] + chunk - 1) / chunk);
+        total += chunks[i];
+    }
+    if (total > most_chunks) Py_RETURN_NONE;
+    at::Tensor out;
+    int rc;
+    {
+        pybind11::gil_scoped_release no_gil;
+        out = at::empty({3 * total}, held[0].options().dtype(at::kFloat));
+        rc = BOUND(mo_value_ranges)(xs, counts, dtypes, (int)count, out.mutable_data_ptr<float>(), total,
+                                    c10::hip::getCurrentHIPStream().stream());
+    }
+    if (rc != MO_OK) return PyLong_FromLong(rc);
+    pybind11::list each;
+    for (int64_t i = 0; i < count; ++i) each.append(chunks[i]);
+    return pybind11::make_tuple(pybind11::reinterpret_steal<pybind11::object>(THPVariable_Wrap(out)), each).release().ptr();
+    END_HANDLE_TH_ERRORS
+}
+
+// amax_fold([accumulator], [[parts]], [dtype code]): the folded maximum of each as a tensor of no dims in its type (mo_amax_fold),
+// a status, or None where an accumulator is not one fp32 element on the current GPU
+PyObject* amax_fold(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 3 || !PyList_Check(a[0]) || !PyList_Check(a[1]) || !PyList_Check(a[2]) || !g_address[k_mo_amax_fold]) Py_RETURN_NONE;
+    const Py_ssize_t count = PyList_GET_SIZE(a[0]);
+    if (count == 0 || PyList_GET_SIZE(a[1]) != count || PyList_GET_SIZE(a[2]) != count) Py_RETURN_NONE;
+    std::vector<at::Tensor> held, outs;
+    std::vector<float*> accs;
+    std::vector<void*> out_ptrs;
+    std::vector<int> dtypes, first{0};
+    std::vector<const uint32_t*> parts;
+    std::vector<int64_t> words;
+    static const at::ScalarType kTypes[3] = {at::kFloat, at::kHalf, at::kBFloat16};
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        const at::Tensor* acc = plain(PyList_GET_ITEM(a[0], i));
+        PyObject* runs = PyList_GET_ITEM(a[1], i);
+        int code;
+        if (!convert(PyList_GET_ITEM(a[2], i), code)) return nullptr;
+        if (!acc || acc->numel() != 1 || acc->scalar_type() != at::kFloat || !PyList_Check(runs) || code < MO_F32 || code > MO_BF16)
+            Py_RETURN_NONE;
+        held.push_back(*acc);
+        for (Py_ssize_t j = 0; j < PyList_GET_SIZE(runs); ++j) {
+            PyObject* r = PyList_GET_ITEM(runs, j);
+            if (!THPVariable_Check(r)) Py_RETURN_NONE;
+            const at::Tensor& t = THPVariable_Unpack(r);
+            if (t.scalar_type() != at::kInt || !t.is_contiguous() || !t.is_cuda() || t.device() != acc->device()) Py_RETURN_NONE;
+            held.push_back(t);
+            parts.push_back((const uint32_t*)t.const_data_ptr());
+            words.push_back(t.numel());
+        }
+        first.push_back((int)parts.size());
+        accs.push_back((float*)acc->mutable_data_ptr());
+        dtypes.push_back(code);
+    }
+    int rc;
+    {
+        pybind11::gil_scoped_release no_gil;
+        for (Py_ssize_t i = 0; i < count; ++i) {
+            outs.push_back(at::empty({}, held[0].options().dtype(kTypes[dtypes[i]])));
+            out_ptrs.push_back(outs.back().mutable_data_ptr());
+        }
+        rc = BOUND(mo_amax_fold)(accs.data(), out_ptrs.data(), dtypes.data(), first.data(), parts.data(), words.data(),
+                                 (int)count, c10::hip::getCurrentHIPStream().stream());
+    }
+    if (rc != MO_OK) return PyLong_FromLong(rc);
+    pybind11::list made;
+    for (const at::Tensor& t : outs) made.append(pybind11::reinterpret_steal<pybind11::object>(THPVariable_Wrap(t)));
+    return made.release().ptr();
+    END_HANDLE_TH_ERRORS
+}
+
+// bind({name: address}): where the calls go; a name left out has no compiled call.  Returns the names of those that have one.
 PyObject* bind(PyObject*, PyObject* table) {
     PyObject* names = PyList_New(0);
     if (!names) return nullptr;
@@ -193,6 +287,10 @@ PyObject* bind(PyObject*, PyObject* table) {
         PyObject* v = PyDict_GetItemString(table, kNames[i]);
         if (!v) continue;
         void* p = PyLong_AsVoidPtr(v);
+        if (!PyErr_Occurred() && i >= kCalls) {
+            g_address[i] = p;
+            continue;
+        }
         PyObject* name = PyErr_Occurred() ? nullptr : PyUnicode_FromString(kNames[i]);
         if (!name || PyList_Append(names, name)) {
             Py_XDECREF(name);
@@ -211,6 +309,8 @@ PyMethodDef kMethods[] = {
 #undef X
     {"row_qdq", (PyCFunction)(void (*)(void))row_qdq, METH_FASTCALL, nullptr},
     {"dynamic_qdq", (PyCFunction)(void (*)(void))dynamic_qdq, METH_FASTCALL, nullptr},
+    {"value_ranges", (PyCFunction)(void (*)(void))value_ranges, METH_FASTCALL, nullptr},
+    {"amax_fold", (PyCFunction)(void (*)(void))amax_fold, METH_FASTCALL, nullptr},
     {"bind", bind, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -37,6 +37,7 @@ SIGNATURES = {
     "mo_nvfp4_quantize_dynamic": [_P, _I64, _I64, _INT, _INT, _P, _P, _P, _P, _INT, _P],
     "mo_absmax_pair": [_P, _I64, _P, _P, _I64, _P, _INT, _P],
     "mo_value_ranges": [_P, _P, _P, _INT, _P, _I64, _P],
+    "mo_amax_fold": [_P, _P, _P, _P, _P, _P, _INT, _P],
     "mo_awq_pick_scale": [_P, _I64, _P, _I64, _P, _P, _P, _P, _P, _INT, _P],
     "mo_smooth_scales": [_P, _P, _I64, ctypes.c_float, _INT, ctypes.c_float, _INT, _INT, _P, _P, _P, _P, _P, _P],
     "mo_absmax_tensor_parts": [_P, _I64, _INT, _P, _P, _I64, _P, _P],
@@ -309,6 +310,11 @@ def value_ranges(tensors):
     n = len(tensors)
     if n == 0:
         return []
+    if _timer is None and _launch is not None:
+        made = _launch.value_ranges(tensors if type(tensors) is list else list(tensors), VALUE_RANGES_MAX,
+                                    VALUE_RANGES_CHUNK, VALUE_RANGES_MAX_CHUNKS)
+        if made is not None:
+            return _ranges_of(*made) if type(made) is not int else _raise("mo_value_ranges", made)
     device = tensors[0].device
     if n > VALUE_RANGES_MAX or device.type != "cuda":
         return None
@@ -327,6 +333,10 @@ def value_ranges(tensors):
     counts = (ctypes.c_int64 * n)(*[t.numel() for t in tensors])
     dtypes = (ctypes.c_int * n)(*[dtype_code(t.dtype) for t in tensors])
     call("mo_value_ranges", tensors[0], ptrs, counts, dtypes, n, _ptr(out), total, _stream(tensors[0]))
+    return _ranges_of(out, chunks)
+
+
+def _ranges_of(out, chunks):
     flat = out.tolist()
     result, at = [], 0
     for c in chunks:
@@ -334,6 +344,18 @@ def value_ranges(tensors):
         result.append((min(part[0::3]), max(part[1::3]), any(part[2::3])))
         at += c
     return result
+
+
+def amax_fold(accs, parts, dtypes):
+    """The end of a calibration for per-tensor accumulators (one fp32 element each, on one GPU): each takes in the largest word of
+    its list of ``parts`` and comes back as a tensor of its own without dims, of its type in ``dtypes``.  One launch; None, with
+    nothing launched, where that is not what the arguments are."""
+    if _launch is None:
+        load()
+    if any(d not in _DTYPES for d in dtypes):
+        return None
+    made = _launch.amax_fold(accs, parts, [_DTYPES[d] for d in dtypes])
+    return made if type(made) is not int else _raise("mo_amax_fold", made)
 
 
 _parts_ring = {}   # device index -> [int32 buffer, words handed out]

@@ -23,7 +23,7 @@ from .conversion import set_quantizer_by_cfg_context
 from .nn import QuantModule, SequentialQuantizer, TensorQuantizer
 from .nn.modules.quant_linear import _QuantLinear
 from .nn.modules.tensor_quantizer import calibration_pass
-from .utils import all_positive, all_valid_scales, deferred_scale_checks, is_quantized_linear
+from .utils import all_positive, all_valid_scales, deferred_scale_checks, is_quantized_linear, modules_of
 
 __all__ = ["max_calibrate", "smoothquant", "awq", "awq_lite", "enable_stats_collection",
            "finish_stats_collection", "apply_pre_quant_scale_and_smooth",
@@ -33,19 +33,15 @@ __all__ = ["max_calibrate", "smoothquant", "awq", "awq_lite", "enable_stats_coll
 # ----------------------------------------------------------------------------- max
 def weight_only_quantize(model: nn.Module):
     """Show every weight to its quantizer once (no activations involved)."""
-    seen = set()
-    for module in model.modules():
-        if module in seen:
-            continue
+    for module in modules_of(model):
         if isinstance(module, QuantModule) and hasattr(module, "weight_quantizer") and getattr(
                 module, "weight", None) is not None:
             module.weight_quantizer(module.weight)
-        seen.add(module)
 
 
 def enable_stats_collection(model: nn.Module):
     """Switch every enabled quantizer to calibration (quantisation off, statistics on)."""
-    for module in model.modules():
+    for module in modules_of(model):
         if isinstance(module, TensorQuantizer) and not module._disabled:
             if module._calibrator is not None:
                 module.disable_quant()
@@ -58,19 +54,18 @@ def finish_stats_collection(model: nn.Module, method: str | None = None):
     """Load the collected amax into ``_amax`` and switch quantisation back on."""
     # the calibrators' deferred sanity checks, for all of them at once: one host synchronisation
     # instead of one per quantizer (a calibrator that fails is left to raise its own message)
-    pending = [m._calibrator for m in model.modules()
-               if isinstance(m, TensorQuantizer) and not m._disabled
-               and getattr(m._calibrator, "_acc", None) is not None
-               and not m._calibrator._validated]
+    quantizers = [m for m in modules_of(model) if isinstance(m, TensorQuantizer) and not m._disabled]
+    pending = [m._calibrator for m in quantizers
+               if getattr(m._calibrator, "_acc", None) is not None and not m._calibrator._validated]
+    if method is None:   # every calibrator is asked for its amax below
+        calib.max.fold_calibrators([m._calibrator for m in quantizers if not m._dynamic])
     for c in pending:
         if hasattr(c, "_fold_pending"):
             c._fold_pending()   # tile maxima of reductions shared with another calibrator
     if pending and all_valid_scales([c._acc for c in pending]):
         for c in pending:
             c._validated = True
-    for module in model.modules():
-        if not isinstance(module, TensorQuantizer) or module._disabled:
-            continue
+    for module in quantizers:
         cal = getattr(module, "_calibrator", None)
         if cal and not getattr(module, "_dynamic", False):
             if type(cal) is MaxCalibrator:

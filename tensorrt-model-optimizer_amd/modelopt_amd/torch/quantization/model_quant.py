@@ -19,7 +19,7 @@ from . import model_calib
 from .config import QuantizeConfig, QuantizerAttributeConfig, normalize_algorithm
 from .conversion import is_converted, replace_quant_module, set_quantizer_attribute, set_quantizer_by_cfg
 from .nn import TensorQuantizer
-from .utils import DeferredCheckError, deferred_scale_checks
+from .utils import DeferredCheckError, deferred_scale_checks, modules_of, set_training
 
 __all__ = ["quantize", "calibrate", "disable_quantizer", "enable_quantizer", "print_quant_summary",
            "fold_weight", "postprocess_amax", "auto_quantize"]
@@ -105,7 +105,10 @@ def calibrate(model: nn.Module, algorithm="max", forward_loop: ForwardLoop | Non
         def forward_loop(model):
             return no_arg_loop()
     training = model.training
-    model.eval()
+    if type(model).eval is nn.Module.eval and "eval" not in model.__dict__:
+        set_training(model, False)
+    else:
+        model.eval()
     try:
         # every "amax / scale is finite and non-negative" check of the algorithm and the final look at
         # what it left on the quantizers are one device reduction and one host synchronisation
@@ -123,14 +126,13 @@ def calibrate(model: nn.Module, algorithm="max", forward_loop: ForwardLoop | Non
             elif method == "awq_lite":
                 model_calib.awq(model, forward_loop, "awq_lite", alpha_step=kwargs.get("alpha_step", 0.1),
                                 debug=kwargs.get("debug", False))
-            quantizers = [(n, m) for n, m in model.named_modules() if isinstance(m, TensorQuantizer)]
             attrs = ("_amax", "_pre_quant_scale")
-            checks.report = [t for _, m in quantizers for a in attrs
-                             if isinstance(t := getattr(m, a, None), torch.Tensor)]
+            checks.report = [t for m in modules_of(model) if isinstance(m, TensorQuantizer) for a in attrs
+                             if isinstance(t := m.calibrated_value(a), torch.Tensor)]
         # only a failure is walked through to name the culprit
         if not checks.report_ok:
-            for name, module in quantizers:
-                for attr in attrs:
+            for name, module in model.named_modules():
+                for attr in attrs if isinstance(module, TensorQuantizer) else ():
                     module.validate_attr(attr_name=attr, warn_error=True, name=name)
     except DeferredCheckError:
         # a calibrator whose running maximum is bad says so in its own words (the reference's
@@ -142,7 +144,7 @@ def calibrate(model: nn.Module, algorithm="max", forward_loop: ForwardLoop | Non
                 cal.compute_amax()
         raise
     finally:
-        model.train(training)
+        set_training(model, training)
     return model
 
 

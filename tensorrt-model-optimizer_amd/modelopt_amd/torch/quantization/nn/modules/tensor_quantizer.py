@@ -227,6 +227,14 @@ class TensorQuantizer(nn.Module):
                 raise RuntimeError("Changing shape when setting amax is not allowed.")
             self._amax.data.copy_(value.clone().detach().to(self._amax.device))
 
+    def calibrated_value(self, name):
+        """``getattr(self, name, None)`` for a value that is a buffer or missing in nearly every quantizer: a missing one
+        costs ``nn.Module`` an exception to look for."""
+        value = self._buffers.get(name)
+        if value is None and (name in self.__dict__ or name in self._parameters or type(self) is not TensorQuantizer):
+            value = getattr(self, name, None)
+        return value
+
     def reset_amax(self):
         if hasattr(self, "_amax"):
             delattr(self, "_amax")
@@ -335,11 +343,15 @@ class TensorQuantizer(nn.Module):
             warnings.warn("Set amax to NaN!")
             calib_amax = torch.tensor(math.nan)
         if type(self._calibrator) is calib.MaxCalibrator and calib_amax.device.type != "meta":
-            fresh = calib_amax.detach()          # already a tensor of its own
+            fresh = calib_amax.detach() if calib_amax.requires_grad else calib_amax   # already a tensor of its own
         else:
             fresh = calib_amax.clone().detach()
-        if not hasattr(self, "_amax"):
-            self.register_buffer("_amax", fresh)
+        if self.calibrated_value("_amax") is None and not hasattr(self, "_amax"):
+            if _module_hooks._global_buffer_registration_hooks:
+                self.register_buffer("_amax", fresh)
+            else:   # what that comes to: a tensor under a name that is free
+                self._buffers["_amax"] = fresh
+                self._non_persistent_buffers_set.discard("_amax")
         else:
             self._amax.data.copy_(fresh)
 
@@ -655,6 +667,9 @@ class TensorQuantizer(nn.Module):
         """Scale -> (calibrate) -> (quantise); returns a tensor of the input dtype for fake
         quantisation, a ``QTensorWrapper``-able packed tensor for real quantisation."""
         if type(inputs) in _PLAIN_TENSORS and not torch.compiler.is_compiling():
+            own = self.__dict__
+            if (own["_disabled"] or own["_if_calib"]) and self._hands_back(own, inputs):
+                return inputs
             outputs = self._direct_fake_quant(inputs)
             if outputs is not None:
                 return outputs
@@ -696,6 +711,22 @@ class TensorQuantizer(nn.Module):
             outputs = self._reset_to_original_shape(outputs)
         return outputs
 
+    def _hands_back(self, own, inputs) -> bool:
+        """Whether ``forward`` comes down to returning ``inputs``, shown to the calibrator on the way: a quantizer that is
+        switched off, or only collects, with no scale or blocks to see to.  (Most calls of a calibration loop; the
+        steps of ``forward`` take four times as long to find it out.)"""
+        if (type(self) is not TensorQuantizer or own["_rotate"] or "_pre_quant_scale" in own["_buffers"]
+                or "_pre_quant_scale" in own or "_pre_quant_scale" in own["_parameters"] or inputs.numel() == 0):
+            return False
+        if own["_disabled"]:
+            own["_input_dtype"] = inputs.dtype
+            return True
+        if own["_if_quant"] or own["_dynamic"] or own["_block_sizes"] is not None or own["_calibrator"] is None:
+            return False
+        if not self._seen_this_parameter(inputs):
+            self.collect(inputs)
+        return True
+
     # A weight is shown to its quantizer on every forward of a calibration loop.  Inside one
     # ``forward_loop`` run by this package (``calibration_pass``) its abs-max cannot change while
     # the parameter is untouched, so a repeat of the same parameter (same storage, same version
@@ -707,9 +738,10 @@ class TensorQuantizer(nn.Module):
     cache_weight_amax = True
 
     def _seen_this_parameter(self, source) -> bool:
-        if not (self.cache_weight_amax and _CALIBRATION_PASS[0] and isinstance(source, nn.Parameter)):
+        if type(source) is torch.Tensor or not (self.cache_weight_amax and _CALIBRATION_PASS[0]
+                                                and isinstance(source, nn.Parameter)):
             return False
-        cal = self._calibrator
+        cal = self.__dict__["_calibrator"]
         if type(cal) is not calib.MaxCalibrator or cal._track_amax:
             return False
         pqs = self.pre_quant_scale

@@ -18,6 +18,40 @@ __all__ = [
 ]
 
 
+_STOCK = torch.nn.Module
+
+
+def modules_of(model) -> list:
+    """``list(model.modules())`` without a chain of nested generators (a third of their time)."""
+    found, seen = [], set()
+
+    def walk(module):
+        seen.add(module)
+        found.append(module)
+        children = module._modules
+        if children:
+            for child in children.values():
+                if child is not None and child not in seen:
+                    walk(child)
+
+    walk(model)
+    if any(c.named_modules is not _STOCK.named_modules or c.modules is not _STOCK.modules for c in set(map(type, found))):
+        return list(model.modules())   # a class that lists its modules itself
+    return found
+
+
+def set_training(model, mode: bool):
+    """``model.train(mode)``, written to the modules that are in the other mode only."""
+    modules = modules_of(model)
+    if (any(c.train is not _STOCK.train or c.children is not _STOCK.children for c in set(map(type, modules)))
+            or any("train" in m.__dict__ for m in modules)):
+        model.train(mode)
+        return
+    for m in modules:
+        if m.training is not mode:
+            m.training = mode
+
+
 def true_divide(t: torch.Tensor, divisor: float) -> torch.Tensor:
     """``t / divisor`` as one correctly rounded division.
 

@@ -7,7 +7,7 @@ from modelopt_amd import _hip
 
 DEV = "cuda:0"
 # host arrays, results by reference, or no pointers at all
-THROUGH_CTYPES = {"mo_version", "mo_error_string", "mo_value_ranges", "mo_absmax_tensor_parts", "mo_absmax_multi",
+THROUGH_CTYPES = {"mo_version", "mo_error_string", "mo_value_ranges", "mo_amax_fold", "mo_absmax_tensor_parts", "mo_absmax_multi",
                   "mo_nvfp4_quantize_multi", "mo_awq_clip_losses"}
 
 
