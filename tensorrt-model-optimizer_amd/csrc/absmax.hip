@@ -295,6 +295,36 @@ __global__ __launch_bounds__(256) void absmax_short_rows_kernel(const void* __re
     }
 }
 
+// Long aligned rows (more than 256 chunks): a row is cut into `segs` runs of at most 512 chunks, and a wavefront takes
+// one run, eight chunks a lane in straight-line code; a chunk past the end re-reads the last one.  Bound by
+// memory: absmax_rows_kernel waits for four loads at a time and has each row's reduction between its loads.
+// Against it, bf16: 8192 x 8192 30.8 -> 21.8 us = 6.2 TB/s, 14336 x 4096 30.2 -> 19.5, 4096 x 14336 22.3 -> 20.9,
+// 4096 x 2560 (five of the eight loads of a lane are its own) 7.3 -> 6.1; fp32 8192 x 8192 60.7 -> 47.5.  Shorter rows
+// leave it too few loads: 4096 x 1024 5.5 -> 6.6 us with four rows a wavefront.
+template <int DT>
+__global__ __launch_bounds__(256) void absmax_row_runs_kernel(const void* __restrict__ x, int64_t nrows,
+                                                              int64_t row_chunks, int64_t axis, uint32_t segs,
+                                                              uint32_t seg_chunks, uint32_t* __restrict__ acc) {
+    const int lane = threadIdx.x & 63;
+    const int64_t run = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row = run <= 0xFFFFFFFFll ? (int64_t)((uint32_t)run / segs) : run / segs;
+    if (row >= nrows) return;
+    const int64_t first = (run - row * segs) * seg_chunks;
+    const int64_t end = first + seg_chunks < row_chunks ? first + seg_chunks : row_chunks;
+    RawChunk<DT> raw[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        int64_t c = first + u * 64 + lane;
+        c = c < end ? c : end - 1;
+        load_raw<DT>(x, (row * row_chunks + c) << 3, raw[u]);
+    }
+    AbsAcc<DT> a;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a.raw(raw[u]);
+    const uint32_t v = group_max_u32(a.bits(), 6);
+    if (lane == 0) fold_max(acc + row % axis, v);
+}
+
 // ------------------------------------------------------------------------------ columns
 // x viewed as [outer, axis] (inner == 1).  Vector path (axis % 8 == 0, aligned): a lane owns 8
 // adjacent columns, a wavefront 512; the four wavefronts of a workgroup take interleaved rows of
@@ -558,6 +588,15 @@ static int launch_absmax(const void* x, int64_t outer, int64_t axis, int64_t inn
         if (tiles <= 0x7FFFFFFF) {
             absmax_short_rows_kernel<DT><<<dim3((unsigned)tiles), 256, mo::ballast_bytes("absmax_short_rows_kernel", 0), s>>>(
                 x, nrows, axis, lg_l, outer == 1 ? 1 : 0, acc);
+            return MO_OK;
+        }
+    }
+    if (base_ok && inner % 8 == 0 && row_chunks > 256) {
+        const int64_t runs = (row_chunks + 511) / 512, seg = (row_chunks + runs - 1) / runs;
+        const int64_t segs = (row_chunks + seg - 1) / seg, blocks = (nrows * segs + 3) / 4;
+        if (blocks <= 0x7FFFFFFF && segs <= 0x7FFFFFFF) {
+            absmax_row_runs_kernel<DT><<<(unsigned)blocks, 256, mo::ballast_bytes("absmax_row_runs_kernel", 0), s>>>(
+                x, nrows, row_chunks, axis, (uint32_t)segs, (uint32_t)seg, acc);
             return MO_OK;
         }
     }

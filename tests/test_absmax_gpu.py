@@ -40,6 +40,22 @@ def test_per_row_keep_axis0(dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+# the shortest row of one run, a full run, two of them (the second shorter), rows that do not fill a workgroup
+@pytest.mark.parametrize("shape", [(1, 2056), (5, 4096), (3, 4104), (129, 8192), (2, 9000), (6, 12296)])
+@pytest.mark.parametrize("outer", [1, 2])
+def test_long_rows_in_runs(dtype, shape, outer):
+    x = _rand((outer, *shape), dtype, 6)
+    for r, c in ((0, 0), (-1, -1), (-1, shape[1] // 2), (0, min(4096, shape[1] - 1))):   # the maximum at the ends of runs
+        x[:, r, c] = 50.0 + c % 7
+    got = _gpu_reduce(x, outer, *shape).to(dtype)
+    assert_bits_equal(got, reduce.reduce_amax(x, axis=[0, 2], keepdims=False).reshape(-1), str(shape))
+    x[0, -1, shape[1] // 2] = float("inf")
+    x[0, 0, -1] = float("nan")
+    got = _gpu_reduce(x, outer, *shape)
+    assert torch.isnan(got[0]) and (shape[0] == 1 or got[-1] == float("inf"))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape", [(5, 16), (300, 128), (4096, 512), (77, 13), (8192, 8)])
 def test_per_column_keep_last_axis(dtype, shape):
     x = _rand(shape, dtype, 2)
