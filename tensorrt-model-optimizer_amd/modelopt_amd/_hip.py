@@ -49,6 +49,8 @@ SIGNATURES = {
     "mo_int_qdq": [_P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _P],
     "mo_ste_mask": [_P, _P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _P],
     "mo_wgrad_masked": [_P, _P, _P, _P, _I64, _I64, _I64, _INT, _P, _INT, _I64, _INT, _P],
+    "mo_input_grad_splits": [_I64, _I64, _I64],
+    "mo_input_grad": [_P, _P, _P, _P, _I64, _I64, _I64, _INT, _INT, _P],
     "mo_row_qdq": [_P, _P, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _P, _INT, _P],
     "mo_nvfp4_qdq": [_P, _P, _I64, _I64, _INT, _P, _INT, _INT, _INT, _P],
     "mo_qdq_sq_err": [_P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _INT, _INT, _P, _P],
@@ -437,6 +439,27 @@ def wgrad_masked(dy, x, w, amax, inner=0, narrow_amax=False):
     call("mo_wgrad_masked", w, _ptr(dy), _ptr(x), _ptr(w), _ptr(dw), tokens, n, k, dtype_code(w.dtype), _ptr(amax),
          dtype_code(amax.dtype), inner, int(narrow_amax), _stream(w))
     return dw
+
+
+def input_grad(dy, w):
+    """``dy @ w`` in the dtype of ``w`` with sums in fp32 (``dy`` [tokens, n], ``w`` [n, k]).  None, with nothing
+    launched, where the kernel has no such form."""
+    if (w.dtype not in (torch.bfloat16, torch.float16) or dy.dtype != w.dtype or not dy.is_cuda
+            or dy.device != w.device or not dy.is_contiguous() or not w.is_contiguous()
+            or (dy.data_ptr() | w.data_ptr()) % 16):
+        return None
+    if _lib is None:
+        load()
+    (tokens, n), k = dy.shape, w.shape[1]
+    assert w.shape[0] == n
+    splits = _entry["mo_input_grad_splits"](tokens, n, k)
+    if splits == 0:
+        return None
+    dx = torch.empty((tokens, k), dtype=w.dtype, device=w.device)
+    partial = torch.empty((splits, tokens, k), dtype=torch.float32, device=w.device) if splits > 1 else None
+    call("mo_input_grad", w, _ptr(dy), _ptr(w), _ptr(dx), _ptr(partial), tokens, n, k, dtype_code(w.dtype), splits,
+         _stream(w))
+    return dx
 
 
 def blocks2d_covered(x, rows, cols, block_rows, block_cols) -> bool:

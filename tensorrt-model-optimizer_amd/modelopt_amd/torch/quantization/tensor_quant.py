@@ -313,7 +313,10 @@ class MaskedGradientLinear(Function):
             used = quantized
             if differentiated:   # its value, with the straight-through path back to the weight
                 used = quantized + masked(weight, weight - weight.detach())
-            grads[0] = (rows @ used).reshape(x.shape)
+            product = None
+            if plain and kernels.input_grad_pays(rows.shape[0], n, k):
+                product = _hip.input_grad(rows.contiguous(), used)
+            grads[0] = (rows @ used if product is None else product).reshape(x.shape)
         if _is_wanted(ctx, 1):
             x2 = x.reshape(-1, k)
             if plain:

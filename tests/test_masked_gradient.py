@@ -21,6 +21,13 @@ def test_the_sizes_at_which_one_pass_pays(n, k, most):
         assert kernels.wgrad_mask_pays(tokens, n, k) == (1 <= tokens <= most), tokens
 
 
+@pytest.mark.parametrize("n,k,most", [(14336, 4096, 1024), (4096, 4096, 1024), (4088, 4096, 512), (6144, 6144, 512),
+                                      (6136, 6144, 256), (7168, 7168, 256), (8, 8, 1024), (8, 16384, 256), (12, 8, 0), (8, 12, 0)])
+def test_the_sizes_at_which_the_input_gradient_is_left_to_the_kernel(n, k, most):
+    for tokens in (0, 1, most, most + 1, 4096):
+        assert kernels.input_grad_pays(tokens, n, k) == (1 <= tokens <= most), tokens
+
+
 def _halves(w):   # a quantizer of the CPU: to steps of a half within +-1
     return (w.clamp(-1, 1) * 2).round() / 2
 

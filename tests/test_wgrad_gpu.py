@@ -131,3 +131,39 @@ def test_what_does_not_take_it():
     with torch.no_grad():
         assert layer(x).grad_fn is None
     assert _hip.wgrad_masked(x, x[:, :60].contiguous(), x.new_zeros(96, 60), x.new_ones(1)) is None   # 60 columns
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+# one token and one chunk; tokens at and past the three tiles; n below, at and past a step, in several runs, an odd
+# number of steps a run; columns with part of a tile
+@pytest.mark.parametrize("tokens,n,k", [(1, 8, 8), (64, 64, 128), (65, 72, 136), (129, 1160, 264), (200, 4104, 520),
+                                        (257, 2056, 4096), (512, 520, 4104), (700, 14336, 1024), (31, 4096, 1 << 16)])
+def test_input_gradient_against_float64(dtype, tokens, n, k):
+    g = torch.Generator(DEV).manual_seed(tokens)
+    dy, w = (torch.randn(s, device=DEV, generator=g).to(dtype) for s in ((tokens, n), (n, k)))
+    got, exact = _hip.input_grad(dy, w), dy.double() @ w.double()
+    # as for the weight gradient, with sums of n products
+    step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    bound = step * 1.01 * exact.abs() + n * 2.0 ** -24 * (dy.double().abs() @ w.double().abs()) + 2.0 ** -25
+    assert got.shape == exact.shape and ((got.double() - exact).abs() <= bound).all()
+    assert torch.equal(got, _hip.input_grad(dy, w))
+    dy[0, n // 2] = float("nan")
+    got = _hip.input_grad(dy, w)
+    assert torch.isnan(got[0]).all() and not torch.isnan(got[1:]).any()
+
+
+def test_input_gradient_stays_inside_its_operands():
+    """What lies around the operands is NaN: n and k end inside a step and a tile, the tokens inside a tile."""
+    wide = torch.full((70 * 72 + 64,), float("nan"), device=DEV, dtype=torch.bfloat16)
+    dy, w = wide[32:32 + 66 * 72].view(66, 72), torch.full_like(wide, float("nan"))[:72 * 64 + 32][:72 * 64].view(72, 64)
+    dy.fill_(1.0)
+    w.fill_(0.5)
+    assert torch.equal(_hip.input_grad(dy, w), torch.full((66, 64), 36.0, device=DEV, dtype=torch.bfloat16))
+
+
+def test_what_has_no_input_gradient_kernel():
+    ones = torch.ones(8, 64, device=DEV, dtype=torch.bfloat16)
+    assert _hip.input_grad(ones[:, :60].contiguous(), ones.new_ones(60, 8)) is None
+    assert _hip.input_grad(ones.float(), ones.new_ones(64, 8).float()) is None
+    assert _hip.input_grad(ones, ones.new_ones(64, 12)) is None
+    assert _hip.input_grad(ones, ones.new_ones(8, 64).t()) is None
