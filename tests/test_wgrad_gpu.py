@@ -17,9 +17,11 @@ DTYPES = [torch.bfloat16, torch.float16]
 
 @pytest.mark.parametrize("dtype", DTYPES)
 # one token and one chunk; tokens below, at and past an octet and a step; widths with part of a
-# tile; a last group of fewer than eight n tiles; several groups
+# tile; a last group of fewer than eight n tiles; several groups; below and at the kernel for many tokens, a last step of
+# 31 tokens and of 8
 @pytest.mark.parametrize("tokens,n,k", [(1, 8, 8), (7, 24, 136), (8, 128, 128), (64, 136, 264), (65, 1032, 128),
-                                        (200, 520, 392), (513, 1160, 256)])
+                                        (200, 520, 392), (513, 1160, 256),
+                                        (383, 136, 392), (384, 1160, 136), (415, 24, 264), (1000, 520, 1032)])
 @pytest.mark.parametrize("inner", ["all", "row", 8])
 def test_kernel_against_float64(dtype, tokens, n, k, inner):
     g = torch.Generator(DEV).manual_seed(tokens)
@@ -37,6 +39,21 @@ def test_kernel_against_float64(dtype, tokens, n, k, inner):
     step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     bound = step * 1.01 * exact.abs() + tokens * 2.0 ** -24 * (dy.double().abs().t() @ x.double().abs()) + 2.0 ** -25
     assert ((got.double() - exact).abs() <= bound)[mask].all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("narrow", [False, True])
+@pytest.mark.parametrize("tokens", [8, 384])
+def test_the_mask_of_every_value(dtype, narrow, tokens):
+    """All 65536 values of the weight under amax values between, at and beyond those of its type."""
+    values = torch.arange(1 << 16, device=DEV).to(torch.uint16).view(dtype).view(1, -1)
+    amax = torch.tensor([0.0, -0.0, -1.0, float("inf"), float("nan"), 1 + 2.0 ** -12, 1 - 2.0 ** -13, 9e4, 3e-8, 1e-40, -1e-9,
+                         0.75, 3.4e38, 65504.0, 65519.9, 6e-5], device=DEV)
+    w = values.repeat(amax.numel(), 1)
+    dy, x = torch.ones(tokens, w.shape[0], device=DEV, dtype=dtype), torch.ones(tokens, w.shape[1], device=DEV, dtype=dtype)
+    got = _hip.wgrad_masked(dy, x, w, amax, w.shape[1], narrow)
+    limit = amax.to(dtype).float() if narrow else amax
+    assert torch.equal(got, torch.where(w.float().abs() <= limit.view(-1, 1), float(tokens), 0.0).to(dtype))
 
 
 def test_a_token_past_the_end_does_not_count():
