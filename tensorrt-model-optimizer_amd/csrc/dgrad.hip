@@ -15,7 +15,7 @@
 //
 // Measured against the library's product, bf16, weight 14336 x 4096 (n x k): 32 tokens 22.7 us (41.8), 128 28.1 (96.8),
 // 256 44.7 (76.8), 512 72.5 (100 - 110) = 0.83 PFLOP/s, 1024 128 (147).  Up to 128 tokens memory bounds it (117 MB of weight, 4.2 - 5.2 TB/s with
-// the second launch); beyond, the matrix cores are busy a third to half of the time: a step's 1024 cycles of
+// the second launch); beyond, the matrix cores are busy 40 % of the cycles (512 tokens): a step's 1024 cycles of
 // products stand beside 910 of LDS and 768 of L1 (64 bytes a clock), and with no loads at all 512 tokens x 4096 x 14336
 // take 55 us where they take 66 with them.  Operands read three products ahead 66.0, two 66.9, one 67.7; two LDS stages 73.
 // No bank conflicts (counted).

@@ -314,8 +314,9 @@ class MaskedGradientLinear(Function):
             if differentiated:   # its value, with the straight-through path back to the weight
                 used = quantized + masked(weight, weight - weight.detach())
             product = None
-            if plain and kernels.input_grad_pays(rows.shape[0], n, k):
-                product = _hip.input_grad(rows.contiguous(), used)
+            if plain and type(used) is torch.Tensor and kernels.input_grad_pays(rows.shape[0], n, k):
+                rows = rows.contiguous()   # the weight's gradient reads it too
+                product = _hip.input_grad(rows, used)
             grads[0] = (rows @ used if product is None else product).reshape(x.shape)
         if _is_wanted(ctx, 1):
             x2 = x.reshape(-1, k)
