@@ -1,5 +1,8 @@
 """The end of a max calibration in one launch, accumulators cleared together, and the walk over a model's modules."""
 
+import gc
+import weakref
+
 import pytest
 import torch
 from torch import nn
@@ -29,6 +32,19 @@ def test_modules_in_the_order_of_the_stock_walk():
 
     odd = nn.Sequential(Lists(2, 2), nn.ReLU())
     assert [id(m) for m in modules_of(odd)] == [id(m) for m in odd.modules()]
+
+
+def test_a_walk_keeps_no_module_alive():
+    model = nn.Sequential(nn.Linear(2, 2), nn.ReLU())
+    alive = weakref.ref(model[0])
+    gc.disable()
+    try:
+        modules_of(model)
+        set_training(model, False)
+        del model
+        assert alive() is None
+    finally:
+        gc.enable()
 
 
 def test_modes_are_set_as_train_sets_them():
