@@ -19,6 +19,7 @@ __all__ = [
 
 
 _STOCK = torch.nn.Module
+_HOW_MODES_ARE_SET = ("train", "children", "named_children")   # the methods that the stock ``train`` goes through
 
 
 def _walk(module, found, seen):
@@ -43,10 +44,11 @@ def modules_of(model) -> list:
 
 def set_training(model, mode: bool):
     """``model.train(mode)``, written to the modules that are in the other mode only."""
-    modules = modules_of(model)
-    if (any(c.train is not _STOCK.train or c.children is not _STOCK.children for c in set(map(type, modules)))
-            or any("train" in m.__dict__ for m in modules)):
-        model.train(mode)
+    modules = []
+    _walk(model, modules, set())
+    if any(getattr(c, n) is not getattr(_STOCK, n) for c in set(map(type, modules)) for n in _HOW_MODES_ARE_SET) or any(
+            n in m.__dict__ for m in modules for n in _HOW_MODES_ARE_SET):
+        model.train(mode)   # a module that sets its mode, or lists its children, itself
         return
     for m in modules:
         if m.training is not mode:

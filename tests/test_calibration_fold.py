@@ -62,6 +62,33 @@ def test_modes_are_set_as_train_sets_them():
             assert [m.training for m in a.modules()] == [m.training for m in b.modules()]
 
 
+class _Unlisted(nn.Sequential):
+    def named_modules(self, *a, **k):   # its children are in no list of modules, but have a mode
+        yield "", self
+
+
+class _Hidden(nn.Sequential):
+    def named_children(self):           # its children keep their mode
+        return iter(())
+
+
+def _hidden_by_instance(*children):
+    block = nn.Sequential(*children)
+    block.named_children = lambda: iter(())
+    return block
+
+
+@pytest.mark.parametrize("block", [_Unlisted, _Hidden, _hidden_by_instance])
+def test_modes_of_children_that_a_block_does_not_list(block):
+    for start in (True, False):
+        a, b = (nn.Sequential(nn.ReLU(), block(nn.Dropout())) for _ in range(2))
+        for m in (a[0], b[0], a[1][0], b[1][0]):
+            m.training = start
+        a.train(not start)
+        set_training(b, not start)
+        assert [m.training for m in (a, a[0], a[1], a[1][0])] == [m.training for m in (b, b[0], b[1], b[1][0])]
+
+
 class _Layer(nn.Module):
     def __init__(self):
         super().__init__()
