@@ -37,8 +37,9 @@ def modules_of(model) -> list:
     here: one that names itself is a cycle, and the modules it has seen would live until the garbage collector runs."""
     found = []
     _walk(model, found, set())
-    if any(c.named_modules is not _STOCK.named_modules or c.modules is not _STOCK.modules for c in set(map(type, found))):
-        return list(model.modules())   # a class that lists its modules itself
+    if any(getattr(c, n) is not getattr(_STOCK, n) for c in set(map(type, found)) for n in ("modules", "named_modules")) or any(
+            "named_modules" in m.__dict__ or "modules" in m.__dict__ for m in found):
+        return list(model.modules())   # a module that lists its modules itself
     return found
 
 

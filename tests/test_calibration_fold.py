@@ -34,6 +34,15 @@ def test_modules_in_the_order_of_the_stock_walk():
     assert [id(m) for m in modules_of(odd)] == [id(m) for m in odd.modules()]
 
 
+def test_modules_of_a_block_whose_list_is_its_own():
+    hidden = nn.Sequential(nn.ReLU())
+    hidden.named_modules = lambda *a, **k: iter((("", hidden),))
+    for model in (nn.Sequential(hidden, nn.ReLU()), hidden):
+        assert [id(m) for m in modules_of(model)] == [id(m) for m in model.modules()]
+    model.modules = lambda: iter(())
+    assert modules_of(model) == []
+
+
 def test_a_walk_keeps_no_module_alive():
     model = nn.Sequential(nn.Linear(2, 2), nn.ReLU())
     alive = weakref.ref(model[0])
