@@ -721,8 +721,8 @@ class TensorQuantizer(nn.Module):
         if own["_disabled"]:
             own["_input_dtype"] = inputs.dtype
             return True
-        if own["_if_quant"] or own["_dynamic"] or own["_block_sizes"] is not None or own["_calibrator"] is None:
-            return False
+        if own["_if_quant"] or own["_dynamic"] or own["_block_sizes"] is not None or own.get("_calibrator") is None:
+            return False   # a calibrator that is a module is none of the quantizer's own attributes
         if not self._seen_this_parameter(inputs):
             self.collect(inputs)
         return True
@@ -741,7 +741,7 @@ class TensorQuantizer(nn.Module):
         if type(source) is torch.Tensor or not (self.cache_weight_amax and _CALIBRATION_PASS[0]
                                                 and isinstance(source, nn.Parameter)):
             return False
-        cal = self.__dict__["_calibrator"]
+        cal = self._calibrator
         if type(cal) is not calib.MaxCalibrator or cal._track_amax:
             return False
         pqs = self.pre_quant_scale

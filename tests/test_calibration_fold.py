@@ -123,6 +123,24 @@ def test_a_disabled_and_a_collecting_quantizer_hand_their_input_back():
     assert torch.equal(q(x), 2 * x)
 
 
+@pytest.mark.parametrize("in_a_pass", [False, True])
+def test_a_calibrator_that_is_a_module(in_a_pass):
+    class Calibrator(nn.Module):
+        def collect(self, x):
+            self.seen = x
+
+    q = TensorQuantizer()
+    q._calibrator = Calibrator()
+    q.disable_quant(), q.enable_calib()
+    for x in (torch.randn(4, 8), nn.Parameter(torch.randn(4, 8))):
+        if in_a_pass:
+            with calibration_pass():
+                assert q(x) is x
+        else:
+            assert q(x) is x
+        assert q._calibrator.seen is x
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 3, 48, 49, 130])
 def test_folded_maxima(n):
