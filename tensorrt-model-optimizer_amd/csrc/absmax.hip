@@ -594,7 +594,19 @@ static int launch_absmax(const void* x, int64_t outer, int64_t axis, int64_t inn
     if (base_ok && inner % 8 == 0 && row_chunks > 256) {
         const int64_t runs = (row_chunks + 511) / 512, seg = (row_chunks + runs - 1) / runs;
         const int64_t segs = (row_chunks + seg - 1) / seg, blocks = (nrows * segs + 3) / 4;
-        if (blocks <= 0x7FFFFFFF && segs <= 0x7FFFFFFF) {
+        // Every run ends in an atomic at its accumulator, and those that start together all find a fresh one empty.  With
+        // many runs for each of many accumulators that costs more than the loads in flight win; the kernel below makes a
+        // thousand pieces at most.  First batch of a calibration, bf16 (fp32), us, that kernel -> this one, outer x axis x inner:
+        //   inside  1 x 8192 x 32768 100 -> 89 (207 -> 195), 8 x 2048 x 8192 63 -> 42 (109 -> 89), 32 x 256 x 16384 78 -> 49 (116 ->
+        //           91); few runs in all: 1 x 64 x 131072 33 -> 13 (48 -> 16), 1 x 16 x 1M 124 -> 51 (92 -> 55), 1 x 4 x 4M 103 -> 51 (92 -> 55),
+        //           8 x 3 x 50176 8.0 -> 6.5 (8.8 -> 7.4)
+        //   beyond  1 x 2048 x 65536 52 -> 57 (100 -> 119), 1 x 64 x 2M 125 -> 147 (130 -> 219), 1 x 2 x 8M 36 -> 51, 1 x 2 x 32M 37 -> 169,
+        //           28 x 3 x 32776 11.5 -> 9.5 (9.1 -> 10.7), 256 x 2 x 8192 11.2 -> 11.6 (13.2 -> 14.0), 2048 x 2 x 16384 66 -> 144,
+        //           16384 x 2 x 2304 181 -> 120 (141 -> 239)
+        // Into an accumulator that holds a maximum this one is faster, or at fp32 up to 6 % slower (8192 x 2056 14.8 -> 15.7).
+        const int64_t each = outer * segs;
+        const bool few = each <= 128 ? segs <= 8 || axis * each <= 4096 : outer == 1 && each <= 1024 && axis * each <= 4096;
+        if (few && blocks <= 0xFFFFFF) {   // a launch has fewer than 2^32 work items
             absmax_row_runs_kernel<DT><<<(unsigned)blocks, 256, mo::ballast_bytes("absmax_row_runs_kernel", 0), s>>>(
                 x, nrows, row_chunks, axis, (uint32_t)segs, (uint32_t)seg, acc);
             return MO_OK;

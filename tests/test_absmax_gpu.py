@@ -32,6 +32,24 @@ def test_per_tensor(dtype, n):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+# at and past the runs of an accumulator that the kernel of runs is given: by rows of it, by the length of a row, and with few
+# accumulators by both
+@pytest.mark.parametrize("outer,axis,inner", [(128, 33, 2056), (129, 33, 2056), (16, 33, 32768), (16, 33, 32776), (1, 513, 32768),
+                                              (1, 513, 32776), (14, 3, 32776), (15, 3, 32776), (1, 4, 4 << 20), (1, 4, (4 << 20) + 8),
+                                              (1, 1, 4096), (2, 1, 4104)])
+def test_long_rows_at_the_most_runs_of_an_accumulator(dtype, outer, axis, inner):
+    x = torch.zeros(outer, axis, inner, dtype=dtype, device=DEV)
+    want = torch.arange(1, axis + 1, device=DEV).to(dtype)   # once a channel: ends of the first and of the last row, a middle
+    for c in range(axis):
+        o, i = ((0, 0), (outer - 1, inner - 1), (outer // 2, inner // 2))[c % 3]
+        x[o, c, i] = -want[c]
+    acc = torch.zeros(axis, device=DEV)
+    for _ in range(2):   # a fresh accumulator, and one that holds the maximum
+        _hip.absmax_into(x, acc, outer, axis, inner)
+        assert torch.equal(acc, want.float())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape", [(5, 16), (300, 128), (64, 4096), (3, 100000), (1000, 7), (2, 9)])
 def test_per_row_keep_axis0(dtype, shape):
     x = _rand(shape, dtype, 1)
