@@ -242,15 +242,21 @@ def wgrad_mask_pays(tokens: int, n: int, k: int) -> bool:
 
 
 def input_grad_pays(tokens: int, n: int, k: int) -> bool:
-    """Whether the input gradient of ``tokens`` rows behind a [n, k] weight is left to ``_hip.input_grad``: up to 256
-    tokens (14336 x 4096 bf16, 128 tokens 32 us and 96 in the library, 4096 x 14336 32 and 36, 256 tokens 48 and 77, 45 and 48;
-    the worst seen 2752 x 4096 at 256 tokens, 20.6 and 19.2).  With more, a wide result has tiles enough for the
-    library's larger ones and a short sum does not pay for the partial sums: up to 512 tokens k <= 4096, or 6144 where
-    n >= k (14336 x 4096 73 and 106, 6144 x 6144 56 and 70; 4096 x 14336 66 and 62, 7168 x 7168 70 and 64), up to 1024 k <= 4096 and
-    n >= k (14336 x 4096 129 and 147, 4096 x 4096 45 and 46; 2752 x 4096 32 and 30, 5120 x 5120 85 and 76)."""
+    """Whether the input gradient of ``tokens`` rows behind a [n, k] weight is left to ``_hip.input_grad``.  us, it and the
+    library's product, bf16 (fp16 is the same):
+
+    up to 128 tokens k <= 32768 (14336 x 4096 at 128 tokens 34 and 125, 8192 x 28672 at 64 88 and 93, 4096 x 32768 at 100 51 and 55;
+    wider results have tiles enough for the library: 4096 x 40960 at 64 78 and 70, 16384 x 53248 at 128 419 and 378);
+    up to 256 tokens k <= 8192, or 16384 where n <= 16384 (16384 x 16384 at 192 tokens 135 and 184, 53248 x 8192 211 and 334; 8192 x 24576
+    135 and 113, 28672 x 16384 at 192 233 and 226, 53248 x 14336 at 144 412 and 381);
+    up to 512 tokens k <= 4096, or 6144 where n >= k, as a short sum does not pay for the partial sums (14336 x 4096 73 and 106, 6144 x 6144
+    56 and 70; 4096 x 14336 66 and 62, 7168 x 7168 70 and 64);
+    up to 1024 tokens k <= 4096 and n >= k (14336 x 4096 129 and 147, 4096 x 4096 45 and 46; 2752 x 4096 32 and 30, 5120 x 5120 85 and 76)."""
     if not 1 <= tokens <= 1024 or n % 8 or k % 8:
         return False
-    return tokens <= 256 or (k <= 4096 and (n >= k or tokens <= 512)) or (k <= 6144 and n >= k and tokens <= 512)
+    if tokens <= 256:
+        return k <= (32768 if tokens <= 128 else 16384 if n <= 16384 else 8192)
+    return (k <= 4096 and (n >= k or tokens <= 512)) or (k <= 6144 and n >= k and tokens <= 512)
 
 
 def fake_quant_nvfp4(x, global_amax, block_size=16, mode=0):

@@ -28,6 +28,13 @@ def test_the_sizes_at_which_the_input_gradient_is_left_to_the_kernel(n, k, most)
         assert kernels.input_grad_pays(tokens, n, k) == (1 <= tokens <= most), tokens
 
 
+@pytest.mark.parametrize("n,k,most", [(8, 32768, 128), (53248, 32768, 128), (8192, 28672, 128), (4096, 40960, 0), (8, 32776, 0),
+                                      (16384, 16384, 256), (16392, 16384, 128), (53248, 8192, 256), (53248, 8200, 128), (8, 16392, 128)])
+def test_the_widest_results_that_are_left_to_the_input_gradient_kernel(n, k, most):
+    for tokens in (0, 1, 128, 129, 256, 257):
+        assert kernels.input_grad_pays(tokens, n, k) == (1 <= tokens <= most), tokens
+
+
 def _halves(w):   # a quantizer of the CPU: to steps of a half within +-1
     return (w.clamp(-1, 1) * 2).round() / 2
 
