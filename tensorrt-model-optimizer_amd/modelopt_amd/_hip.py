@@ -215,17 +215,20 @@ def call(name: str, anchor: torch.Tensor, *args):
         rc = fn(*args)   # the common case, without the context manager's cost
     else:
         with torch.cuda.device(anchor.device):
-            if _timer is None:
-                rc = fn(*args)
-            else:
-                start = torch.cuda.Event(enable_timing=True)
-                end = torch.cuda.Event(enable_timing=True)
-                start.record()
-                rc = fn(*args)
-                end.record()
-                _timer.pairs.append((name, start, end))
+            rc = fn(*args) if _timer is None else _timed(name, fn, *args)
     if rc != 0:
         _raise(name, rc)
+
+
+def _timed(name, fn, *args):
+    """``fn(*args)`` on the current device between two events of the active ``KernelTimer``; None (nothing launched) is no call."""
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    start.record()
+    made = fn(*args)
+    end.record()
+    if made is not None:
+        _timer.pairs.append((name, start, end))
+    return made
 
 
 def _raise(name, rc):
@@ -356,7 +359,8 @@ def amax_fold(accs, parts, dtypes):
         load()
     if any(d not in _DTYPES for d in dtypes):
         return None
-    made = _launch.amax_fold(accs, parts, [_DTYPES[d] for d in dtypes])
+    args = accs, parts, [_DTYPES[d] for d in dtypes]
+    made = _launch.amax_fold(*args) if _timer is None else _timed("mo_amax_fold", _launch.amax_fold, *args)
     return made if type(made) is not int else _raise("mo_amax_fold", made)
 
 

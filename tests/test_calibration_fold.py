@@ -199,3 +199,12 @@ def test_calibrated_values_and_accumulators_of_their_own():
     assert torch.equal(model.a.input_quantizer.amax, (2 * data).abs().max())
     assert torch.equal(model.b.weight_quantizer.amax, model.b.weight.abs().max())
     assert "a.input_quantizer._amax" in model.state_dict()
+
+
+@pytest.mark.gpu
+def test_a_timer_lists_the_fold():
+    acc = torch.ones(1, device=DEV)
+    with _hip.KernelTimer() as t:
+        assert _hip.amax_fold([acc, acc], [[], []], [torch.float32] * 2)[1].item() == 1
+        assert _hip.amax_fold([acc.cpu()], [[]], [torch.float32]) is None
+    assert t.calls == {"mo_amax_fold": 1} and t.seconds["mo_amax_fold"] > 0
