@@ -20,6 +20,7 @@ OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libmodelopt_hip.so")
 LAUNCH_SRC = os.path.join(HERE, "binding", "launch.cpp")   # compiled calls of the C ABI for the Python layer
 LAUNCH_LIB = os.path.join(HERE, "modelopt_amd", "_launch.so")
+LAUNCH_FOR = os.path.join(OBJ, "launch.txt")   # the interpreter and torch that LAUNCH_LIB was compiled against
 PROBE_SRC = os.path.join(HERE, "probe", "l2_read_probe.hip")   # measurement aid for bench.py: its own library, outside csrc/
 PROBE_LIB = os.path.join(HERE, "libmodelopt_probe.so")
 HEADERS = [os.path.join(CSRC, h) for h in ("common.h", "qdq_ops.h", "awq_ops.h", "nvfp4_ops.h", "blockfp_ops.h")] + [
@@ -56,6 +57,20 @@ def _compile(src, force, obj_dir, extra):
     return out
 
 
+def _interpreter():
+    import torch
+
+    return f"{sys.implementation.cache_tag} {torch.__version__} {torch.__file__}"
+
+
+def _launch_is_stale():
+    """Older than its sources, or compiled against another torch or Python: their layouts may differ."""
+    if _stale(LAUNCH_LIB, [LAUNCH_SRC, HEADERS[-1]]) or not os.path.exists(LAUNCH_FOR):
+        return True
+    with open(LAUNCH_FOR) as f:
+        return f.read() != _interpreter()
+
+
 def _build_launch():
     """The Python extension module: host code only, against the installed torch's headers."""
     import sysconfig
@@ -72,6 +87,8 @@ def _build_launch():
          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
          "-I", include[0], *(f for d in include[1:] for f in ("-isystem", d)), LAUNCH_SRC, "-o", LAUNCH_LIB,
          "-L", os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"], check=True)
+    with open(LAUNCH_FOR, "w") as f:
+        f.write(_interpreter())
 
 
 def build(force=False, jobs=4, tuning=False):
@@ -81,7 +98,7 @@ def build(force=False, jobs=4, tuning=False):
     os.makedirs(obj_dir, exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         launch = None
-        if not tuning and (force or _stale(LAUNCH_LIB, [LAUNCH_SRC, HEADERS[-1]])):
+        if force or _launch_is_stale():   # the Python layer needs it with either library
             launch = ex.submit(_build_launch)
         objs = list(ex.map(lambda s: _compile(s, force, obj_dir, extra), _sources()))
         if launch is not None:
