@@ -265,8 +265,10 @@ int mo_wgrad_masked(const void* dy, const void* x, const void* w, void* dw, int6
 /* Input gradient of that layer: dx[t, k] = T(sum over n of dy[t, n] * w[n, k]), sums in fp32; dy [tokens, n],
  * w [n, k], dx [tokens, k], all of type dtype (fp16 or bf16) and 16-byte aligned, n and k multiples of 8.
  * The sum over n is cut into `splits` runs; with more than one, partial holds splits * tokens * k floats.
- * mo_input_grad_splits: the number of runs that fills the chip, 0 for a size that the kernel does not take. */
+ * mo_input_grad_splits: the number of runs that fills the chip, 0 for a size that the kernel does not take.
+ * mo_input_grad_tile: the tokens of a workgroup's tile at that size (64, 128 or 256), 0 as above. */
 int mo_input_grad_splits(int64_t tokens, int64_t n, int64_t k);
+int mo_input_grad_tile(int64_t tokens, int64_t n, int64_t k);
 int mo_input_grad(const void* dy, const void* w, void* dx, float* partial, int64_t tokens, int64_t n, int64_t k,
                   int dtype, int splits, void* stream);
 

@@ -31,7 +31,7 @@ namespace {
     X(mo_absmax) X(mo_absmax_hinted) X(mo_absmax_tensor) X(mo_dynamic_qdq) X(mo_nvfp4_quantize_dynamic)       \
     X(mo_absmax_pair) X(mo_awq_pick_scale) X(mo_smooth_scales) X(mo_absmax_cols_staged)                       \
     X(mo_absmax_cols_noalloc) X(mo_fp8_qdq) X(mo_int_qdq) X(mo_ste_mask) X(mo_wgrad_masked) X(mo_row_qdq)     \
-    X(mo_input_grad_splits) X(mo_input_grad)                                                                  \
+    X(mo_input_grad_splits) X(mo_input_grad_tile) X(mo_input_grad)                                            \
     X(mo_nvfp4_qdq) X(mo_qdq_sq_err) X(mo_mxfp4_quantize) X(mo_mxfp4_dequantize) X(mo_block_fp_qdq)           \
     X(mo_convert_to_format) X(mo_nvfp4_quantize) X(mo_nvfp4_quantize_fused) X(mo_fused_amax_qdq)              \
     X(mo_nvfp4_dequantize) X(mo_real_quantize) X(mo_real_dequantize) X(mo_int4_block_quantize)                \

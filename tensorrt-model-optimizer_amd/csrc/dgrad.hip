@@ -284,11 +284,20 @@ static DgradPlan dgrad_plan(int64_t tokens, int64_t n, int64_t k) {
 
 }  // namespace mo
 
+static bool dgrad_takes(int64_t tokens, int64_t n, int64_t k) {
+    if (tokens <= 0 || n <= 0 || k <= 0 || n % 8 || k % 8) return false;
+    const int64_t limit = 0x7FFFFFFF;   // 32-bit byte offsets, of the loads past the last run too
+    return tokens <= 65536 && (tokens + 256) * n * 2 <= limit && (n + 512) * k * 2 <= limit;
+}
+
 extern "C" int mo_input_grad_splits(int64_t tokens, int64_t n, int64_t k) {
-    if (tokens <= 0 || n <= 0 || k <= 0 || n % 8 || k % 8) return 0;
-    const int64_t limit = 0x7FFFFFFF;
-    if (tokens > 65536 || (tokens + 256) * n * 2 > limit || (n + 512) * k * 2 > limit) return 0;
-    return (int)mo::dgrad_plan(tokens, n, k).splits;
+    return dgrad_takes(tokens, n, k) ? (int)mo::dgrad_plan(tokens, n, k).splits : 0;
+}
+
+extern "C" int mo_input_grad_tile(int64_t tokens, int64_t n, int64_t k) {
+    if (!dgrad_takes(tokens, n, k)) return 0;
+    const mo::DgradPlan p = mo::dgrad_plan(tokens, n, k);
+    return p.wm * p.mi * 32;
 }
 
 extern "C" int mo_input_grad(const void* dy, const void* w, void* dx, float* partial, int64_t tokens, int64_t n,
@@ -297,7 +306,7 @@ extern "C" int mo_input_grad(const void* dy, const void* w, void* dx, float* par
     if (dtype < MO_F32 || dtype > MO_BF16) return MO_ERR_DTYPE;
     if (dtype == MO_F32) return MO_ERR_UNSUPPORTED;
     if (tokens == 0 || k == 0) return MO_OK;
-    if (mo_input_grad_splits(tokens, n, k) == 0) return MO_ERR_UNSUPPORTED;
+    if (!dgrad_takes(tokens, n, k)) return MO_ERR_UNSUPPORTED;
     if (!dy || !w || !dx || splits < 1 || splits > (int)mo::kDgSplits || (splits > 1 && !partial)) return MO_ERR_ARG;
     if (((uintptr_t)dy | (uintptr_t)w | (uintptr_t)dx | (uintptr_t)partial) & 15u) return MO_ERR_UNSUPPORTED;
     mo::DgradPlan p = mo::dgrad_plan(tokens, n, k);

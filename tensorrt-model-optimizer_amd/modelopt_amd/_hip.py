@@ -50,6 +50,7 @@ SIGNATURES = {
     "mo_ste_mask": [_P, _P, _P, _I64, _I64, _I64, _INT, _P, _INT, _INT, _P],
     "mo_wgrad_masked": [_P, _P, _P, _P, _I64, _I64, _I64, _INT, _P, _INT, _I64, _INT, _P],
     "mo_input_grad_splits": [_I64, _I64, _I64],
+    "mo_input_grad_tile": [_I64, _I64, _I64],
     "mo_input_grad": [_P, _P, _P, _P, _I64, _I64, _I64, _INT, _INT, _P],
     "mo_row_qdq": [_P, _P, _I64, _I64, _INT, _P, _INT, _INT, _INT, _INT, _P, _INT, _P],
     "mo_nvfp4_qdq": [_P, _P, _I64, _I64, _INT, _P, _INT, _INT, _INT, _P],

@@ -151,8 +151,8 @@ def test_what_does_not_take_it():
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-# one token and one chunk; tokens at and past the three tiles; n below, at and past a step, in several runs, an odd
-# number of steps a run; columns with part of a tile
+# one token and one chunk; tokens at and past a tile; n below, at and past a step, in several runs, an odd number of
+# steps a run; columns with part of a tile
 @pytest.mark.parametrize("tokens,n,k", [(1, 8, 8), (64, 64, 128), (65, 72, 136), (129, 1160, 264), (200, 4104, 520),
                                         (257, 2056, 4096), (512, 520, 4104), (700, 14336, 1024), (31, 4096, 1 << 16)])
 def test_input_gradient_against_float64(dtype, tokens, n, k):
@@ -167,6 +167,20 @@ def test_input_gradient_against_float64(dtype, tokens, n, k):
     dy[0, n // 2] = float("nan")
     got = _hip.input_grad(dy, w)
     assert torch.isnan(got[0]).all() and not torch.isnan(got[1:]).any()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+# every tile, in one run and in several, with parts of a tile, of a step and of a run of steps
+@pytest.mark.parametrize("tile,several,tokens,n,k", [(64, False, 129, 72, 520), (64, True, 200, 4104, 520), (128, False, 257, 520, 16392),
+                                                     (128, True, 513, 4104, 2056), (256, False, 1000, 520, 8200),
+                                                     (256, False, 200, 72, 32776), (256, True, 257, 4104, 3976),
+                                                     (256, True, 700, 4104, 2056), (256, True, 385, 8200, 2056),
+                                                     (256, True, 512, 14336, 4096)])
+def test_every_tile_of_the_input_gradient(dtype, tile, several, tokens, n, k):
+    _hip.load()
+    assert _hip._entry["mo_input_grad_tile"](tokens, n, k) == tile
+    assert (_hip._entry["mo_input_grad_splits"](tokens, n, k) > 1) == several
+    test_input_gradient_against_float64(dtype, tokens, n, k)
 
 
 def test_input_gradient_stays_inside_its_operands():
