@@ -23,7 +23,7 @@ LAUNCH_LIB = os.path.join(HERE, "modelopt_amd", "_launch.so")
 LAUNCH_FOR = os.path.join(OBJ, "launch.txt")   # the interpreter and torch that LAUNCH_LIB was compiled against
 PROBE_SRC = os.path.join(HERE, "probe", "l2_read_probe.hip")   # measurement aid for bench.py: its own library, outside csrc/
 PROBE_LIB = os.path.join(HERE, "libmodelopt_probe.so")
-HEADERS = [os.path.join(CSRC, h) for h in ("common.h", "qdq_ops.h", "awq_ops.h", "nvfp4_ops.h", "blockfp_ops.h")] + [
+HEADERS = [os.path.join(CSRC, h) for h in ("common.h", "qdq_ops.h", "awq_ops.h", "nvfp4_ops.h", "blockfp_ops.h", "mfma_ops.h")] + [
     os.path.join(HERE, "..", "include", "modelopt_hip.h")]
 
 # -ffp-contract=off: the rounding tricks rely on separately rounded fp32 multiplies and adds.

@@ -19,40 +19,14 @@
 // products stand beside 910 of LDS and 768 of L1 (64 bytes a clock), and with no loads at all 512 tokens x 4096 x 14336
 // take 55 us where they take 66 with them.  Operands read three products ahead 66.0, two 66.9, one 67.7; two LDS stages 73.
 // No bank conflicts (counted).
-#include "common.h"
+#include "mfma_ops.h"
 
 namespace mo {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kDgCols = 128;     // results of a workgroup along k
 constexpr uint32_t kDgSplits = 16;   // most runs that the sum over n is cut into
 constexpr int kDgStep = 64;      // n of a step
 constexpr int kAhead = 3;        // of the four products of a step, how far ahead their operands are read
-
-template <int DT>
-__device__ __forceinline__ f32x16 dgrad_mfma(u32x4 a, u32x4 b, f32x16 c) {
-    if constexpr (DT == MO_BF16) {
-        bf16x8 av, bv;
-        __builtin_memcpy(&av, &a, 16);
-        __builtin_memcpy(&bv, &b, 16);
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, c, 0, 0, 0);
-    } else {
-        f16x8 av, bv;
-        __builtin_memcpy(&av, &a, 16);
-        __builtin_memcpy(&bv, &b, 16);
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, c, 0, 0, 0);
-    }
-}
-
-template <int DT>
-__device__ __forceinline__ uint32_t dgrad_pair(float lo, float hi) {
-    if constexpr (DT == MO_BF16) return f32x2_to_bf16x2(lo, hi);
-    else return f32_to_f16_bits(lo) | (f32_to_f16_bits(hi) << 16);
-}
 
 // Byte offset of 8 columns of n of a token in its tile (128 bytes a token)
 __device__ __forceinline__ int dgrad_dy_slot(int row, int octet) {
@@ -61,14 +35,6 @@ __device__ __forceinline__ int dgrad_dy_slot(int row, int octet) {
 // Byte offset of 8 columns of k of an n in the weight's tile (256 bytes an n)
 __device__ __forceinline__ int dgrad_w_slot(int row, int octet) {
     return row * 256 + ((octet ^ (row << 2)) & 15) * 16;
-}
-
-__device__ __forceinline__ u32x2 lds_transposed(const uint8_t* p) {
-    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
-    u32x2 r;
-    __builtin_memcpy(&r, &v, 8);
-    return r;
 }
 
 // WM x 2 wavefronts, 32 * MI tokens x 64 columns each
@@ -82,8 +48,7 @@ __global__ __launch_bounds__(WM * 128, 2) void dgrad_kernel(
     constexpr int kABytes = kRows * 128, kStage = kABytes + kDgStep * 256;
     __shared__ __align__(16) uint8_t lds[3 * kStage];
 
-    const uint32_t total = tiles_t * tiles_k * splits, xcd = blockIdx.x & 7u, q = total >> 3, rest = total & 7u;
-    const uint32_t id = xcd * q + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
+    const uint32_t id = xcd_tile(tiles_t * tiles_k * splits);
     const uint32_t t0 = id % tiles_t * kRows, rem = id / tiles_t, k0 = rem % tiles_k * kDgCols;
     const uint32_t split = rem / tiles_k;
     const uint32_t first = (uint32_t)((uint64_t)steps * split / splits);
@@ -165,7 +130,7 @@ __global__ __launch_bounds__(WM * 128, 2) void dgrad_kernel(
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < MI; ++j) acc[i][j] = dgrad_mfma<DT>(f.a[i], f.b[j], acc[i][j]);
+            for (int j = 0; j < MI; ++j) acc[i][j] = mfma_32x32x16<DT>(f.a[i], f.b[j], acc[i][j]);
     };
 
     const uint32_t count = last - first;
@@ -219,8 +184,8 @@ __global__ __launch_bounds__(WM * 128, 2) void dgrad_kernel(
                     *(f32x4*)(partial + ((size_t)split * tokens + t) * k_all + k) = o;
                 } else {
                     u32x2 o;
-                    o.x = dgrad_pair<DT>(v[4 * g], v[4 * g + 1]);
-                    o.y = dgrad_pair<DT>(v[4 * g + 2], v[4 * g + 3]);
+                    o.x = round_pair<DT>(v[4 * g], v[4 * g + 1]);
+                    o.y = round_pair<DT>(v[4 * g + 2], v[4 * g + 3]);
                     *(u32x2*)(dx + (size_t)t * k_all + k) = o;
                 }
             }
@@ -244,10 +209,10 @@ __global__ __launch_bounds__(256) void dgrad_sum_kernel(const float* __restrict_
         }
     }
     u32x4 o;
-    o.x = dgrad_pair<DT>(lo[0], lo[1]);
-    o.y = dgrad_pair<DT>(lo[2], lo[3]);
-    o.z = dgrad_pair<DT>(hi[0], hi[1]);
-    o.w = dgrad_pair<DT>(hi[2], hi[3]);
+    o.x = round_pair<DT>(lo[0], lo[1]);
+    o.y = round_pair<DT>(lo[2], lo[3]);
+    o.z = round_pair<DT>(hi[0], hi[1]);
+    o.w = round_pair<DT>(hi[2], hi[3]);
     *(u32x4*)(dx + c * 8) = o;
 }
 

@@ -24,39 +24,74 @@
 // SIMD do not fit the registers (128 of them spill: 243 us at 512 tokens).
 // Sums run in fp32 over the tokens in order, 16 an instruction, and round once: against sums in 64 bits as many results
 // are off by a rounding as the library's product has (32 to 1024 tokens, both types: the same ones).
-#include "common.h"
+#include "mfma_ops.h"
 
 namespace mo {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWgTile = 128;     // results of a workgroup along n and along k
 constexpr int kWgTokens = 64;    // tokens of a step
 constexpr int kWgLongTokens = 32;   // the same of the kernel for many tokens
 constexpr int kWgGroup = 8;      // n tiles that the workgroups of one XCD share their k tiles over
 
-template <int DT>
-__device__ __forceinline__ f32x16 wgrad_mfma(u32x4 a, u32x4 b, f32x16 c) {
-    if constexpr (DT == MO_BF16) {
-        bf16x8 av, bv;
-        __builtin_memcpy(&av, &a, 16);
-        __builtin_memcpy(&bv, &b, 16);
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, c, 0, 0, 0);
-    } else {
-        f16x8 av, bv;
-        __builtin_memcpy(&av, &a, 16);
-        __builtin_memcpy(&bv, &b, 16);
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, c, 0, 0, 0);
-    }
+// First result of this workgroup along n and along k: each XCD gets a run of tiles, group by group of n tiles with the
+// k tiles outside, so that what runs at a time shares its operands in the XCD's L2
+struct WgradOrigin { int64_t n, k; };
+__device__ __forceinline__ WgradOrigin wgrad_origin(uint32_t tiles_n, uint32_t tiles_k) {
+    const uint32_t id = xcd_tile(tiles_n * tiles_k);
+    const uint32_t per_group = kWgGroup * tiles_k, group = id / per_group, first = group * kWgGroup;
+    const uint32_t wide = tiles_n - first < kWgGroup ? tiles_n - first : kWgGroup;
+    const uint32_t in_group = id - group * per_group;
+    return {(int64_t)(first + in_group % wide) * kWgTile, (int64_t)(in_group / wide) * kWgTile};
 }
 
+// The weight's chunks of a lane at column k, 8 rows 16 apart from n on, and their limits as fp32 bits (one branch for all of them).
+// `inner` elements share an amax and a row is a whole number of them; 0: one amax
 template <int DT>
-__device__ __forceinline__ uint32_t wgrad_pair(float lo, float hi) {
-    if constexpr (DT == MO_BF16) return f32x2_to_bf16x2(lo, hi);
-    else return f32_to_f16_bits(lo) | (f32_to_f16_bits(hi) << 16);
+__device__ __forceinline__ void wgrad_weight(const uint16_t* __restrict__ w, int64_t n_first, int64_t n_all, int64_t k, int64_t k_all,
+                                             const void* __restrict__ amax, int amax_dtype, uint32_t inner,
+                                             RawChunk<DT> (&rw)[8], uint32_t (&raw_limit)[8]) {
+    const int64_t amax_row = inner ? (uint32_t)k_all / inner : 0, amax_col = inner ? (uint32_t)k / inner : 0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        int64_t n = n_first + u * 16;
+        n = n < n_all ? n : n_all - 1;
+        load_raw<DT>(w, n * k_all + k, rw[u]);
+    }
+    auto limits = [&](auto read) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            int64_t n = n_first + u * 16;
+            n = n < n_all ? n : n_all - 1;
+            raw_limit[u] = read(n * amax_row + amax_col);
+        }
+    };
+    if (amax_dtype == MO_F32) limits([&](int64_t i) { return ((const uint32_t*)amax)[i]; });
+    else if (amax_dtype == MO_BF16) limits([&](int64_t i) { return (uint32_t)((const uint16_t*)amax)[i] << 16; });
+    else limits([&](int64_t i) { return f2u(f16_bits_to_f32(((const uint16_t*)amax)[i])); });
+}
+
+// The sums of a wavefront at wn, wk of the tile, rounded, to LDS: 16-byte slots of a row of 128 results, permuted by the
+// row number
+template <int DT>
+__device__ __forceinline__ void wgrad_results(uint8_t* lds, const f32x16 (&acc)[2][2], int wn, int wk, int lane) {
+    const int l32 = lane & 31, half = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                // accumulators 4 g .. 4 g + 3 of lane l: k = 8 g + 4 (l / 32) + 0 .. 3, n = l % 32
+                const int row = wn + j * 32 + l32, slot = (wk + i * 32) / 8 + g;
+                u32x2 o;
+                o.x = round_pair<DT>(acc[i][j][4 * g], acc[i][j][4 * g + 1]);
+                o.y = round_pair<DT>(acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+                *(u32x2*)(lds + row * 256 + ((slot ^ row) & 15) * 16 + half * 8) = o;
+            }
+}
+// 8 results of a row of the tile
+__device__ __forceinline__ u32x4 wgrad_result(const uint8_t* lds, int row, int chunk) {
+    return *(const u32x4*)(lds + row * 256 + ((chunk ^ row) & 15) * 16);
 }
 
 // Byte offset of a column's octet of tokens in its operand tile.  A 16-byte store is served eight lanes at a
@@ -94,14 +129,8 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_kernel(
     uint8_t* const xs = lds;                               // columns of x: [128][64 tokens]
     uint8_t* const ys = lds + kWgTile * kWgTokens * 2;     // columns of dy
 
-    // workgroups go round the eight XCDs: each XCD gets a run of tiles, group by group of n tiles with the
-    // k tiles outside, so that what runs at a time shares its operands in the XCD's L2
-    const uint32_t total = tiles_n * tiles_k, xcd = blockIdx.x & 7u, q = total >> 3, rest = total & 7u;
-    const uint32_t id = xcd * q + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
-    const uint32_t per_group = kWgGroup * tiles_k, group = id / per_group, first = group * kWgGroup;
-    const uint32_t wide = tiles_n - first < kWgGroup ? tiles_n - first : kWgGroup;
-    const uint32_t in_group = id - group * per_group;
-    const int64_t n0 = (int64_t)(first + in_group % wide) * kWgTile, k0 = (int64_t)(in_group / wide) * kWgTile;
+    const WgradOrigin origin = wgrad_origin(tiles_n, tiles_k);
+    const int64_t n0 = origin.n, k0 = origin.k;
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // loading: lanes 0 .. 127 x, 128 .. 255 dy; 16 chunks of 8 columns by 8 octets of tokens
@@ -148,7 +177,7 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_kernel(
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = wgrad_mfma<DT>(a[i], b[j], acc[i][j]);
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma_32x32x16<DT>(a[i], b[j], acc[i][j]);
         }
         __syncthreads();
     }
@@ -160,45 +189,13 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_kernel(
     int64_t k = k0 + out_chunk * 8;
     const bool k_ok = k < k_all;
     k = k_ok ? k : k_all - 8;
-    // inner elements share an amax and a row is a whole number of them; 0: one amax
-    const int64_t amax_row = inner ? (uint32_t)k_all / inner : 0, amax_col = inner ? (uint32_t)k / inner : 0;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        int64_t n = n0 + u * 16 + out_row;
-        n = n < n_all ? n : n_all - 1;
-        load_raw<DT>(w, n * k_all + k, rw[u]);
-    }
-    // the limits as fp32 bits, one branch for all of them
-    auto limits = [&](auto read) {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            int64_t n = n0 + u * 16 + out_row;
-            n = n < n_all ? n : n_all - 1;
-            raw_limit[u] = read(n * amax_row + amax_col);
-        }
-    };
-    if (amax_dtype == MO_F32) limits([&](int64_t i) { return ((const uint32_t*)amax)[i]; });
-    else if (amax_dtype == MO_BF16) limits([&](int64_t i) { return (uint32_t)((const uint16_t*)amax)[i] << 16; });
-    else limits([&](int64_t i) { return f2u(f16_bits_to_f32(((const uint16_t*)amax)[i])); });
-    // 16-byte slots of a row of 128 results, permuted by the row number
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                // accumulators 4 g .. 4 g + 3 of lane l: k = 8 g + 4 (l / 32) + 0 .. 3, n = l % 32
-                const int row = wn + j * 32 + l32, slot = (wk + i * 32) / 8 + g;
-                u32x2 o;
-                o.x = wgrad_pair<DT>(acc[i][j][4 * g], acc[i][j][4 * g + 1]);
-                o.y = wgrad_pair<DT>(acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-                *(u32x2*)(lds + row * 256 + ((slot ^ row) & 15) * 16 + half * 8) = o;
-            }
+    wgrad_weight<DT>(w, n0 + out_row, n_all, k, k_all, amax, amax_dtype, inner, rw, raw_limit);
+    wgrad_results<DT>(lds, acc, wn, wk, lane);
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
         const int row = u * 16 + out_row;
-        u32x4 g = *(const u32x4*)(lds + row * 256 + ((out_chunk ^ row) & 15) * 16);
+        u32x4 g = wgrad_result(lds, row, out_chunk);
         float v[8], limit = u2f(raw_limit[u]);
         const float rounded = DT == MO_BF16 ? round_to_bf16(limit) : f16_bits_to_f32(f32_to_f16_bits(limit));
         limit = narrow ? rounded : limit;
@@ -225,14 +222,6 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_kernel(
 // bytes for 32 lanes: the four lie in different quarters of a row.
 __device__ __forceinline__ int wgrad_row_slot(int token, int octet) {
     return token * 256 + ((octet ^ (token << 2)) & 15) * 16;
-}
-
-__device__ __forceinline__ u32x2 wgrad_transposed(const uint8_t* p) {
-    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
-    u32x2 r;
-    __builtin_memcpy(&r, &v, 8);
-    return r;
 }
 
 // The mask on the two elements of a word at a time: |w| <= amax is an order of the 15 bits below the sign, with amax
@@ -267,14 +256,8 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_long_kernel(
     constexpr int kTile = kWgLongTokens * 256, kStage = 2 * kTile, kChunks = kWgLongTokens / 16;
     __shared__ __align__(16) uint8_t lds[3 * kStage];   // a stage: x, then dy
 
-    // workgroups go round the eight XCDs: each XCD gets a run of tiles, group by group of n tiles with the
-    // k tiles outside, so that what runs at a time shares its operands in the XCD's L2
-    const uint32_t total = tiles_n * tiles_k, xcd = blockIdx.x & 7u, q = total >> 3, rest = total & 7u;
-    const uint32_t id = xcd * q + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
-    const uint32_t per_group = kWgGroup * tiles_k, group = id / per_group, first = group * kWgGroup;
-    const uint32_t wide = tiles_n - first < kWgGroup ? tiles_n - first : kWgGroup;
-    const uint32_t in_group = id - group * per_group;
-    const int64_t n0 = (int64_t)(first + in_group % wide) * kWgTile, k0 = (int64_t)(in_group / wide) * kWgTile;
+    const WgradOrigin origin = wgrad_origin(tiles_n, tiles_k);
+    const int64_t n0 = origin.n, k0 = origin.k;
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // Buffer descriptors of one step's rows (scalar): what is past the last token reads as zero, what is past the
@@ -326,26 +309,7 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_long_kernel(
     {
         RawChunk<DT> rw[8];
         uint32_t raw_limit[8];
-        // inner elements share an amax and a row is a whole number of them; 0: one amax
-        const int64_t amax_row = inner ? (uint32_t)k_all / inner : 0, amax_col = inner ? (uint32_t)k / inner : 0;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            int64_t n = n0 + u * 16 + out_row;
-            n = n < n_all ? n : n_all - 1;
-            load_raw<DT>(w, n * k_all + k, rw[u]);
-        }
-        // the limits as fp32 bits, one branch for all of them
-        auto limits = [&](auto read) {
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                int64_t n = n0 + u * 16 + out_row;
-                n = n < n_all ? n : n_all - 1;
-                raw_limit[u] = read(n * amax_row + amax_col);
-            }
-        };
-        if (amax_dtype == MO_F32) limits([&](int64_t i) { return ((const uint32_t*)amax)[i]; });
-        else if (amax_dtype == MO_BF16) limits([&](int64_t i) { return (uint32_t)((const uint16_t*)amax)[i] << 16; });
-        else limits([&](int64_t i) { return f2u(f16_bits_to_f32(((const uint16_t*)amax)[i])); });
+        wgrad_weight<DT>(w, n0 + out_row, n_all, k, k_all, amax, amax_dtype, inner, rw, raw_limit);
         load(r0);
         load(r1);
 #pragma unroll
@@ -359,7 +323,7 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_long_kernel(
     asm volatile("" : "+v"(keep[0]), "+v"(keep[1]));   // here, not after the products, with the weight spilled until then
 
     // multiplying: 64 x 64 of a wavefront, 2 x 2 blocks of 32
-    const int wk = (wave & 1) * 64, wn = (wave >> 1) * 64, l32 = lane & 31, half = lane >> 5;
+    const int wk = (wave & 1) * 64, wn = (wave >> 1) * 64, half = lane >> 5;
     int a_at[2], b_at[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -371,10 +335,10 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_long_kernel(
     auto read = [&](Operands& f, int at, int s) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            u32x2 lo = wgrad_transposed(lds + at + a_at[i] + s * 4096), hi = wgrad_transposed(lds + at + a_at[i] + s * 4096 + 1024);
+            u32x2 lo = lds_transposed(lds + at + a_at[i] + s * 4096), hi = lds_transposed(lds + at + a_at[i] + s * 4096 + 1024);
             f.a[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
-            lo = wgrad_transposed(lds + at + b_at[i] + s * 4096);
-            hi = wgrad_transposed(lds + at + b_at[i] + s * 4096 + 1024);
+            lo = lds_transposed(lds + at + b_at[i] + s * 4096);
+            hi = lds_transposed(lds + at + b_at[i] + s * 4096 + 1024);
             f.b[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
         }
     };
@@ -389,7 +353,7 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_long_kernel(
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = wgrad_mfma<DT>(f.a[i], f.b[j], acc[i][j]);
+            for (int j = 0; j < 2; ++j) acc[i][j] = mfma_32x32x16<DT>(f.a[i], f.b[j], acc[i][j]);
     };
 
     int now = 0, next = kStage, after = 2 * kStage;   // LDS stages: multiplied, complete, being written
@@ -425,25 +389,12 @@ __global__ __launch_bounds__(256, 3) void wgrad_masked_long_kernel(
     }
     __syncthreads();   // the operands read ahead of the loop's end
 
-    // 16-byte slots of a row of 128 results, permuted by the row number
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                // accumulators 4 g .. 4 g + 3 of lane l: k = 8 g + 4 (l / 32) + 0 .. 3, n = l % 32
-                const int row = wn + j * 32 + l32, slot = (wk + i * 32) / 8 + g;
-                u32x2 o;
-                o.x = wgrad_pair<DT>(acc[i][j][4 * g], acc[i][j][4 * g + 1]);
-                o.y = wgrad_pair<DT>(acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-                *(u32x2*)(lds + row * 256 + ((slot ^ row) & 15) * 16 + half * 8) = o;
-            }
+    wgrad_results<DT>(lds, acc, wn, wk, lane);
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
         const int row = u * 16 + out_row;
-        u32x4 g = *(const u32x4*)(lds + row * 256 + ((out_chunk ^ row) & 15) * 16);
+        u32x4 g = wgrad_result(lds, row, out_chunk);
 #pragma unroll
         for (int j = 0; j < 4; ++j) g[j] &= wgrad_mask(keep[u >> 2] >> ((u & 3) * 4 + j));
         if (k_ok && n0 + row < n_all) __builtin_nontemporal_store(g, (u32x4*)(dw + (n0 + row) * k_all + k));
