@@ -19,7 +19,6 @@ __all__ = [
 
 
 _STOCK = torch.nn.Module
-_HOW_MODES_ARE_SET = ("train", "children", "named_children")   # the methods that the stock ``train`` goes through
 
 
 def _walk(module, found, seen):
@@ -32,24 +31,37 @@ def _walk(module, found, seen):
                 _walk(child, found, seen)
 
 
+# Loops and not any(...) below: a calibration asks six times, and a generator is resumed for every module.
+
+
 def modules_of(model) -> list:
     """``list(model.modules())`` without a chain of nested generators (a third of their time).  The walk is no function in
     here: one that names itself is a cycle, and the modules it has seen would live until the garbage collector runs."""
     found = []
     _walk(model, found, set())
-    if any(getattr(c, n) is not getattr(_STOCK, n) for c in set(map(type, found)) for n in ("modules", "named_modules")) or any(
-            "named_modules" in m.__dict__ or "modules" in m.__dict__ for m in found):
-        return list(model.modules())   # a module that lists its modules itself
-    return found
+    listed = type(model).modules is not _STOCK.modules or "modules" in model.__dict__   # by the model itself
+    for c in set(map(type, found)):
+        listed = listed or c.named_modules is not _STOCK.named_modules
+    for m in found:
+        if "named_modules" in m.__dict__:
+            listed = True
+    return list(model.modules()) if listed else found
 
 
 def set_training(model, mode: bool):
     """``model.train(mode)``, written to the modules that are in the other mode only."""
     modules = []
     _walk(model, modules, set())
-    if any(getattr(c, n) is not getattr(_STOCK, n) for c in set(map(type, modules)) for n in _HOW_MODES_ARE_SET) or any(
-            n in m.__dict__ for m in modules for n in _HOW_MODES_ARE_SET):
-        model.train(mode)   # a module that sets its mode, or lists its children, itself
+    own = False   # a module that sets its mode, or lists its children, itself
+    for c in set(map(type, modules)):
+        own = own or (c.train is not _STOCK.train or c.children is not _STOCK.children
+                      or c.named_children is not _STOCK.named_children)
+    for m in modules:
+        names = m.__dict__
+        if "train" in names or "children" in names or "named_children" in names:
+            own = True
+    if own:
+        model.train(mode)
         return
     for m in modules:
         if m.training is not mode:
