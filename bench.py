@@ -368,8 +368,8 @@ def single_tensor_configs(torch, steps, warmup):
 
     # AWQ clip search on the same weight: 11 clip ratios x every 128-wide block, 64 calibration
     # tokens, one launch.  Bound by the issue of matrix instructions: 2048 rounded products are one
-    # outer-product instruction and four that sum, 128 cycles of a SIMD, beside 64 conversions on
-    # its vector ALU (half an instruction per product): 1024 SIMDs at 2.4 GHz
+    # outer-product instruction, 64 cycles of a SIMD, and two sparse ones that sum, 16 each, beside
+    # 16 conversions on its vector ALU (half an instruction per product): 1024 SIMDs at 2.4 GHz
     ratios = [round(float(v), 2) for v in torch.arange(0.5, 1.0, 0.05)] + [1.0]
     x64 = x3[::8].contiguous()
     w_amax = w3.view(-1, 128).abs().amax(1, keepdim=True)
@@ -381,8 +381,8 @@ def single_tensor_configs(torch, steps, warmup):
     products = 4096 * 4096 * 64 * (len(ratios) + 1)
     out["awq_clip_search_kernel_11_ratios_4096x4096_64_tokens"] = {
         "ms": round(ms, 4), "rounded_products_per_s": round(products / ms * 1e3, 0), "bound": "mfma",
-        "matrix_cycles_per_2048_products": 128, "peak_products_per_s": 39.32e12,
-        "frac": round(products / ms * 1e3 / 39.32e12, 4)}
+        "matrix_cycles_per_2048_products": 96, "peak_products_per_s": 52.43e12,
+        "frac": round(products / ms * 1e3 / 52.43e12, 4)}
     cfg = copy.deepcopy(mtq.INT4_AWQ_CFG)
     cfg["algorithm"] = {"method": "awq_clip"}
     out["awq_clip_4096x4096_end_to_end_ms"] = round(end_to_end(w3, x3, cfg) * 1e3, 3)
