@@ -807,16 +807,18 @@ extern "C" int mo_awq_clip_losses(const void* x, int64_t tokens, const void* w, 
     } else {
         smem = (size_t)mo::kClipWaves * mo::kClipLanes * (dtype == MO_F16 ? mo::kClipTokens * 2 : 8 * (16 + 8));
         // A wavefront goes through all ratios unless there are too few of them to fill the chip; then
-        // 2 to 11 of them share the ratios, each scoring the unclipped block once more.  11 ratios, 64
-        // tokens, blocks of 128 (with dense sums, where the lines were drawn):
-        //   bf16  4096 x 4096, 4096 wavefronts: 484 us, 503 with 2 shares; 1024 x 4096, 1024: 157, 145 with 2,
-        //         142 with 3, 149 with 4; 1024 x 1024, 256: 156, 91 with 2, 56 with 4, 59 with 8
-        //   fp16  4096 x 4096, 2048 wavefronts: 506 us, 444 with 2 shares, 465 with 4; 1024 x 4096, 512:
-        //         313, 148 with 4, 162 with 8; 1024 x 1024, 128: 280, 99 with 4, 76 with 8, 72 with 11
-        // (cards differ by some 8 %; 1024 x 1024 now 45 and 66.)  What bounds the bf16 form: a step of 2048 products is
-        // 96 cycles of matrix instructions (64 of products) and about 90 of vector instructions (72 of conversions) plus
-        // 24 of the port that issues both; measured 160.  Higher priority for the wavefront at its matrix
-        // instructions (402 us), sums between the conversions (424) or products behind the first of them (444) win nothing.
+        // 2 to 11 of them share the ratios, each scoring the unclipped block once more.  The lines lie where they were drawn
+        // for dense sums; with sparse ones, 11 ratios, 64 tokens, blocks of 128, us by number of shares:
+        //   bf16  4096 x 4096, 4096 wavefronts: 411, 433 with 2; 2048 x 4096, 2048: 211, 219 with 2; 1024 x 4096, 1024: 131, 117
+        //         with 2, 119 with 3, 125 with 4; 1024 x 1024, 256: 129, 76 with 2, 45 with 4, 48 with 8
+        //   fp16  4096 x 4096, 2048 wavefronts: 485, 443 with 2, 440 with 3, 462 with 4; 1024 x 4096, 512: 289, 142 with 4, 140 - 145
+        //         with 6 (the line's), 159 with 8; 1024 x 1024, 128: 280, 98 with 4, 74 with 8, 67 with 11
+        // The line is within 2 % of the best of them from 256 wavefronts on (blocks of 32 and 64 too); with fewer, bf16 would gain by
+        // more than four shares (512 x 512, 64 wavefronts: 45 and 25 with 11).  Cards differ by some 8 %.
+        // What bounds the bf16 form: a step of 2048 products is 96 cycles of matrix instructions (64 of products) and about
+        // 90 of vector instructions (72 of conversions) plus 24 of the port that issues both; measured 160.  Higher
+        // priority for the wavefront at its matrix instructions (402 us), sums between the conversions (424) or products
+        // behind the first of them (444) win nothing.
         const int64_t sets = (int64_t)grid.x * grid.y * mo::kClipWaves;
         int64_t share = ((dtype == MO_BF16 ? 2048 : 3072) + sets - 1) / sets;
         if (dtype == MO_BF16 && share > 4) share = 4;
