@@ -5,7 +5,9 @@ without given scales can run as ONE launch that reads the tensor once (``mo_fuse
 ``mo_nvfp4_quantize_fused``).  Those kernels want all their workgroups on the device at the same
 time; when that cannot be had (another stream's kernel holds the compute units, a masked device)
 they still return the right bits, but only after a bounded wait.  Off by default: the two-launch
-path has no such dependence on what else the device is doing.
+path has no such dependence on what else the device is doing, and since its abs-max leaves parts
+instead of filling an accumulator it is faster at every size measured (bf16, us, one launch against
+two: FP8 2 MB 11.5 and 8.5, 34 MB 20.6 and 19.0; NVFP4 quantize 34 MB 20.4 and 15.3).
 
 ``set_strict_checks`` -- the reference's CPU path looks at the data on the host before it
 quantises (``tensor_quant.py:577-587``: negative values with ``unsigned=True`` raise ``TypeError``,
