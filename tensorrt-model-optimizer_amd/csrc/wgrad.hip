@@ -420,7 +420,8 @@ extern "C" int mo_wgrad_masked(const void* dy, const void* x, const void* w, voi
     mo::KERNEL<DT><<<(unsigned)(tn * tk), 256, 0, s>>>(                                                     \
         (const uint16_t*)dy, (const uint16_t*)x, (const uint16_t*)w, (uint16_t*)dw, tokens, n, k, (uint32_t)tn, \
         (uint32_t)tk, amax, amax_dtype, (uint32_t)inner, narrow_amax)
-    // from where it is faster at every size measured, and where 32 rows have 32-bit byte offsets
+    // From where it is faster at every size measured (16 shapes, both types, 384 to 4096 tokens: at 384 bf16 14336 x 4096 92.8 -> 82.1 us,
+    // 4096 x 64 9.2 -> 8.5, 2752 x 4096 20.7 -> 19.9; at 256 14336 x 4096 62 and 62), and where 32 rows have 32-bit byte offsets
     if (tokens >= 384 && n < 1 << 25 && k < 1 << 25) {
         if (dtype == MO_BF16) CALL(wgrad_masked_long_kernel, MO_BF16); else CALL(wgrad_masked_long_kernel, MO_F16);
     } else {
